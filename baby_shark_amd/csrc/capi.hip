@@ -302,7 +302,7 @@ bs_status bs_volume_clone(const bs_volume* v, bs_volume** out) {
     });
 }
 
-void bs_release_cached_memory(void) { release_cached_leaves(); }
+void bs_release_cached_memory(void) { release_cached_memory(); }
 
 void bs_volume_free(bs_volume* v) {
     if (!v) return;
@@ -526,11 +526,11 @@ bs_status bs_dual_contour(bs_ctx* ctx, const bs_volume* v, float voxel_size, flo
         if (!n) return;
         float* h = static_cast<float*>(std::malloc(sizeof(float) * 9 * n));
         if (!h) {
-            (void)hipFree(d);
+            free_block(d);
             throw Error(BS_ERR_INTERNAL, "host out of memory");
         }
         hipError_t e = hipMemcpy(h, d, sizeof(float) * 9 * n, hipMemcpyDeviceToHost);
-        (void)hipFree(d);
+        free_block(d);
         if (e != hipSuccess) {
             std::free(h);
             BS_HIP(e);
@@ -544,11 +544,11 @@ bs_status bs_dual_contour(bs_ctx* ctx, const bs_volume* v, float voxel_size, flo
 static float* soup_to_host(float* d, uint64_t n) {
     float* h = static_cast<float*>(std::malloc(sizeof(float) * 9 * n));
     if (!h) {
-        (void)hipFree(d);
+        free_block(d);
         throw Error(BS_ERR_INTERNAL, "host out of memory");
     }
     hipError_t e = hipMemcpy(h, d, sizeof(float) * 9 * n, hipMemcpyDeviceToHost);
-    (void)hipFree(d);
+    free_block(d);
     if (e != hipSuccess) {
         std::free(h);
         BS_HIP(e);
@@ -678,7 +678,7 @@ bs_status bs_stl_write(const char* path, const float* tri_xyz, size_t n_tris) {
 void bs_free(void* p) { std::free(p); }
 
 void bs_device_free(void* p) {
-    if (p) (void)hipFree(p);
+    free_block(p);
 }
 
 bs_status bs_volume_densify_tiles(bs_ctx* ctx, bs_volume* v) {

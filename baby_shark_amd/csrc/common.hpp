@@ -36,6 +36,19 @@ void set_last_error(const std::string& msg);
         if (!(cond)) throw ::bs::Error((status), (msg));       \
     } while (0)
 
+// hipMalloc on the current device; when memory runs out, the library's pools
+// are emptied and it tries once more.
+hipError_t device_malloc(void** p, uint64_t bytes);
+
+// Device blocks from a per-device pool of released ones (device_pool.hip).
+// free_block takes any device pointer (one that the pool did not hand out goes
+// to hipFree); it waits for the block's device first, as hipFree does, unless
+// `wait` is false: the caller then knows that nothing still uses the block.
+void* alloc_block(uint64_t bytes);
+void free_block(void* p, bool wait = true);
+// Empties the pools of leaf arrays and blocks.
+void release_cached_memory();
+
 // ---------------------------------------------------------------- scratch arena
 // Named device buffers owned by a context that only ever grow, so a steady
 // stream of same-sized calls allocates nothing after the first.
@@ -46,7 +59,7 @@ enum ScratchSlot : int {
     S_BVH_LINKS, S_BVH_PARENT, S_BVH_FLAGS, S_BVH_INIT, S_BVH_BOX, S_RECHECK, S_ARGMIN, S_MISC0, S_MISC1,
     S_MISC2, S_MISC3, S_INPUT, S_BVH_KIDS, S_FLAGS_A, S_FLAGS_B, S_CSG_PLAN, S_DC_MAP, S_DC_KEYS, S_DC_FAIL, S_DC_CELLS, S_SIGN_ROOTS, S_REP_CNT, S_REP_OFF, S_REPS,
     S_BVH_HEIGHT, S_BVH_HEIGHT_S, S_BVH_INODE, S_BVH_INODE_S, S_BVH_MISC, S_BVH_STARTS, S_CUB_B,
-    S_DC_CELLMASK, S_DC_TRICNT, S_DC_TRIOFF, S_MC_TAB, S_MC_UNITS, S_MC_TILES, S_MC_T8, S_MC_T8K, S_MC_T128,
+    S_DC_CELLMASK, S_DC_NEGMASK, S_DC_TRICNT, S_DC_TRIOFF, S_MC_TAB, S_MC_UNITS, S_MC_TILES, S_MC_T8, S_MC_T8K, S_MC_T128,
     S_MC_T128K, S_MC_TORG, S_MC_LANES, S_LEAF_BOX, S_SG_PRED, S_MLP_PART, S_MLP_GRAD, S_MLP_PERM, S_MC_FLAGS, S_MC_CV, S_MC_V12,
     S_PLOC_BOX, S_PLOC_INFO, S_PLOC_C0, S_PLOC_C1, S_PLOC_NN, S_PLOC_KEEP, S_PLOC_POS, S_PLOC_RING,
     S_TD_PRIMS, S_TD_FR, S_TD_BINS, S_TD_TASKS, S_TD_TCNT, S_TD_SPLIT, S_TD_SMALL, S_TD_HIST,
@@ -62,7 +75,7 @@ struct Scratch {
             if (ptr[slot]) BS_HIP(hipFree(ptr[slot]));
             ptr[slot] = nullptr;
             size_t b = bytes + bytes / 4 + 256;
-            BS_HIP(hipMalloc(&ptr[slot], b));
+            BS_HIP(device_malloc(&ptr[slot], b));
             cap[slot] = b;
         }
         return ptr[slot];

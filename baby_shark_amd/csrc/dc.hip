@@ -4,15 +4,17 @@
 // The reference runs three visitor passes and keeps the edge crossings and
 // the cell points in sparse trees behind locks.  Here:
 //   * cell pass: one wavefront per leaf stages the leaf and a one-to-two voxel
-//     halo (an 11^3 block from the 27 surrounding leaves) in LDS; every lane
-//     owns one z-row.  It checks the gradient of every crossing edge (the
-//     reference's unreachable!() case), and for every fully active
-//     sign-changing cube recomputes the crossings of its edges on the fly
-//     (deterministic, so bit-identical to storing them) and runs the damped
-//     particle iteration.  Cell points go to a per-leaf 8^3 block plus a
-//     512-bit presence mask.
-//   * triangle pass: the same staging; each active voxel emits two triangles
-//     per sign-changing edge whose four cells exist, scaled by the voxel size,
+//     halo (an 11^3 block from the 27 surrounding leaves) in LDS, one z-row per
+//     lane, with a word of activity and sign bits per row.  Bit operations on
+//     those words find the rows' crossing edges without all six gradients (the
+//     reference's unreachable!() case), the crossing edges and the fully
+//     active sign-changing cubes.  Then a lane takes an edge each (its crossing
+//     and normal, to LDS) and after that a cube each (the damped particle
+//     iteration over its listed edges).  Cell points go to the leaf's compact
+//     list, in cell order, with a 512-bit presence mask and the leaf's signs.
+//   * triangle pass: from the presence masks and signs alone, each row's
+//     sign-changing edges whose four cells exist; a lane per such edge fetches
+//     the four points and emits two triangles, scaled by the voxel size,
 //     degenerate ones dropped.  A counting launch, a scan and a writing
 //     launch give the sequential order: leaves by origin, voxels x-y-z, edges
 //     X-Y-Z.
@@ -33,107 +35,156 @@ Topology& ensure_topology(bs_ctx* ctx, bs_volume* v);
 namespace {
 
 constexpr int HB = 11;  // staged block edge: leaf-local -1 .. 9
-constexpr int HB3 = HB * HB * HB;
+constexpr int HR = HB * HB;
+constexpr int CB = 9;    // rows of corners that the leaf's cells touch: 0 .. 8
+constexpr int CR = CB * CB;
+constexpr int EDGE_LDS = 192;  // crossing edges kept in LDS per leaf (about 45 on a smooth surface)
 
 struct DcArgs {
     LeafMap map;
     const int4* origins;
     const uint64_t* masks;
     const float* values;
-    float* cell_pts;        // n_leaves * 512 * 3
+    float* cell_pts;        // per leaf 512 * 3: the points of its cells, in cell order, from its start
     uint64_t* cell_mask;    // n_leaves * 8
+    uint64_t* neg_mask;     // n_leaves * 8: active voxels with the sign bit set
     float voxel_size;
     uint32_t* fail;         // bit 0: gradient without neighbours
 };
 
 struct Block {
-    float val[HB3];
-    uint8_t act[HB3];
+    float val[HB * HR];
+    uint32_t row[HR];        // z-row (x, y): bit z + 1 active, bit z + 17 active with the sign bit set
+    uint32_t edge_row[CR];   // crossing edges from row (x, y), bit 9 * axis + z
+    uint32_t edge_pre[CR];   // edges of the rows before
+    float4 edge[EDGE_LDS];   // crossing coordinate along the edge, unit normal
+    uint16_t list[EDGE_LDS > 512 ? EDGE_LDS : 512];  // edges, then cells
     int32_t nb[27];
 };
 
-__device__ inline int bidx(int x, int y, int z) { return ((x + 1) * HB + (y + 1)) * HB + (z + 1); }
+__device__ inline int ridx(int x, int y) { return (x + 1) * HB + (y + 1); }
 
-// Stages the values and activity of leaf-local voxels -1..9 on each axis.
+// One workgroup is one wavefront and takes leaves dc_leaf(blockIdx.x),
+// dc_leaf(blockIdx.x + gridDim.x), ... below dc_span(n).  Workgroups go to
+// the 8 XCDs in turn; each XCD takes runs of DC_RUN consecutive leaves, so a
+// leaf's z- and y-neighbours, whose layers it stages, are read through the
+// same L2.
+constexpr uint64_t DC_RUN = 64;
+__host__ __device__ inline uint64_t dc_span(uint64_t n) { return (n + 8 * DC_RUN - 1) / (8 * DC_RUN) * (8 * DC_RUN); }
+__device__ inline uint64_t dc_leaf(uint64_t v) {
+    const uint64_t k = v >> 3;
+    return ((k / DC_RUN) * 8 + (v & 7)) * DC_RUN + k % DC_RUN;
+}
+
+// Exclusive prefix sum over the wave; total in every lane.
+__device__ inline uint32_t wave_prefix(uint32_t v, int lane, uint32_t& total) {
+    uint32_t incl = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t u = (uint32_t)__shfl_up((int)incl, d, 64);
+        if (lane >= d) incl += u;
+    }
+    total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    return incl - v;
+}
+
+// Row r of the staged block: its eight own voxels in two 16-byte loads, one
+// voxel of the leaf below and two of the leaf above, and the rows' mask bytes
+// (byte y of word x holds row (x, y)).  A missing leaf's loads go to leaf 0 and
+// are masked off, so all of a row's loads travel together.
+struct RowLoads {
+    float4 v0, v1;
+    float2 up;
+    float down;
+    uint32_t m0, m1, m2;
+};
+__device__ inline void row_issue(const Block& B, const DcArgs& a, int r, RowLoads& q) {
+    const int x = r / HB - 1, y = r % HB - 1;
+    const int32_t* nb = B.nb + ((x >> 3) + 1) * 9 + ((y >> 3) + 1) * 3;
+    const int32_t s0 = nb[0], s1 = nb[1], s2 = nb[2];
+    const uint64_t t0 = s0 >= 0 ? s0 : 0, t1 = s1 >= 0 ? s1 : 0, t2 = s2 >= 0 ? s2 : 0;
+    const int ro = ((x & 7) << 6) | ((y & 7) << 3), mo = ((x & 7) << 3) | (y & 7);
+    const uint8_t* mb = reinterpret_cast<const uint8_t*>(a.masks);
+    q.m0 = mb[t0 * 64 + mo];
+    q.m1 = mb[t1 * 64 + mo];
+    q.m2 = mb[t2 * 64 + mo];
+    const float4* p = reinterpret_cast<const float4*>(a.values + t1 * 512 + ro);
+    q.v0 = p[0];
+    q.v1 = p[1];
+    q.down = a.values[t0 * 512 + ro + 7];
+    q.up = *reinterpret_cast<const float2*>(a.values + t2 * 512 + ro);
+    if (s0 < 0) q.m0 = 0;
+    if (s1 < 0) q.m1 = 0;
+    if (s2 < 0) q.m2 = 0;
+}
+__device__ inline void row_store(Block& B, int r, const RowLoads& q) {
+    const float v[HB] = {q.down, q.v0.x, q.v0.y, q.v0.z, q.v0.w, q.v1.x, q.v1.y, q.v1.z, q.v1.w, q.up.x, q.up.y};
+    const uint32_t act = (q.m0 >> 7) | (q.m1 << 1) | ((q.m2 & 3u) << 9);
+    uint32_t neg = 0;
+#pragma unroll
+    for (int k = 0; k < HB; ++k) {
+        B.val[r * HB + k] = v[k];
+        neg |= (__float_as_uint(v[k]) >> 31) << k;
+    }
+    B.row[r] = act | ((neg & act) << 16);
+}
+
+// Stages the values and the activity and sign bits of leaf-local voxels -1..9.
 __device__ inline void stage_block(Block& B, const DcArgs& a, int4 org, int lane) {
     if (lane < 27) {
         const int dx = lane / 9 - 1, dy = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
         B.nb[lane] = a.map.find((org.x >> 3) + dx, (org.y >> 3) + dy, (org.z >> 3) + dz);
     }
     __syncthreads();
-    for (int i = lane; i < HB3; i += 64) {
-        const int bx = i / (HB * HB), by = (i / HB) % HB, bz = i % HB;
-        const int x = bx - 1, y = by - 1, z = bz - 1;
-        const int dx = x >> 3, dy = y >> 3, dz = z >> 3;  // -1, 0 or 1
-        const int32_t s = B.nb[(dx + 1) * 9 + (dy + 1) * 3 + (dz + 1)];
-        float v = 0.0f;
-        uint8_t on = 0;
-        if (s >= 0) {
-            const int o = ((x & 7) << 6) | ((y & 7) << 3) | (z & 7);
-            on = (a.masks[(uint64_t)s * 8 + (o >> 6)] >> (o & 63)) & 1ull;
-            if (on) v = a.values[(uint64_t)s * 512 + o];
-        }
-        B.val[i] = v;
-        B.act[i] = on;
-    }
+    const int r1 = min(lane + 64, HR - 1);
+    RowLoads q0, q1;
+    row_issue(B, a, lane, q0);
+    row_issue(B, a, r1, q1);
+    row_store(B, lane, q0);
+    if (lane + 64 < HR) row_store(B, lane + 64, q1);
     __syncthreads();
 }
 
-// dual_contouring.rs:332-349; false where the reference reaches unreachable!()
-__device__ inline bool grad(const Block& B, int x, int y, int z, int axis, float& g) {
-    const int c = bidx(x, y, z);
-    const int step = axis == 0 ? HB * HB : (axis == 1 ? HB : 1);
-    const bool hp = B.act[c], hl = B.act[c - step], hr = B.act[c + step];
-    if (hp && hl && hr) {
-        g = (B.val[c + step] - B.val[c - step]) * 0.5f;
-        return true;
-    }
-    if (hp && hr) {
-        g = B.val[c + step] - B.val[c];
-        return true;
-    }
-    if (hp && hl) {
-        g = B.val[c] - B.val[c - step];
-        return true;
-    }
-    return false;
-}
-
-// dual_contouring.rs:257-330: crossing of edge (v1, v1 + e_dir) at leaf-local
-// v1, in voxel units of the global grid.  Both ends active, signs differ.
-__device__ inline void crossing(const Block& B, int4 org, int x, int y, int z, int dir, float p[3], float n[3]) {
-    const int c1 = bidx(x, y, z);
-    const int c2 = c1 + (dir == 0 ? HB * HB : (dir == 1 ? HB : 1));
-    const float v1 = B.val[c1], v2 = B.val[c2];
+// Crossing edge (v, v + e_d), v = (x, y, z) leaf-local, both ends active and of
+// different sign (dual_contouring.rs:257-349): the crossing's coordinate along
+// the edge in voxel units of the global grid, and the unit normal.  A gradient
+// without both neighbours is one-sided; one without any is the reference's
+// unreachable!(), reported before this is used.
+__device__ inline float4 edge_crossing(const Block& B, int4 org, int x, int y, int z, int d) {
+    const int step = d == 0 ? HR : (d == 1 ? HB : 1);
+    const int rstep = d == 0 ? HB : (d == 1 ? 1 : 0);
+    const int r1 = ridx(x, y), c1 = r1 * HB + z + 1;
+    const float v1 = B.val[c1], v2 = B.val[c1 + step];
     const float t = (v1 == v2) ? 0.5f : v1 / (v1 - v2);
-    const float px = (float)(org.x + x), py = (float)(org.y + y), pz = (float)(org.z + z);
-    p[0] = dir == 0 ? px + t : px;
-    p[1] = dir == 1 ? py + t : py;
-    p[2] = dir == 2 ? pz + t : pz;
-    const int x2 = x + (dir == 0), y2 = y + (dir == 1), z2 = z + (dir == 2);
-    float nv[3];
+    float g[2][3];
 #pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-        float g1 = 0.0f, g2 = 0.0f;
-        grad(B, x, y, z, ax, g1);  // availability was checked in the edge sweep
-        grad(B, x2, y2, z2, ax, g2);
-        nv[ax] = (1.0f - t) * g1 + t * g2;
+    for (int e = 0; e < 2; ++e) {
+        const int r = r1 + e * rstep, c = c1 + e * step, b = z + 1 + (d == 2 ? e : 0);
+        const float vc = e ? v2 : v1;
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            const int s = ax == 0 ? HR : (ax == 1 ? HB : 1), rs = ax == 0 ? HB : (ax == 1 ? 1 : 0);
+            const float l = B.val[c - s], h = B.val[c + s];
+            const bool hl = (B.row[r - rs] >> (ax == 2 ? b - 1 : b)) & 1u, hr = (B.row[r + rs] >> (ax == 2 ? b + 1 : b)) & 1u;
+            g[e][ax] = (hl && hr) ? (h - l) * 0.5f : (hr ? h - vc : vc - l);
+        }
     }
-    const float len = sqrt_rn((nv[0] * nv[0] + nv[1] * nv[1]) + nv[2] * nv[2]);
-    n[0] = nv[0] / len;
-    n[1] = nv[1] / len;
-    n[2] = nv[2] / len;
+    float n[3];
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) n[ax] = (1.0f - t) * g[0][ax] + t * g[1][ax];
+    const float len = sqrt_rn((n[0] * n[0] + n[1] * n[1]) + n[2] * n[2]);
+    const float base = (float)(d == 0 ? org.x + x : (d == 1 ? org.y + y : org.z + z));
+    return make_float4(base + t, n[0] / len, n[1] / len, n[2] / len);
 }
 
-// dual_contouring.rs:410-423 (base offset, direction) and utils.rs:86-95
-__constant__ int8_t kEdge[12][4] = {{0, 0, 0, 0}, {0, 0, 0, 1}, {0, 0, 0, 2}, {1, 0, 0, 1}, {1, 0, 0, 2}, {0, 0, 1, 0},
-                                    {0, 0, 1, 1}, {0, 1, 0, 0}, {0, 1, 0, 2}, {1, 0, 1, 1}, {0, 1, 1, 0}, {1, 1, 0, 2}};
-__constant__ int8_t kCube[8][3] = {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0},
-                                   {0, 0, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 1}};
-// dual_contouring.rs:389-408
-__constant__ int8_t kCell[3][4][3] = {{{0, 0, 0}, {0, 0, -1}, {0, -1, -1}, {0, -1, 0}},
-                                      {{0, 0, 0}, {-1, 0, 0}, {-1, 0, -1}, {0, 0, -1}},
-                                      {{0, -1, 0}, {-1, -1, 0}, {-1, 0, 0}, {0, 0, 0}}};
+// EDGE_OFFSETS (dual_contouring.rs:410-423): edge e's base offset and axis,
+// five bits each (dx, dy, dz, axis).
+constexpr uint64_t edge_code(int dx, int dy, int dz, int d) { return (uint64_t)(dx | dy << 1 | dz << 2 | d << 3); }
+constexpr uint64_t EDGE_CODES =
+    edge_code(0, 0, 0, 0) | edge_code(0, 0, 0, 1) << 5 | edge_code(0, 0, 0, 2) << 10 | edge_code(1, 0, 0, 1) << 15 |
+    edge_code(1, 0, 0, 2) << 20 | edge_code(0, 0, 1, 0) << 25 | edge_code(0, 0, 1, 1) << 30 |
+    edge_code(0, 1, 0, 0) << 35 | edge_code(0, 1, 0, 2) << 40 | edge_code(1, 0, 1, 1) << 45 |
+    edge_code(0, 1, 1, 0) << 50 | edge_code(1, 1, 0, 2) << 55;
 
 // Opt-in vertex placement (BS_DC_VERTEX_QEF_F64; the reference has only the
 // particle iteration): the point minimising sum_i (n_i . (x - p_i))^2 over the
@@ -214,124 +265,174 @@ __device__ inline void qef_point(const float (&P)[12][3], const float (&N)[12][3
     out[2] = (float)fmin(fmax(x[2], (double)cz0), (double)cz0 + 1.0);
 }
 
+// Bound by latency at 12 to 15 waves per CU (120 VGPRs, 10.7 KB of LDS), the
+// staging loads first.  The bit words replace per-voxel scans, a shared edge is
+// computed once instead of by its four cells, and a cell's loop runs over its
+// own edges instead of all twelve: 1.45 ms for 571 k leaves with 12.8 M cells
+// (9.07 ms with those scans and per-cell edges, 3200 vector instructions a
+// leaf), 0.84 TB/s of leaf data.
 template <bool QEF>
 __global__ __launch_bounds__(64) void k_dc_cells(uint64_t n_leaves, DcArgs a) {
     __shared__ Block B;
-    __shared__ uint16_t cell_list[512];  // offset x*64 + y*8 + z of each listed cell
     const int lane = threadIdx.x;
     const int x = lane >> 3, y = lane & 7;
-    for (uint64_t leaf = blockIdx.x; leaf < n_leaves; leaf += gridDim.x) {
+    const uint64_t span = dc_span(n_leaves);
+    for (uint64_t v = blockIdx.x; v < span; v += gridDim.x) {
+        const uint64_t leaf = dc_leaf(v);
+        if (leaf >= n_leaves) continue;
         const int4 org = a.origins[leaf];
         stage_block(B, a, org, lane);
-        // edge sweep (dual_contouring.rs:352-387): every crossing edge from a
-        // voxel of this leaf needs all six gradients
-        bool bad = false;
-        for (int z = 0; z < 8; ++z) {
-            const int c = bidx(x, y, z);
-            if (!B.act[c]) continue;
-            const uint32_t s1 = __float_as_uint(B.val[c]) >> 31;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const int c2 = c + (d == 0 ? HB * HB : (d == 1 ? HB : 1));
-                if (!B.act[c2] || (__float_as_uint(B.val[c2]) >> 31) == s1) continue;
-                float g;
-                const int x2 = x + (d == 0), y2 = y + (d == 1), z2 = z + (d == 2);
-#pragma unroll
-                for (int ax = 0; ax < 3; ++ax) bad |= !grad(B, x, y, z, ax, g) || !grad(B, x2, y2, z2, ax, g);
+        uint32_t cells;
+        {
+            // the words of rows (x - 1 .. x + 2, y - 1 .. y + 2) that the row's own edges and cells meet
+            const int r = ridx(x, y);
+            const uint32_t w00 = B.row[r], w10 = B.row[r + HB], w01 = B.row[r + 1], w11 = B.row[r + HB + 1];
+            const uint32_t wm0 = B.row[r - HB], w20 = B.row[r + 2 * HB], w0m = B.row[r - 1], w02 = B.row[r + 2];
+            const uint32_t w1m = B.row[r + HB - 1], wm1 = B.row[r - HB + 1];
+            // edge sweep (dual_contouring.rs:352-387): every crossing edge from a voxel of this leaf needs
+            // all six gradients; bit z + 1 of g** says that voxel z of that row has its three
+            const uint32_t g00 = w00 & (w00 << 1 | w00 >> 1) & (wm0 | w10) & (w0m | w01);
+            const uint32_t g10 = w10 & (w10 << 1 | w10 >> 1) & (w00 | w20) & (w1m | w11);
+            const uint32_t g01 = w01 & (w01 << 1 | w01 >> 1) & (wm1 | w11) & (w00 | w02);
+            const uint32_t n00 = w00 >> 16, n10 = w10 >> 16, n01 = w01 >> 16, n11 = w11 >> 16;
+            const uint32_t bad = (w00 & w10 & (n00 ^ n10) & ~(g00 & g10)) | (w00 & w01 & (n00 ^ n01) & ~(g00 & g01)) |
+                                 (w00 & w00 >> 1 & (n00 ^ n00 >> 1) & ~(g00 & g00 >> 1));
+            if (__ballot((bad & 0x1FEu) != 0) && lane == 0) atomicOr(a.fail, 1u);
+            // cells with all eight corners active and mixed signs (dual_contouring.rs:176-247)
+            const uint32_t all = w00 & w10 & w01 & w11, some = n00 | n10 | n01 | n11, every = n00 & n10 & n01 & n11;
+            cells = ((all & all >> 1 & (some | some >> 1) & ~(every & every >> 1)) >> 1) & 0xFFu;
+            const uint64_t cw = gather_word(cells, y), nw = gather_word((n00 >> 1) & 0xFFu, y);
+            if (y == 0) {
+                a.cell_mask[leaf * 8 + x] = cw;
+                a.neg_mask[leaf * 8 + x] = nw;
             }
         }
-        if (bad) atomicOr(a.fail, 1u);
-        // cells (dual_contouring.rs:176-247): the leaf's cells with all eight
-        // corners active and mixed signs are listed first, then each lane
-        // takes one listed cell, so the feature-point work runs on full waves
-        uint32_t present = 0;
-        int n_cells = 0;
-        for (int z = 0; z < 8; ++z) {
-            bool all = true;
-            uint32_t neg = 0;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int c = bidx(x + kCube[i][0], y + kCube[i][1], z + kCube[i][2]);
-                all &= B.act[c] != 0;
-                neg |= (__float_as_uint(B.val[c]) >> 31) << i;
+        if (!__ballot(cells != 0)) {
+            __syncthreads();
+            continue;
+        }
+        // the crossing edges between corners 0..8, counted per row and listed (row-major, axis, z)
+        uint32_t n_edges = 0;
+        for (int r0 = 0; r0 < CR; r0 += 64) {
+            const int r = r0 + lane, rx = r / CB, ry = r % CB;
+            uint32_t e = 0;
+            if (r < CR) {
+                const uint32_t w = B.row[ridx(rx, ry)], wx = B.row[ridx(rx, ry) + HB], wy = B.row[ridx(rx, ry) + 1];
+                const uint32_t ex = rx < 8 ? (w & wx & (w ^ wx) >> 16) >> 1 & 0x1FFu : 0;
+                const uint32_t ey = ry < 8 ? (w & wy & (w ^ wy) >> 16) >> 1 & 0x1FFu : 0;
+                const uint32_t ez = (w & w >> 1 & (w ^ w >> 1) >> 16) >> 1 & 0xFFu;
+                e = ex | ey << 9 | ez << 18;
             }
-            const bool surface = all && neg != 0 && neg != 0xFFu;
-            const unsigned long long b = __ballot(surface);
-            if (surface) {
-                present |= 1u << z;
-                cell_list[n_cells + __popcll(b & ((1ull << lane) - 1))] = (uint16_t)((lane << 3) | z);
+            uint32_t total;
+            uint32_t at = n_edges + wave_prefix((uint32_t)__popc(e), lane, total);
+            if (r < CR) {
+                B.edge_row[r] = e;
+                B.edge_pre[r] = at;
             }
-            n_cells += __popcll(b);
+            for (; e && at < EDGE_LDS; e &= e - 1, ++at) B.list[at] = (uint16_t)(r << 5 | (__ffs((int)e) - 1));
+            n_edges += total;
         }
         __syncthreads();
-        for (int k = lane; k < n_cells; k += 64) {
-            const int cell = cell_list[k];
-            const int x = cell >> 6, y = (cell >> 3) & 7, z = cell & 7;
-            // crossings in EDGE_OFFSETS order; all indexing static so they stay in registers
-            float P[12][3], N[12][3];
+        // one lane per listed edge (past EDGE_LDS each cell computes its own)
+        for (uint32_t k = lane; k < min(n_edges, (uint32_t)EDGE_LDS); k += 64) {
+            const int code = B.list[k], r = code >> 5, bit = code & 31, d = bit >= 18 ? 2 : (bit >= 9 ? 1 : 0);
+            B.edge[k] = edge_crossing(B, org, r / CB, r % CB, bit - 9 * d, d);
+        }
+        __syncthreads();
+        uint32_t n_cells;
+        {
+            uint32_t at = wave_prefix((uint32_t)__popc(cells), lane, n_cells);
+            for (uint32_t c = cells; c; c &= c - 1, ++at) B.list[at] = (uint16_t)((lane << 3) | (__ffs((int)c) - 1));
+        }
+        __syncthreads();
+        for (uint32_t k0 = 0; k0 < n_cells; k0 += 64) {
+            const uint32_t k = k0 + lane;
+            const bool on = k < n_cells;
+            const int cell = B.list[on ? k : 0];
+            const int cx0 = cell >> 6, cy0 = (cell >> 3) & 7, cz0 = cell & 7;
+            // the cell's crossing edges in EDGE_OFFSETS order, packed to the front
             uint32_t valid = 0;
 #pragma unroll
             for (int e = 0; e < 12; ++e) {
-                const int ex = x + kEdge[e][0], ey = y + kEdge[e][1], ez = z + kEdge[e][2], d = kEdge[e][3];
-                const int c1 = bidx(ex, ey, ez);
-                const int c2 = c1 + (d == 0 ? HB * HB : (d == 1 ? HB : 1));
-                P[e][0] = P[e][1] = P[e][2] = 0.0f;
-                N[e][0] = N[e][1] = N[e][2] = 0.0f;
-                if ((__float_as_uint(B.val[c1]) >> 31) == (__float_as_uint(B.val[c2]) >> 31)) continue;
-                crossing(B, org, ex, ey, ez, d, P[e], N[e]);
-                valid |= 1u << e;
+                constexpr uint64_t codes = EDGE_CODES;
+                const int code = (int)(codes >> (5 * e)) & 31, d = code >> 3;
+                const uint32_t w = B.edge_row[(cx0 + (code & 1)) * CB + cy0 + ((code >> 1) & 1)];
+                valid |= ((w >> (9 * d + cz0 + ((code >> 2) & 1))) & 1u) << e;
             }
-            float* out = a.cell_pts + (leaf * 512 + (uint64_t)cell) * 3;
+            const int cnt = __popc(valid);
+            int most = on ? cnt : 0;
+#pragma unroll
+            for (int s = 32; s >= 1; s >>= 1) most = max(most, __shfl_xor(most, s));
+            most = __builtin_amdgcn_readfirstlane(most);
+            // point and normal of the lane's edge e: from the list, or past it computed here
+            auto fetch = [&](int e, float (&p)[3], float (&n)[3]) {
+                const int code = (int)(EDGE_CODES >> (5 * e)) & 31, d = code >> 3;
+                const int ex = cx0 + (code & 1), ey = cy0 + ((code >> 1) & 1), ez = cz0 + ((code >> 2) & 1);
+                const uint32_t w = B.edge_row[ex * CB + ey];
+                const uint32_t at = B.edge_pre[ex * CB + ey] + __popc(w & ((1u << (9 * d + ez)) - 1u));
+                const float4 q = at < EDGE_LDS ? B.edge[at] : edge_crossing(B, org, ex, ey, ez, d);
+                p[0] = d == 0 ? q.x : (float)(org.x + ex);
+                p[1] = d == 1 ? q.x : (float)(org.y + ey);
+                p[2] = d == 2 ? q.x : (float)(org.z + ez);
+                n[0] = q.y, n[1] = q.z, n[2] = q.w;
+            };
+            // the first KEEP stay in registers (a smooth surface crosses 3 to 6 of a cell's edges)
+            constexpr int KEEP = QEF ? 12 : 6;
+            float P[KEEP][3], N[KEEP][3];
+#pragma unroll
+            for (int j = 0; j < KEEP; ++j) {
+                P[j][0] = P[j][1] = P[j][2] = N[j][0] = N[j][1] = N[j][2] = 0.0f;
+                if (j >= most || !valid) continue;
+                fetch(__ffs((int)valid) - 1, P[j], N[j]);
+                valid &= valid - 1;
+            }
+            if (!on) continue;
+            float* out = a.cell_pts + (leaf * 512 + (uint64_t)k) * 3;
             if constexpr (QEF) {
-                qef_point(P, N, valid, (float)(org.x + x), (float)(org.y + y), (float)(org.z + z), out);
+                qef_point(P, N, (1u << cnt) - 1u, (float)(org.x + cx0), (float)(org.y + cy0), (float)(org.z + cz0), out);
                 continue;
-            }
-            // find_feature_point (dual_contouring.rs:433-458)
-            const float fc = (float)__popc(valid);
-            float cx = 0.0f, cy = 0.0f, cz = 0.0f;
+            } else {
+                // find_feature_point (dual_contouring.rs:433-458)
+                const float fc = (float)cnt;
+                float cx = 0.0f, cy = 0.0f, cz = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 12; ++e)
-                if (valid & (1u << e)) cx = cx + P[e][0], cy = cy + P[e][1], cz = cz + P[e][2];
-            cx = cx / fc, cy = cy / fc, cz = cz / fc;
-            for (int it = 0; it < 50; ++it) {
-                float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 12; ++e) {
-                    if (!(valid & (1u << e))) continue;
-                    const float d = (N[e][0] * (cx - P[e][0]) + N[e][1] * (cy - P[e][1])) + N[e][2] * (cz - P[e][2]);
-                    fx = fx + (N[e][0] * -1.0f) * d;
-                    fy = fy + (N[e][1] * -1.0f) * d;
-                    fz = fz + (N[e][2] * -1.0f) * d;
+                for (int j = 0; j < KEEP; ++j)
+                    if (j < most && j < cnt) cx = cx + P[j][0], cy = cy + P[j][1], cz = cz + P[j][2];
+                for (uint32_t rest = valid; rest; rest &= rest - 1) {
+                    float p[3], n[3];
+                    fetch(__ffs((int)rest) - 1, p, n);
+                    cx = cx + p[0], cy = cy + p[1], cz = cz + p[2];
                 }
-                const float damping = 1.0f - (float)it / 50.0f;
-                cx = cx + (fx * damping) / fc;
-                cy = cy + (fy * damping) / fc;
-                cz = cz + (fz * damping) / fc;
-                if ((fx * fx + fy * fy) + fz * fz < 1e-6f) break;
+                cx = cx / fc, cy = cy / fc, cz = cz / fc;
+                for (int it = 0; it < 50; ++it) {
+                    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+                    auto pull = [&](const float (&p)[3], const float (&n)[3]) {
+                        const float d = (n[0] * (cx - p[0]) + n[1] * (cy - p[1])) + n[2] * (cz - p[2]);
+                        fx = fx + (n[0] * -1.0f) * d;
+                        fy = fy + (n[1] * -1.0f) * d;
+                        fz = fz + (n[2] * -1.0f) * d;
+                    };
+#pragma unroll
+                    for (int j = 0; j < KEEP; ++j)
+                        if (j < most && j < cnt) pull(P[j], N[j]);
+                    for (uint32_t rest = valid; rest; rest &= rest - 1) {
+                        float p[3], n[3];
+                        fetch(__ffs((int)rest) - 1, p, n);
+                        pull(p, n);
+                    }
+                    const float damping = 1.0f - (float)it / 50.0f;
+                    cx = cx + (fx * damping) / fc;
+                    cy = cy + (fy * damping) / fc;
+                    cz = cz + (fz * damping) / fc;
+                    if ((fx * fx + fy * fy) + fz * fz < 1e-6f) break;
+                }
+                out[0] = cx;
+                out[1] = cy;
+                out[2] = cz;
             }
-            out[0] = cx;
-            out[1] = cy;
-            out[2] = cz;
         }
-        // cell presence mask: word x, bits y*8+z
-        const uint64_t w = gather_word(present, y);
-        if (y == 0) a.cell_mask[leaf * 8 + x] = w;
         __syncthreads();
     }
-}
-
-// Cell point at leaf-local (x, y, z) in -1..7, through the 27-leaf table.
-__device__ inline bool cell_at(const Block& B, const DcArgs& a, int x, int y, int z, float p[3]) {
-    const int dx = x >> 3, dy = y >> 3, dz = z >> 3;
-    const int32_t s = B.nb[(dx + 1) * 9 + (dy + 1) * 3 + (dz + 1)];
-    if (s < 0) return false;
-    const int o = ((x & 7) << 6) | ((y & 7) << 3) | (z & 7);
-    if (!((a.cell_mask[(uint64_t)s * 8 + (o >> 6)] >> (o & 63)) & 1ull)) return false;
-    const float* q = a.cell_pts + ((uint64_t)s * 512 + o) * 3;
-    p[0] = q[0];
-    p[1] = q[1];
-    p[2] = q[2];
-    return true;
 }
 
 // Triangle3::is_degenerate (triangle3.rs:272-275) of the scaled corners
@@ -342,103 +443,143 @@ __device__ inline bool degenerate(const float a[3], const float b[3], const floa
     return (cx * cx + cy * cy) + cz * cz == 0.0f;
 }
 
-// The quad of crossing edge d from voxel (x, y, z) with sign bit s1
-// (dual_contouring.rs:93-174, :62-79): its two triangles, scaled, in q, and
-// whether each survives the degenerate-triangle filter; false when one of the
-// four cells around the edge is missing.
-__device__ inline bool edge_quad(const Block& B, const DcArgs& a, int x, int y, int z, int d, uint32_t s1,
-                                 float q[6][3], bool keep[2]) {
-    float p[4][3];
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        ok = ok && cell_at(B, a, x + kCell[d][k][0], y + kCell[d][k][1], z + kCell[d][k][2], p[k]);
-    if (!ok) return false;
-    // [p0, p1, p2, p2, p3, p0], with 1<->2 and 4<->5 swapped when v is negative
-    const int f1 = s1 ? 2 : 1, f2 = s1 ? 1 : 2, f4 = s1 ? 0 : 3, f5 = s1 ? 3 : 0;
-    const int f[6] = {0, f1, f2, 2, f4, f5};
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const int src = f[k];
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            q[k][j] = (src == 0 ? p[0][j] : src == 1 ? p[1][j] : src == 2 ? p[2][j] : p[3][j]) * a.voxel_size;
-    }
-    keep[0] = !degenerate(q[0], q[1], q[2]);
-    keep[1] = !degenerate(q[3], q[4], q[5]);
-    return true;
-}
-
-// Crossing edges from the voxels of this lane's z-row, in the sequential
-// order (z, then axis); emit(z, d) is called for each.
-template <class F>
-__device__ inline void row_edges(const Block& B, int x, int y, F&& emit) {
-    for (int z = 0; z < 8; ++z) {
-        const int c = bidx(x, y, z);
-        if (!B.act[c]) continue;
-        const uint32_t s1 = __float_as_uint(B.val[c]) >> 31;
-        for (int d = 0; d < 3; ++d) {
-            const int c2 = c + (d == 0 ? HB * HB : (d == 1 ? HB : 1));
-            if (!B.act[c2] || (__float_as_uint(B.val[c2]) >> 31) == s1) continue;
-            emit(z, d);
-        }
-    }
-}
+// dual_contouring.rs:389-408: the four cells around an edge, as offsets 0 or
+// -1 on the two other axes, in three bits per cell (x, y, z; set = -1).
+constexpr uint32_t cell_codes(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3) { return c0 | c1 << 3 | c2 << 6 | c3 << 9; }
+constexpr uint32_t CELLS_X = cell_codes(0, 4, 6, 2), CELLS_Y = cell_codes(0, 1, 5, 4), CELLS_Z = cell_codes(2, 3, 1, 0);
 
 // WRITE = false: triangles per leaf into tri_count.  WRITE = true: the
-// triangles at tri_off[leaf].  A leaf's crossing edges are listed in the
-// sequential order (z-rows = lanes, then z, then axis), then taken 64 at a
-// time, one per lane; each lane's triangles go after those of the edges
-// before it (two ballots give the prefix), so the soup keeps that order.
+// triangles at tri_off[leaf].  Everything but the points comes from the
+// presence masks of the leaf and its seven neighbours towards -x, -y, -z and
+// the sign masks of the leaf and its three neighbours towards +x, +y, +z
+// (704 B a leaf).  A leaf's quads (crossing edges whose four cells exist, so
+// whose ends are active) are listed in the sequential order (z-rows = lanes,
+// then z, then axis) and taken 64 at a time, one per lane; each lane's
+// triangles go after those of the quads before it (two ballots give the
+// prefix), assembled in LDS and written coalesced, so the soup keeps that
+// order (dual_contouring.rs:93-174, :62-79).  At 571 k leaves and 38.4 M
+// triangles counting takes 0.35 ms and writing 0.73 ms (1.9 TB/s of soup; the
+// scattered point fetches bound it); 5.45 and 7.18 ms when both staged the
+// leaf's values again and looked each cell up in memory.
 template <bool WRITE>
 __global__ __launch_bounds__(64) void k_dc_triangles(uint64_t n_leaves, DcArgs a, uint32_t* __restrict__ tri_count,
                                                      const uint64_t* __restrict__ tri_off, float* __restrict__ out) {
-    __shared__ Block B;
-    __shared__ uint32_t lane_cnt[64];
-    __shared__ uint16_t edges[512 * 3];  // lane << 5 | z << 2 | axis
+    __shared__ int32_t slot[8];        // leaves at offsets 0 or -1 (bit 0 x, bit 1 y, bit 2 z set = -1)
+    __shared__ uint64_t word[64];      // their presence words
+    __shared__ uint16_t before[64];    // cells of the leaf's words before
+    __shared__ uint16_t quads[512 * 3];  // lane << 5 | z << 2 | axis, sign in bit 15
+    __shared__ float tri[WRITE ? 64 * 18 : 1];
     const int lane = threadIdx.x;
     const int x = lane >> 3, y = lane & 7;
     const unsigned long long lt = (1ull << lane) - 1;
-    for (uint64_t leaf = blockIdx.x; leaf < n_leaves; leaf += gridDim.x) {
-        stage_block(B, a, a.origins[leaf], lane);
-        uint32_t cnt = 0;
-        row_edges(B, x, y, [&](int, int) { ++cnt; });
-        lane_cnt[lane] = cnt;
-        __syncthreads();
-        uint32_t before = 0, n_edges = 0;
-        for (int l = 0; l < 64; ++l) {
-            before += l < lane ? lane_cnt[l] : 0;
-            n_edges += lane_cnt[l];
+    const uint64_t span = dc_span(n_leaves);
+    for (uint64_t v = blockIdx.x; v < span; v += gridDim.x) {
+        const uint64_t leaf = dc_leaf(v);
+        if (leaf >= n_leaves) continue;
+        const int4 org = a.origins[leaf];
+        int32_t s = (int32_t)leaf;
+        if (lane >= 1 && lane < 11) {
+            const int k = lane;  // 1..7: towards -, 8..10: towards + on one axis
+            const int dx = k < 8 ? -(k & 1) : k == 8, dy = k < 8 ? -((k >> 1) & 1) : k == 9,
+                      dz = k < 8 ? -((k >> 2) & 1) : k == 10;
+            s = a.map.find((org.x >> 3) + dx, (org.y >> 3) + dy, (org.z >> 3) + dz);
         }
-        row_edges(B, x, y, [&](int z, int d) { edges[before++] = (uint16_t)((lane << 5) | (z << 2) | d); });
+        if (lane < 8) slot[lane] = s;
+        const int32_t sx = __builtin_amdgcn_readlane(s, 8), sy = __builtin_amdgcn_readlane(s, 9),
+                      sz = __builtin_amdgcn_readlane(s, 10);
+        const int32_t sq = __shfl(s, lane >> 3);
+        const uint64_t w = sq >= 0 ? a.cell_mask[(uint64_t)sq * 8 + (lane & 7)] : 0;
+        const uint8_t* nb = reinterpret_cast<const uint8_t*>(a.neg_mask);  // byte y of word x is row (x, y)
+        const uint32_t n0 = nb[leaf * 64 + lane];
+        const int32_t lx = x < 7 ? (int32_t)leaf : sx, ly = y < 7 ? (int32_t)leaf : sy;
+        const uint32_t nx = lx >= 0 ? nb[(uint64_t)lx * 64 + (((x + 1) & 7) << 3 | y)] : 0;
+        const uint32_t ny = ly >= 0 ? nb[(uint64_t)ly * 64 + (x << 3 | ((y + 1) & 7))] : 0;
+        const uint32_t nz = sz >= 0 ? nb[(uint64_t)sz * 64 + lane] : 0;
+        word[lane] = w;
+        uint32_t pre = (uint32_t)__popcll(w);
+        const uint32_t own = pre;
+#pragma unroll
+        for (int d = 1; d < 8; d <<= 1) {
+            const uint32_t u = (uint32_t)__shfl_up((int)pre, d, 64);
+            if ((lane & 7) >= d) pre += u;
+        }
+        before[lane] = (uint16_t)(pre - own);
+        __syncthreads();
+        // presence bits z - 1 .. 7 of the cell rows (x, y), (x - 1, y), (x, y - 1), (x - 1, y - 1): bit z + 1
+        auto cell_row = [&](int mx, int my) {
+            const int cx = x - mx, cy = y - my, q = (cx < 0) | (cy < 0) << 1, wi = cx & 7, sh = (cy & 7) * 8;
+            return (uint32_t)((word[q * 8 + wi] >> sh) & 0xFFu) << 1 | (uint32_t)((word[(q | 4) * 8 + wi] >> (sh + 7)) & 1u);
+        };
+        const uint32_t c00 = cell_row(0, 0), cm0 = cell_row(1, 0), c0m = cell_row(0, 1), cmm = cell_row(1, 1);
+        const uint32_t ax = c00 & c0m, ay = c00 & cm0, az = ax & cm0 & cmm;
+        const uint32_t qx = ax >> 1 & ax & (n0 ^ nx), qy = ay >> 1 & ay & (n0 ^ ny),
+                       qz = az >> 1 & (n0 ^ (n0 >> 1 | (nz & 1u) << 7)) & 0xFFu;
+        uint32_t n_quads;
+        uint32_t at = wave_prefix((uint32_t)(__popc(qx) + __popc(qy) + __popc(qz)), lane, n_quads);
+        for (uint32_t any = qx | qy | qz; any; any &= any - 1) {
+            const int z = __ffs((int)any) - 1;
+            const uint32_t code = (uint32_t)(lane << 5 | z << 2) | ((n0 >> z) & 1u) << 15;
+            if (qx >> z & 1u) quads[at++] = (uint16_t)code;
+            if (qy >> z & 1u) quads[at++] = (uint16_t)(code | 1u);
+            if (qz >> z & 1u) quads[at++] = (uint16_t)(code | 2u);
+        }
         __syncthreads();
         const uint64_t base = WRITE ? tri_off[leaf] : 0;
         uint32_t done = 0;
-        for (uint32_t k0 = 0; k0 < n_edges; k0 += 64) {
+        for (uint32_t k0 = 0; k0 < n_quads; k0 += 64) {
             const uint32_t k = k0 + (uint32_t)lane;
             float q[6][3];
             bool keep[2] = {false, false};
-            if (k < n_edges) {
-                const int e = edges[k];
-                const int el = e >> 5, ex = el >> 3, ey = el & 7, ez = (e >> 2) & 7, d = e & 3;
-                const uint32_t s1 = __float_as_uint(B.val[bidx(ex, ey, ez)]) >> 31;
-                if (!edge_quad(B, a, ex, ey, ez, d, s1, q, keep)) keep[0] = keep[1] = false;
+            if (k < n_quads) {
+                const uint32_t e = quads[k];
+                const int el = (e >> 5) & 63, ex = el >> 3, ey = el & 7, ez = (e >> 2) & 7, d = e & 3;
+                const bool s1 = e >> 15;
+                const uint32_t codes = d == 0 ? CELLS_X : (d == 1 ? CELLS_Y : CELLS_Z);
+                float p[4][3];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const uint32_t m = codes >> (3 * c);
+                    const int cx = ex - (int)(m & 1), cy = ey - (int)(m >> 1 & 1), cz = ez - (int)(m >> 2 & 1);
+                    const int lq = (cx < 0) | (cy < 0) << 1 | (cz < 0) << 2, wi = lq * 8 + (cx & 7);
+                    const int bit = (cy & 7) * 8 + (cz & 7);
+                    const uint32_t rank = before[wi] + (uint32_t)__popcll(word[wi] & ((1ull << bit) - 1));
+                    const float* src = a.cell_pts + ((uint64_t)(uint32_t)slot[lq] * 512 + rank) * 3;
+                    p[c][0] = src[0];
+                    p[c][1] = src[1];
+                    p[c][2] = src[2];
+                }
+                // [p0, p1, p2, p2, p3, p0], with 1<->2 and 4<->5 swapped when v is negative
+                const int f1 = s1 ? 2 : 1, f2 = s1 ? 1 : 2, f4 = s1 ? 0 : 3, f5 = s1 ? 3 : 0;
+                const int f[6] = {0, f1, f2, 2, f4, f5};
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    const int src = f[c];
+#pragma unroll
+                    for (int j = 0; j < 3; ++j)
+                        q[c][j] = (src == 0 ? p[0][j] : src == 1 ? p[1][j] : src == 2 ? p[2][j] : p[3][j]) * a.voxel_size;
+                }
+                keep[0] = !degenerate(q[0], q[1], q[2]);
+                keep[1] = !degenerate(q[3], q[4], q[5]);
             }
             const unsigned long long b0 = __ballot(keep[0]), b1 = __ballot(keep[1]);
+            const uint32_t n_tri = (uint32_t)(__popcll(b0) + __popcll(b1));
             if (WRITE) {
-                uint64_t at = base + done + (uint64_t)(__popcll(b0 & lt) + __popcll(b1 & lt));
+                uint32_t to = (uint32_t)(__popcll(b0 & lt) + __popcll(b1 & lt));
 #pragma unroll
                 for (int tr = 0; tr < 2; ++tr) {
                     if (!keep[tr]) continue;
-                    float* o = out + at * 9;
 #pragma unroll
                     for (int kk = 0; kk < 3; ++kk)
 #pragma unroll
-                        for (int j = 0; j < 3; ++j) o[kk * 3 + j] = q[3 * tr + kk][j];
-                    ++at;
+                        for (int j = 0; j < 3; ++j) tri[to * 9 + kk * 3 + j] = q[3 * tr + kk][j];
+                    ++to;
                 }
+                __syncthreads();
+                float* o = out + 9 * (base + done);
+                for (uint32_t i = lane; i < 9 * n_tri; i += 64) o[i] = tri[i];
+                __syncthreads();
             }
-            done += (uint32_t)(__popcll(b0) + __popcll(b1));
+            done += n_tri;
         }
         if (!WRITE && lane == 0) tri_count[leaf] = done;
         __syncthreads();
@@ -465,11 +606,15 @@ struct DcWork {
     uint32_t* fail;
     float* cell_pts;
     uint64_t* cell_mask;
+    uint64_t* neg_mask;
     uint32_t* tri_count;
     uint64_t* tri_off;
     void* scan_tmp;
     size_t scan_bytes;
 };
+
+// A multiple of 8 workgroups (dc_leaf), enough to fill 256 CUs several times.
+unsigned dc_grid(uint64_t n) { return (unsigned)std::min<uint64_t>(dc_span(n), 8192); }
 
 uint64_t hash_capacity(uint64_t n) {
     uint64_t cap = 1024;
@@ -499,9 +644,10 @@ uint64_t dc_count(hipStream_t st, const bs_volume* vol, float voxel_size, bool q
     a.values = vol->values;
     a.cell_pts = w.cell_pts;
     a.cell_mask = w.cell_mask;
+    a.neg_mask = w.neg_mask;
     a.voxel_size = voxel_size;
     a.fail = w.fail;
-    const unsigned grid = (unsigned)std::min<uint64_t>(n, 8192);
+    const unsigned grid = dc_grid(n);
     if (qef)
         k_dc_cells<true><<<grid, 64, 0, st>>>(n, a);
     else
@@ -524,7 +670,7 @@ uint64_t dc_count(hipStream_t st, const bs_volume* vol, float voxel_size, bool q
 }
 
 void dc_write(hipStream_t st, uint64_t n, const DcArgs& a, const DcWork& w, float* out) {
-    const unsigned grid = (unsigned)std::min<uint64_t>(n, 8192);
+    const unsigned grid = dc_grid(n);
     k_dc_triangles<true><<<grid, 64, 0, st>>>(n, a, nullptr, w.tri_off, out);
     BS_HIP(hipGetLastError());
 }
@@ -549,7 +695,8 @@ constexpr uint64_t NA_CELLS = NA_KEYS + al256(8 * DC_NOALLOC_HASH_CAP);
 constexpr uint64_t NA_FAIL = NA_CELLS + al256(4 * DC_NOALLOC_HASH_CAP);
 constexpr uint64_t NA_PTS = NA_FAIL + 256;
 constexpr uint64_t NA_CMASK = NA_PTS + al256(4ull * 512 * 3 * DC_NOALLOC_MAX_LEAVES);
-constexpr uint64_t NA_TCNT = NA_CMASK + al256(64ull * DC_NOALLOC_MAX_LEAVES);
+constexpr uint64_t NA_NMASK = NA_CMASK + al256(64ull * DC_NOALLOC_MAX_LEAVES);
+constexpr uint64_t NA_TCNT = NA_NMASK + al256(64ull * DC_NOALLOC_MAX_LEAVES);
 constexpr uint64_t NA_TOFF = NA_TCNT + al256(4ull * DC_NOALLOC_MAX_LEAVES);
 constexpr uint64_t NA_SCAN = NA_TOFF + al256(8ull * (DC_NOALLOC_MAX_LEAVES + 1));
 constexpr uint64_t NA_BYTES = NA_SCAN + DC_NOALLOC_SCAN_BYTES;
@@ -589,7 +736,7 @@ static unsigned char* dc_noalloc_ptr(int device) {
 
 // DualContouringMesher::default().with_voxel_size(h).mesh(volume): the
 // triangle soup (n_tris * 9 floats) in device memory owned by the caller
-// (hipFree), or nullptr for no triangle.
+// (free_block), or nullptr for no triangle.
 void dual_contour_device(bs_ctx* ctx, bs_volume* vol, float voxel_size, float** out_dev, uint64_t* n_tris,
                          bs_dc_stats* stats) {
     hipStream_t st = ctx->stream;
@@ -626,6 +773,7 @@ void dual_contour_device(bs_ctx* ctx, bs_volume* vol, float voxel_size, float** 
     w.fail = ctx->scratch.as<uint32_t>(S_DC_FAIL, 1);
     w.cell_pts = ctx->scratch.as<float>(S_DC_CELLS, n * 512 * 3);
     w.cell_mask = ctx->scratch.as<uint64_t>(S_DC_CELLMASK, n * 8);
+    w.neg_mask = ctx->scratch.as<uint64_t>(S_DC_NEGMASK, n * 8);
     w.tri_count = ctx->scratch.as<uint32_t>(S_DC_TRICNT, n);
     w.tri_off = ctx->scratch.as<uint64_t>(S_DC_TRIOFF, n + 1);
     BS_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, w.scan_bytes, w.tri_count, w.tri_off, (int)n, st));
@@ -634,19 +782,13 @@ void dual_contour_device(bs_ctx* ctx, bs_volume* vol, float voxel_size, float** 
     DcArgs a{};
     const uint64_t total = dc_count(st, vol, voxel_size, ctx->dc_vertex == BS_DC_VERTEX_QEF_F64, w, a);
     if (total) {
-        float* out = nullptr;
-        BS_HIP(hipMalloc(&out, sizeof(float) * 9 * total));
-        hipError_t le = hipSuccess;
+        float* out = static_cast<float*>(alloc_block(sizeof(float) * 9 * total));
         try {
             dc_write(st, n, a, w, out);
+            BS_HIP(hipStreamSynchronize(st));
         } catch (...) {
-            (void)hipFree(out);
+            free_block(out);
             throw;
-        }
-        le = hipStreamSynchronize(st);
-        if (le != hipSuccess) {
-            (void)hipFree(out);
-            BS_HIP(le);
         }
         *out_dev = out;
     }
@@ -691,6 +833,7 @@ void dual_contour_into(bs_ctx* ctx, const bs_volume* vol, float voxel_size, floa
     w.fail = reinterpret_cast<uint32_t*>(base + NA_FAIL);
     w.cell_pts = reinterpret_cast<float*>(base + NA_PTS);
     w.cell_mask = reinterpret_cast<uint64_t*>(base + NA_CMASK);
+    w.neg_mask = reinterpret_cast<uint64_t*>(base + NA_NMASK);
     w.tri_count = reinterpret_cast<uint32_t*>(base + NA_TCNT);
     w.tri_off = reinterpret_cast<uint64_t*>(base + NA_TOFF);
     w.scan_tmp = base + NA_SCAN;

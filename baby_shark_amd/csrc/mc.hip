@@ -786,8 +786,7 @@ void marching_cubes_device(bs_ctx* ctx, bs_volume* vol, float voxel_size, float*
     }
     const uint64_t total = last_off + last_cnt;
     if (total) {
-        float* out = nullptr;
-        BS_HIP(hipMalloc(&out, sizeof(float) * 9 * total));
+        float* out = static_cast<float*>(alloc_block(sizeof(float) * 9 * total));
         if (stale)
             k_mc_units<2, true><<<grid, 64, 0, st>>>(a, nullptr, lane_cnt, off, out);
         else
@@ -795,7 +794,7 @@ void marching_cubes_device(bs_ctx* ctx, bs_volume* vol, float voxel_size, float*
         hipError_t le = hipGetLastError();
         if (le == hipSuccess) le = hipStreamSynchronize(st);
         if (le != hipSuccess) {
-            (void)hipFree(out);
+            free_block(out);
             BS_HIP(le);
         }
         *out_dev = out;

@@ -125,7 +125,7 @@ void alloc_leaves(bs_volume* v, uint64_t n) {
     };
     hipError_t e = attempt();
     if (e == hipErrorOutOfMemory) {  // give the pooled sets back and try once more
-        release_cached_leaves();
+        release_cached_memory();
         e = attempt();
     }
     BS_HIP(e);

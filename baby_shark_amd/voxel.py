@@ -307,8 +307,9 @@ class VolumeBuilder:
 
 def release_cached_memory() -> None:
     """Frees the leaf arrays that dropped volumes left in the library's
-    per-device pool (at most 4 sets and 8 GiB per device), for callers that
-    need that device memory for other work."""
+    per-device pool (at most 4 sets and 8 GiB per device) and the pooled
+    soups and working buffers (at most 16 blocks and 8 GiB per device), for
+    callers that need that device memory for other work."""
     load().bs_release_cached_memory()
 
 

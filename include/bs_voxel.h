@@ -203,9 +203,10 @@ bs_status bs_batch_mesh_to_volume(bs_ctx* ctx, size_t n_meshes, const float* con
 bs_status bs_volume_clone(const bs_volume* v, bs_volume** out);
 void bs_volume_free(bs_volume* v);
 
-/* Frees every pooled leaf array set on every device.  No counterpart in the
- * reference (Rust drop returns memory at once): for callers that need the
- * device memory back for other work. */
+/* Frees every pooled leaf array set and every pooled block (triangle soups
+ * given to bs_device_free, working buffers; at most 16 and 8 GiB per device) on
+ * every device.  No counterpart in the reference (Rust drop returns memory at
+ * once): for callers that need the device memory back for other work. */
 void bs_release_cached_memory(void);
 
 /* Volume::voxel_size and sizes. */
@@ -318,6 +319,8 @@ bs_status bs_ctx_last_dc_stats(const bs_ctx* ctx, bs_dc_stats* out);
 #define BS_DC_VERTEX_QEF_F64 1
 bs_status bs_ctx_set_dc_vertex(bs_ctx* ctx, int mode);
 void bs_free(void* p);
+/* Waits for the block's device, as hipFree does, and keeps the block for later
+ * calls of the library (see bs_release_cached_memory). */
 void bs_device_free(void* p_dev);
 
 /* MarchingCubesMesher::default().with_voxel_size(voxel_size).mesh(volume)

@@ -114,3 +114,47 @@ def test_densify_node_level_tiles(gpu_ctx, oracle_lib):
     s = bs.VolumeBuilder(gpu_ctx, 0.05).sphere(0.4, (0.0, 0.0, 0.0))
     before = s.export()
     assert_same_volume(s.densify_tiles().export(), before)
+
+
+@pytest.mark.parametrize("seed,p_neg,p_hole,lo", [(1, 0.5, 0.0, -11), (2, 0.05, 0.0, -3), (3, 0.93, 0.0, 5),
+                                                  (4, 0.02, 0.0, -20), (5, 0.004, 0.0005, -9), (6, 0.5, 0.3, -1)])
+def test_random_fields_match_oracle(gpu_ctx, oracle_lib, seed, p_neg, p_hole, lo):
+    """A 21^3 block of random values across leaf borders: leaves with far more
+    crossing edges than the kernel keeps in LDS, cells with up to twelve, one
+    each in a hundred leaves, zeros of both signs, and holes (with which the
+    reference may reach unreachable!(): then both sides say so)."""
+    rng = np.random.default_rng(seed)
+    n = 21
+    idx = np.stack(np.meshgrid(*[np.arange(lo, lo + n)] * 3, indexing="ij"), -1).reshape(-1, 3).astype(np.int32)
+    val = rng.uniform(0.05, 1.0, n ** 3).astype(np.float32)
+    val[rng.random(n ** 3) < 0.01] = 0.0
+    val = np.where(rng.random(n ** 3) < p_neg, -val, val)
+    keep = rng.random(n ** 3) >= p_hole
+    ref = oracle_lib.from_voxels(idx[keep], val[keep], 0.05)
+    try:
+        want = ref.dual_contour(0.05)
+    except Exception:
+        with pytest.raises(bs.BSError) as e:
+            bs.DualContouringMesher(gpu_ctx).with_voxel_size(0.05).mesh(_import(gpu_ctx, ref))
+        assert e.value.status == _lib.BS_ERR_INTERNAL
+        return
+    got = bs.DualContouringMesher(gpu_ctx).with_voxel_size(0.05).mesh(_import(gpu_ctx, ref))
+    assert want.shape[0] > 100
+    _same(got, want)
+
+
+def test_soup_blocks_are_reused_whole(gpu_ctx, oracle_lib):
+    """A soup in a block that a larger, freed soup left behind is the soup."""
+    import torch
+    m = bs.DualContouringMesher(gpu_ctx).with_voxel_size(0.02)
+    bs.release_cached_memory()
+    big = m.mesh_device(bs.VolumeBuilder(gpu_ctx, 0.02).sphere(0.6, (0.0, 0.0, 0.0)))
+    torch.as_tensor(big, device="cuda").fill_(12345.0)
+    ptr = big.ptr
+    big.free()
+    small = m.mesh_device(bs.VolumeBuilder(gpu_ctx, 0.02).sphere(0.5, (0.0, 0.0, 0.0)))
+    assert small.ptr == ptr
+    _same(torch.as_tensor(small, device="cuda").cpu().numpy(),
+          oracle_lib.sphere(0.5, (0.0, 0.0, 0.0), 0.02).dual_contour(0.02))
+    small.free()
+    bs.release_cached_memory()
