@@ -64,30 +64,6 @@ struct Block {
 
 __device__ inline int ridx(int x, int y) { return (x + 1) * HB + (y + 1); }
 
-// One workgroup is one wavefront and takes leaves dc_leaf(blockIdx.x),
-// dc_leaf(blockIdx.x + gridDim.x), ... below dc_span(n).  Workgroups go to
-// the 8 XCDs in turn; each XCD takes runs of DC_RUN consecutive leaves, so a
-// leaf's z- and y-neighbours, whose layers it stages, are read through the
-// same L2.
-constexpr uint64_t DC_RUN = 64;
-__host__ __device__ inline uint64_t dc_span(uint64_t n) { return (n + 8 * DC_RUN - 1) / (8 * DC_RUN) * (8 * DC_RUN); }
-__device__ inline uint64_t dc_leaf(uint64_t v) {
-    const uint64_t k = v >> 3;
-    return ((k / DC_RUN) * 8 + (v & 7)) * DC_RUN + k % DC_RUN;
-}
-
-// Exclusive prefix sum over the wave; total in every lane.
-__device__ inline uint32_t wave_prefix(uint32_t v, int lane, uint32_t& total) {
-    uint32_t incl = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t u = (uint32_t)__shfl_up((int)incl, d, 64);
-        if (lane >= d) incl += u;
-    }
-    total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-    return incl - v;
-}
-
 // Row r of the staged block: its eight own voxels in two 16-byte loads, one
 // voxel of the leaf below and two of the leaf above, and the rows' mask bytes
 // (byte y of word x holds row (x, y)).  A missing leaf's loads go to leaf 0 and
@@ -276,9 +252,9 @@ __global__ __launch_bounds__(64) void k_dc_cells(uint64_t n_leaves, DcArgs a) {
     __shared__ Block B;
     const int lane = threadIdx.x;
     const int x = lane >> 3, y = lane & 7;
-    const uint64_t span = dc_span(n_leaves);
+    const uint64_t span = xcd_span(n_leaves);
     for (uint64_t v = blockIdx.x; v < span; v += gridDim.x) {
-        const uint64_t leaf = dc_leaf(v);
+        const uint64_t leaf = xcd_item(v);
         if (leaf >= n_leaves) continue;
         const int4 org = a.origins[leaf];
         stage_block(B, a, org, lane);
@@ -472,9 +448,9 @@ __global__ __launch_bounds__(64) void k_dc_triangles(uint64_t n_leaves, DcArgs a
     const int lane = threadIdx.x;
     const int x = lane >> 3, y = lane & 7;
     const unsigned long long lt = (1ull << lane) - 1;
-    const uint64_t span = dc_span(n_leaves);
+    const uint64_t span = xcd_span(n_leaves);
     for (uint64_t v = blockIdx.x; v < span; v += gridDim.x) {
-        const uint64_t leaf = dc_leaf(v);
+        const uint64_t leaf = xcd_item(v);
         if (leaf >= n_leaves) continue;
         const int4 org = a.origins[leaf];
         int32_t s = (int32_t)leaf;
@@ -613,9 +589,6 @@ struct DcWork {
     size_t scan_bytes;
 };
 
-// A multiple of 8 workgroups (dc_leaf), enough to fill 256 CUs several times.
-unsigned dc_grid(uint64_t n) { return (unsigned)std::min<uint64_t>(dc_span(n), 8192); }
-
 uint64_t hash_capacity(uint64_t n) {
     uint64_t cap = 1024;
     while (cap < 2 * n) cap <<= 1;
@@ -647,7 +620,7 @@ uint64_t dc_count(hipStream_t st, const bs_volume* vol, float voxel_size, bool q
     a.neg_mask = w.neg_mask;
     a.voxel_size = voxel_size;
     a.fail = w.fail;
-    const unsigned grid = dc_grid(n);
+    const unsigned grid = xcd_grid(n);
     if (qef)
         k_dc_cells<true><<<grid, 64, 0, st>>>(n, a);
     else
@@ -670,7 +643,7 @@ uint64_t dc_count(hipStream_t st, const bs_volume* vol, float voxel_size, bool q
 }
 
 void dc_write(hipStream_t st, uint64_t n, const DcArgs& a, const DcWork& w, float* out) {
-    const unsigned grid = dc_grid(n);
+    const unsigned grid = xcd_grid(n);
     k_dc_triangles<true><<<grid, 64, 0, st>>>(n, a, nullptr, w.tri_off, out);
     BS_HIP(hipGetLastError());
 }

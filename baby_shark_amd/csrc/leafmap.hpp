@@ -77,6 +77,34 @@ struct LeafMap {
     }
 };
 
+// Kernels whose workgroup is one wavefront that takes items
+// xcd_item(blockIdx.x), xcd_item(blockIdx.x + gridDim.x), ... of [0, n) (v up to
+// xcd_span(n), items past n skipped).  Workgroups go to the 8 XCDs in turn;
+// each XCD takes runs of XCD_RUN consecutive leaves, so a leaf's neighbours,
+// whose layers it stages, are read through the same L2.
+constexpr uint64_t XCD_RUN = 64;
+__host__ __device__ inline uint64_t xcd_span(uint64_t n) {
+    return (n + 8 * XCD_RUN - 1) / (8 * XCD_RUN) * (8 * XCD_RUN);
+}
+__device__ inline uint64_t xcd_item(uint64_t v) {
+    const uint64_t k = v >> 3;
+    return ((k / XCD_RUN) * 8 + (v & 7)) * XCD_RUN + k % XCD_RUN;
+}
+// a multiple of 8 workgroups, enough to fill 256 CUs several times
+inline unsigned xcd_grid(uint64_t n) { return (unsigned)std::min<uint64_t>(xcd_span(n), 8192); }
+
+// Exclusive prefix sum over the wave; total in every lane.
+__device__ inline uint32_t wave_prefix(uint32_t v, int lane, uint32_t& total) {
+    uint32_t incl = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t u = (uint32_t)__shfl_up((int)incl, d, 64);
+        if (lane >= d) incl += u;
+    }
+    total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    return incl - v;
+}
+
 // Registers leaves [0, n) of an origin array (x, y, z, 0 per leaf) in a
 // map; *fail is set when a key is taken twice or does not fit.
 static __global__ void k_leafmap_insert(uint64_t n, const int4* __restrict__ origins, LeafMap map, uint32_t* fail) {
@@ -106,11 +134,18 @@ static __global__ __launch_bounds__(256) void k_leaf_box(uint64_t n, const int4*
             lo[k] = min(lo[k], __shfl_xor(lo[k], off, 64));
             hi[k] = max(hi[k], __shfl_xor(hi[k], off, 64));
         }
+    // one atomic per block and side: per wave, 4096 of them on each of six
+    // words took 0.28 ms whatever the volume's size
+    __shared__ int32_t part[4][6];
     if ((threadIdx.x & 63) == 0)
         for (int k = 0; k < 3; ++k) {
-            atomicMin(&box[k], lo[k]);
-            atomicMax(&box[3 + k], hi[k]);
+            part[threadIdx.x >> 6][k] = lo[k];
+            part[threadIdx.x >> 6][3 + k] = hi[k];
         }
+    __syncthreads();
+    const int k = threadIdx.x;
+    if (k < 3) atomicMin(&box[k], min(min(part[0][k], part[1][k]), min(part[2][k], part[3][k])));
+    else if (k < 6) atomicMax(&box[k], max(max(part[0][k], part[1][k]), max(part[2][k], part[3][k])));
 }
 
 // The leaf-coordinate box of a volume's n > 0 leaves, computed on the device
@@ -120,7 +155,7 @@ inline void leaf_box(bs_ctx* ctx, const int32_t* origins, uint64_t n, int32_t lo
     int32_t* d = ctx->scratch.as<int32_t>(S_LEAF_BOX, 6);
     k_leaf_box_init<<<1, 64, 0, st>>>(d);
     BS_HIP(hipGetLastError());
-    k_leaf_box<<<(unsigned)std::min<uint64_t>(div_up(n, 256), 1024), 256, 0, st>>>(
+    k_leaf_box<<<(unsigned)std::min<uint64_t>(div_up(n, 256), 256), 256, 0, st>>>(
         n, reinterpret_cast<const int4*>(origins), d);
     BS_HIP(hipGetLastError());
     int32_t h[6];
