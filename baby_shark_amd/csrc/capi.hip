@@ -64,6 +64,18 @@ struct DeviceGuard {
     }
 };
 
+void* pinned_words(bs_ctx* ctx, uint64_t n) {
+    if (ctx->pinned_cap < n) {
+        if (ctx->pinned) BS_HIP(hipHostFree(ctx->pinned));
+        ctx->pinned = nullptr;
+        ctx->pinned_cap = 0;
+        const uint64_t cap = n + n / 4 + 256;
+        BS_HIP(hipHostMalloc(&ctx->pinned, sizeof(uint32_t) * cap, hipHostMallocDefault));
+        ctx->pinned_cap = cap;
+    }
+    return ctx->pinned;
+}
+
 static void free_volume_arrays(bs_volume* v) { free_leaves(v); }
 
 }  // namespace bs
@@ -106,6 +118,9 @@ static void release_side(bs_ctx* c) {
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);
     if (c->ev_leaves) (void)hipEventDestroy(c->ev_leaves);
     if (c->host_pinned) (void)hipHostFree(c->host_pinned);
+    if (c->pinned) (void)hipHostFree(c->pinned);
+    c->pinned = nullptr;
+    c->pinned_cap = 0;
     c->ev_fork = c->ev_join = c->ev_leaves = nullptr;
     c->host_pinned = nullptr;
 }

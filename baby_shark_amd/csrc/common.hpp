@@ -63,7 +63,9 @@ enum ScratchSlot : int {
     S_MC_T128K, S_MC_TORG, S_MC_CUBES, S_LEAF_BOX, S_SG_PRED, S_MLP_PART, S_MLP_GRAD, S_MLP_PERM, S_MC_FLAGS, S_MC_CV, S_MC_V12,
     S_PLOC_BOX, S_PLOC_INFO, S_PLOC_C0, S_PLOC_C1, S_PLOC_NN, S_PLOC_KEEP, S_PLOC_POS, S_PLOC_RING,
     S_TD_PRIMS, S_TD_FR, S_TD_BINS, S_TD_TASKS, S_TD_TCNT, S_TD_SPLIT, S_TD_SMALL, S_TD_HIST,
-    S_LEAF_MKEY, S_LEAF_MKEY_S, S_LEAF_IDS, S_LEAF_PERM, S_COUNT
+    S_LEAF_MKEY, S_LEAF_MKEY_S, S_LEAF_IDS, S_LEAF_PERM,
+    S_OFF_MASKS, S_OFF_KEEP, S_OFF_DST, S_OFF_ORIGINS, S_OFF_FROZEN, S_OFF_WORK, S_OFF_SRC, S_OFF_ORDER,
+    S_OFF_PLANES, S_COUNT
 };
 
 struct Scratch {
@@ -113,6 +115,8 @@ struct bs_ctx {
     hipStream_t stream2 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_leaves = nullptr;
     uint32_t* host_pinned = nullptr;  // 512 words
+    void* pinned = nullptr;           // readbacks of any size (pinned_words)
+    uint64_t pinned_cap = 0;          // words
     // tile classifier of BS_SIGN_SURROGATE (not owned), and its cull threshold
     // in voxels; without a network the gate uses each tile's true smallest |d|
     const struct bs_mlp* surrogate = nullptr;
@@ -131,6 +135,10 @@ struct bs_volume {
 };
 
 namespace bs {
+
+// Pinned host memory of a context, n 32-bit words, valid until the next call
+// (a copy into pageable memory costs about 20 us of staging on its own).
+void* pinned_words(bs_ctx* ctx, uint64_t n);
 
 // Leaf arrays of a volume (origins, masks, values) for n leaves on the current
 // device, drawn from and returned to a per-device pool of released sets.  A

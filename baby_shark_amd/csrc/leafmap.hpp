@@ -114,14 +114,17 @@ static __global__ void k_leafmap_insert(uint64_t n, const int4* __restrict__ ori
     if (!map.put(o.x >> 3, o.y >> 3, o.z >> 3, (int32_t)i)) atomicOr(fail, 1u);
 }
 
-// Leaf-coordinate box (origin >> 3) of leaves [0, n): box[0..2] the minimum,
-// box[3..5] the maximum; box must hold k_leaf_box_init's start values.
+// Leaf-coordinate box (origin >> 3) of leaves [0, n), of those with keep[i] != 0
+// when keep is given: box[0..2] the minimum, box[3..5] the maximum; box must hold
+// k_leaf_box_init's start values.
 static __global__ void k_leaf_box_init(int32_t* box) {
     if (threadIdx.x < 6) box[threadIdx.x] = threadIdx.x < 3 ? INT32_MAX : INT32_MIN;
 }
-static __global__ __launch_bounds__(256) void k_leaf_box(uint64_t n, const int4* __restrict__ origins, int32_t* box) {
+static __global__ __launch_bounds__(256) void k_leaf_box(uint64_t n, const int4* __restrict__ origins, int32_t* box,
+                                                         const uint32_t* __restrict__ keep = nullptr) {
     int32_t lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+        if (keep && !keep[i]) continue;
         const int4 o = origins[i];
         const int32_t c[3] = {o.x >> 3, o.y >> 3, o.z >> 3};
         for (int k = 0; k < 3; ++k) {

@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstring>
 
 #include "common.hpp"
 #include "leafmap.hpp"
@@ -38,21 +39,44 @@ namespace {
 constexpr float FS_FAR = 3.40282347e+38f;
 
 struct OffsetState {
-    uint32_t pool_count;  // leaves in the pool before the sweeps
     uint32_t fail;        // bit 0: a leaf outside the reachable box (bit 2: past the last plane,
                           // bit 3: a pool leaf off the planes, else off the map), bit 1: pool or hash full
+    uint32_t nan;         // some active value is NaN
+    uint32_t live;        // leaves of the result
 };
+
+// Per pool leaf: bit 0, the leaf must be swept; bits 1..6, the face towards -x,
+// +x, -y, +y, -z, +z holds a voxel that can be pushed (fast_sweep.rs:186-273);
+// bit 7, it has an active voxel.
+// A sweep that changes no voxel of a leaf has found each one at the value its
+// neighbours give, in whatever order, so the next sweeps leave the leaf as it
+// is until one of the six layers next to it changes: bit 0 is set where a voxel
+// of the leaf or of such a layer changed since the leaf was last swept, and a
+// leaf without it only pushes.
+constexpr uint32_t WORK_SWEEP = 1u, WORK_LIVE = 128u;
+
+// The sweeps work on a pool of leaves.  A voxel of it is one word: the bits of
+// its magnitude shifted left, bit 0 set when its sign is not the sweeps' (a
+// voxel they set has theirs), or NONE when it is inactive.  NONE is +inf's
+// word, which no active voxel has: a band value beyond 2h was removed and a
+// swept one is at most the limit.  Magnitudes order like their bits.  They are
+// held times `scale`, a power of two that puts h at 1 or above (exact), so that
+// the march's square roots stay in the range of sqrt_normal.
+constexpr uint32_t INF_BITS = 0x7F800000u, FAR_BITS = 0x7F7FFFFFu, NONE = INF_BITS << 1;
 
 struct SweepArgs {
     LeafMap map;
     int4* origins;
-    uint64_t* masks;
-    uint64_t* frozen;
-    float* values;
+    uint64_t* frozen;  // active after remove_if: 8 words per leaf
+    uint32_t* words;   // 512 per leaf
+    uint32_t* work;    // see WORK_SWEEP
     uint32_t capacity;
     int sx, sy, sz;
-    float h, limit_abs;
-    int neg;  // sweep sign
+    int neg;  // the sweeps' sign
+    float h, limit;       // in the words' units
+    float unscale;        // the caller's units per unit of the words
+    uint32_t past_limit;  // bits of the first float above the limit
+    int normal;           // this h and limit, and no NaN: the fast marches serve
 };
 
 // ---------------------------------------------------------------- remove_if
@@ -82,29 +106,40 @@ __global__ __launch_bounds__(256) void k_remove_if(uint64_t n, const uint64_t* _
     if (lane == 0) keep[leaf] = any != 0;
 }
 
-// Copies the kept leaves into the pool (frozen = mask after remove_if) and
-// registers them in the leaf map.
+// Brings the kept leaves into the pool (frozen = mask after remove_if) and
+// registers them in the leaf map; src[slot] = the input leaf.
 __global__ __launch_bounds__(256) void k_pool_init(uint64_t n, const uint32_t* __restrict__ keep,
                                                     const uint32_t* __restrict__ dst, const int32_t* __restrict__ origins,
                                                     const uint64_t* __restrict__ rm_masks,
-                                                    const float* __restrict__ values, SweepArgs a, uint32_t* fail) {
+                                                    const float* __restrict__ values, float scale, SweepArgs a,
+                                                    uint32_t* __restrict__ src, OffsetState* st) {
     const uint64_t leaf = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (leaf >= n || !keep[leaf]) return;
     const int lane = threadIdx.x & 63;
     const uint32_t s = dst[leaf];
-    const float4* src = reinterpret_cast<const float4*>(values + leaf * 512 + (uint64_t)lane * 8);
-    float4* out = reinterpret_cast<float4*>(a.values + (uint64_t)s * 512 + (uint64_t)lane * 8);
-    out[0] = src[0];
-    out[1] = src[1];
-    if (lane < 8) {
-        const uint64_t m = rm_masks[leaf * 8 + lane];
-        a.masks[(uint64_t)s * 8 + lane] = m;
-        a.frozen[(uint64_t)s * 8 + lane] = m;
+    const float4* p = reinterpret_cast<const float4*>(values + leaf * 512 + (uint64_t)lane * 8);
+    const float4 q0 = p[0], q1 = p[1];
+    const float v[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+    const uint32_t act = reinterpret_cast<const uint8_t*>(rm_masks)[leaf * 64 + lane];
+    uint32_t w[8];
+    bool nan = false;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const bool on = (act >> k) & 1u;
+        w[k] = on ? __float_as_uint(fabsf(v[k]) * scale) << 1 | ((__float_as_uint(v[k]) >> 31) ^ (uint32_t)a.neg) : NONE;
+        nan |= on && v[k] != v[k];
     }
+    uint4* out = reinterpret_cast<uint4*>(a.words + (uint64_t)s * 512 + (uint64_t)lane * 8);
+    out[0] = make_uint4(w[0], w[1], w[2], w[3]);
+    out[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    if (lane < 8) a.frozen[(uint64_t)s * 8 + lane] = rm_masks[leaf * 8 + lane];
+    if (nan) atomicOr(&st->nan, 1u);
     if (lane == 0) {
         const int4 o = make_int4(origins[leaf * 4], origins[leaf * 4 + 1], origins[leaf * 4 + 2], 0);
         a.origins[s] = o;
-        if (!a.map.put(o.x >> 3, o.y >> 3, o.z >> 3, (int32_t)s)) atomicOr(fail, 1u);
+        a.work[s] = WORK_SWEEP | WORK_LIVE;
+        src[s] = (uint32_t)leaf;
+        if (!a.map.put(o.x >> 3, o.y >> 3, o.z >> 3, (int32_t)s)) atomicOr(&st->fail, 1u);
     }
 }
 
@@ -113,269 +148,330 @@ __device__ inline int32_t leaf_plane(const int4 o, int sx, int sy, int sz) {
     return sx * (o.x >> 3) + sy * (o.y >> 3) + sz * (o.z >> 3);
 }
 
-__global__ void k_plane_hist(uint32_t n, const int4* __restrict__ origins, int sx, int sy, int sz, int32_t kmin,
-                             uint32_t n_planes, uint32_t* __restrict__ hist, uint32_t* fail) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int32_t k = leaf_plane(origins[i], sx, sy, sz) - kmin;
-    if (k < 0 || (uint32_t)k >= n_planes) {
-        atomicOr(fail, 1u | 8u);
-        return;
+// Leaves per plane.  A block counts its run of leaves in LDS (the planes of a
+// run fit PLANE_LDS bins in every box up to 1300 leaves a side; past that the
+// bins are in memory) and adds each plane's count once: with an atomic per leaf
+// on a few hundred words, 567 k leaves took 0.26 ms, and 0.30 ms to scatter.
+constexpr uint32_t PLANE_LDS = 4096;
+constexpr int PLANE_BLOCK = 256;
+constexpr uint32_t PLANE_RUN = 4096;  // leaves per block
+__global__ __launch_bounds__(PLANE_BLOCK) void k_plane_hist(uint32_t n, const int4* __restrict__ origins, int sx, int sy,
+                                                            int sz, int32_t kmin, uint32_t n_planes,
+                                                            uint32_t* __restrict__ hist, uint32_t* fail) {
+    __shared__ uint32_t bin[PLANE_LDS];
+    const bool lds = n_planes <= PLANE_LDS;
+    const uint32_t i0 = blockIdx.x * PLANE_RUN, i1 = min(n, i0 + PLANE_RUN);
+    for (uint32_t k = threadIdx.x; lds && k < n_planes; k += PLANE_BLOCK) bin[k] = 0;
+    __syncthreads();
+    for (uint32_t i = i0 + threadIdx.x; i < i1; i += PLANE_BLOCK) {
+        const int32_t k = leaf_plane(origins[i], sx, sy, sz) - kmin;
+        if (k < 0 || (uint32_t)k >= n_planes)
+            atomicOr(fail, 1u | 8u);
+        else
+            atomicAdd(lds ? &bin[k] : &hist[k], 1u);
     }
-    atomicAdd(&hist[k], 1u);
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; lds && k < n_planes; k += PLANE_BLOCK)
+        if (bin[k]) atomicAdd(&hist[k], bin[k]);
 }
 
-// order[] = the pool's leaves bucketed by plane; org_order[] their origins in
-// the same order (so a sweep reads a leaf's slot and origin side by side).
-__global__ void k_plane_scatter(uint32_t n, const int4* __restrict__ origins, int sx, int sy, int sz, int32_t kmin,
-                                uint32_t n_planes, uint32_t* __restrict__ cursor, uint32_t* __restrict__ order,
-                                int4* __restrict__ org_order) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int4 o = origins[i];
-    const int32_t k = leaf_plane(o, sx, sy, sz) - kmin;
-    if (k < 0 || (uint32_t)k >= n_planes) return;
-    const uint32_t q = atomicAdd(&cursor[k], 1u);
-    order[q] = i;
-    org_order[q] = o;
+// order[] = the pool's leaves bucketed by plane, each with its origin and, in
+// w, its pool slot.  Counted per block first, so a block takes each plane's
+// range at once.
+__global__ __launch_bounds__(PLANE_BLOCK) void k_plane_scatter(uint32_t n, const int4* __restrict__ origins, int sx,
+                                                               int sy, int sz, int32_t kmin, uint32_t n_planes,
+                                                               uint32_t* __restrict__ cursor, int4* __restrict__ order) {
+    __shared__ uint32_t bin[PLANE_LDS];
+    const bool lds = n_planes <= PLANE_LDS;
+    const uint32_t i0 = blockIdx.x * PLANE_RUN, i1 = min(n, i0 + PLANE_RUN);
+    if (lds) {
+        for (uint32_t k = threadIdx.x; k < n_planes; k += PLANE_BLOCK) bin[k] = 0;
+        __syncthreads();
+        for (uint32_t i = i0 + threadIdx.x; i < i1; i += PLANE_BLOCK) {
+            const int32_t k = leaf_plane(origins[i], sx, sy, sz) - kmin;
+            if (k >= 0 && (uint32_t)k < n_planes) atomicAdd(&bin[k], 1u);
+        }
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < n_planes; k += PLANE_BLOCK)
+            if (bin[k]) bin[k] = atomicAdd(&cursor[k], bin[k]);
+        __syncthreads();
+    }
+    for (uint32_t i = i0 + threadIdx.x; i < i1; i += PLANE_BLOCK) {
+        int4 o = origins[i];
+        const int32_t k = leaf_plane(o, sx, sy, sz) - kmin;
+        if (k < 0 || (uint32_t)k >= n_planes) continue;
+        o.w = (int32_t)i;
+        order[atomicAdd(lds ? &bin[k] : &cursor[k], 1u)] = o;
+    }
 }
 
 // ---------------------------------------------------------------- sweep
-// The leaf and the six neighbour layers touching it in one padded 10^3 block
-// (leaf-local -1..8 per axis; edge and corner cells are never read), so a
-// stencil read is one unconditional LDS load.  st bit 0: active, bit 1: frozen.
-constexpr int PB = 10;
-__device__ inline int pidx(int x, int y, int z) { return ((x + 1) * PB + (y + 1)) * PB + (z + 1); }
+// The leaf and the six neighbour layers touching it in one padded block,
+// leaf-local -1..8 per axis (edge and corner cells are never written or used),
+// a z-row every 16 words with z = 0 on a 16-byte border.
+constexpr int PB = 10, PY = 16, PX = PB * PY;
+__device__ inline int pidx(int x, int y, int z) { return (x + 1) * PX + (y + 1) * PY + 4 + z; }
 
-struct LeafLds {
-    float val[PB * PB * PB];
-    uint8_t st[PB * PB * PB];
-};
-
-// option_min_by(at(+), at(-), cmp_abs) (utils.rs:64-73, fast_sweep.rs:137-140):
-// the + value unless the - value has the strictly smaller magnitude.
-__device__ inline float pick(bool hp, float p, bool hm, float m) {
-    return (hp && hm) ? (fabsf(p) > fabsf(m) ? m : p) : (hp ? p : m);
+// f32 square root, correctly rounded for 0 and from 2^-96 up (NaN below 0):
+// the hardware's is within one ulp, and the signs of two residuals say
+// whether the float below or above it is the rounded one.
+__device__ inline float sqrt_normal(float x) {
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float below = __uint_as_float(__float_as_uint(s) - 1u), above = __uint_as_float(__float_as_uint(s) + 1u);
+    float r = __builtin_fmaf(-below, s, x) <= 0.0f ? below : s;
+    r = __builtin_fmaf(-above, s, x) > 0.0f ? above : r;
+    return r;
 }
 
-// fast_sweep.rs:509-537 with sort3 (helpers/utils.rs:4-16), f32 throughout;
-// the three candidate solutions are all computed and one is selected, which
-// yields the same value as the reference's early returns.
-__device__ inline float compute_distance(float a1, float a2, float a3, float h) {
-    float t;
-    if (a1 > a3) t = a1, a1 = a3, a3 = t;
-    if (a1 > a2) t = a1, a1 = a2, a2 = t;
-    if (a2 > a3) t = a2, a2 = a3, a3 = t;
+// fast_sweep.rs:509-537 for sorted a1 <= a2 <= a3 (sort3, helpers/utils.rs:4-16),
+// f32 throughout; the three candidate solutions are all computed and one is
+// selected, which yields the same value as the reference's early returns.
+// NORMAL: h is at least 1.  A radicand is then 0, negative or at least 2^-72: each
+// of up to three subtractions from 2h^2 or 3h^2 leaves at least an ulp of what
+// it subtracted from, so sqrt_normal serves.
+template <bool NORMAL>
+__device__ inline float solve_sorted(float a1, float a2, float a3, float h, float two_h_sq, float three_h_sq) {
+    auto root = [](float x) { return NORMAL ? sqrt_normal(x) : sqrt_rn(x); };
     const float s1 = a1 + h;
     const float a1a2_sum = a1 + a2;
-    const float h_sq = h * h;
-    const float two_h_sq = h_sq + h_sq;
     const float a1a2_diff = a1 - a2;
     const float a1a2_diff_sq = a1a2_diff * a1a2_diff;
-    const float s2 = (a1a2_sum + sqrt_rn(two_h_sq - a1a2_diff_sq)) * 0.5f;
+    const float s2 = (a1a2_sum + root(two_h_sq - a1a2_diff_sq)) * 0.5f;
     const float a1a2a3_sum = a1a2_sum + a3;
-    const float three_h_sq = two_h_sq + h_sq;
     const float a1a3_diff = a1 - a3;
     const float a1a3_diff_sq = a1a3_diff * a1a3_diff;
     const float a2a3_diff = a2 - a3;
     const float a2a3_diff_sq = a2a3_diff * a2a3_diff;
-    const float s3 = (a1a2a3_sum + sqrt_rn(three_h_sq - a1a2_diff_sq - a1a3_diff_sq - a2a3_diff_sq)) * (1.0f / 3.0f);
-    return fabsf(s1) <= a2 ? s1 : (fabsf(s2) <= a3 ? s2 : s3);
+    const float s3 = (a1a2a3_sum + root(three_h_sq - a1a2_diff_sq - a1a3_diff_sq - a2a3_diff_sq)) * (1.0f / 3.0f);
+    float r = fabsf(s2) <= a3 ? s2 : s3;
+    asm volatile("" : "+v"(r));  // no branch around s2 and s3: nearly every plane of voxels needs them
+    return fabsf(s1) <= a2 ? s1 : r;
 }
 
-// fast_sweep.rs:120-184 for the voxel at padded index o
-__device__ inline void sweep_voxel(LeafLds& L, const SweepArgs& a, int o) {
-    const uint8_t so = L.st[o];
-    const uint8_t sxp = L.st[o + PB * PB], sxm = L.st[o - PB * PB], syp = L.st[o + PB], sym = L.st[o - PB],
-                  szp = L.st[o + 1], szm = L.st[o - 1];
-    const float vxp = L.val[o + PB * PB], vxm = L.val[o - PB * PB], vyp = L.val[o + PB], vym = L.val[o - PB],
-                vzp = L.val[o + 1], vzm = L.val[o - 1], vo = L.val[o];
-    const bool hx = (sxp | sxm) & 1, hy = (syp | sym) & 1, hz = (szp | szm) & 1;
-    const float dx = pick(sxp & 1, vxp, sxm & 1, vxm);
-    const float dy = pick(syp & 1, vyp, sym & 1, vym);
-    const float dz = pick(szp & 1, vzp, szm & 1, vzm);
-    const float first = hx ? dx : (hy ? dy : dz);
-    const bool go = !(so & 2) && (hx || hy || hz) && (int)(__float_as_uint(first) >> 31) == a.neg;
-    if (!go) return;  // a wave with no such voxel skips the solve
-    const float d_abs = compute_distance(fabsf(hx ? dx : FS_FAR), fabsf(hy ? dy : FS_FAR), fabsf(hz ? dz : FS_FAR), a.h);
-    const float d_old = (so & 1) ? vo : FS_FAR;
-    if (!(d_abs > a.limit_abs) && d_abs < fabsf(d_old)) {
-        L.val[o] = a.neg ? -fabsf(d_abs) : fabsf(d_abs);  // copysign(d_abs, sweep sign)
-        L.st[o] = so | 1;
-    }
-}
+// How a leaf is marched.  On one axis the reference takes option_min_by(at(+),
+// at(-), cmp_abs) (utils.rs:64-73, fast_sweep.rs:137-140): the + value unless the
+// - value has the strictly smaller magnitude; the sign of the first axis with a
+// neighbour decides whether the voxel is updated.
+// MARCH_ONE_SIGN  every voxel of the block has the sweeps' sign: an axis takes
+//                 the smaller word, and without any neighbour the solve gives
+//                 more than the limit;
+// MARCH_SIGNED    both signs: that rule on words;
+// MARCH_GENERAL   any h and limit, and NaN: that rule on floats.
+enum MarchKind : int { MARCH_ONE_SIGN = 0, MARCH_SIGNED = 1, MARCH_GENERAL = 2 };
 
-// The leaf's own values and state (this lane's z-row; lane = (lx, ly)) and,
-// in lanes 0..5, its six face-neighbour slots, as registers.  stage_issue
-// only issues the loads (dense map: the raw cell word, resolved when stored),
-// so the leaf's data and its neighbour lookups travel in one round trip.
-struct LeafStage {
-    float4 v0, v1;
-    uint64_t mw, fw;
-    int32_t nb;  // lanes 0..5: neighbour slot or map cell word
-};
-
-__device__ inline void stage_issue(const SweepArgs& a, uint32_t slot, int4 org, int lane, LeafStage& s) {
-    const int lx = lane >> 3;
-    const float4* vp = reinterpret_cast<const float4*>(a.values + (uint64_t)slot * 512 + lane * 8);
-    s.v0 = vp[0];
-    s.v1 = vp[1];
-    s.mw = a.masks[(uint64_t)slot * 8 + lx];
-    s.fw = a.frozen[(uint64_t)slot * 8 + lx];
-    s.nb = -1;
-    if (lane < 6) {
-        const int ax = lane >> 1, dir = (lane & 1) ? 1 : -1;
-        const int32_t nx = (org.x >> 3) + (ax == 0 ? dir : 0), ny = (org.y >> 3) + (ax == 1 ? dir : 0),
-                      nz = (org.z >> 3) + (ax == 2 ? dir : 0);
-        if (a.map.dense) {
-            const uint32_t ix = (uint32_t)(nx - a.map.x0), iy = (uint32_t)(ny - a.map.y0), iz = (uint32_t)(nz - a.map.z0);
-            if (ix < a.map.nx && iy < a.map.ny && iz < a.map.nz)
-                s.nb = a.map.cells[((uint64_t)ix * a.map.ny + iy) * a.map.nz + iz];
-        } else {
-            s.nb = a.map.find(nx, ny, nz);
-        }
-    }
-}
-
-__device__ inline void stage_store(LeafLds& L, const LeafStage& s, int lane) {
-    const int lx = lane >> 3, ly = lane & 7;
-    const uint64_t mw = s.mw >> (ly * 8), fw = s.fw >> (ly * 8);
-    const float v[8] = {s.v0.x, s.v0.y, s.v0.z, s.v0.w, s.v1.x, s.v1.y, s.v1.z, s.v1.w};
-    const int base = pidx(lx, ly, 0);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        L.val[base + k] = v[k];
-        L.st[base + k] = (uint8_t)(((mw >> k) & 1) | (((fw >> k) & 1) << 1));
-    }
-}
-
-// The six neighbour layers next to the leaf, into the padding.  nb: lanes
-// 0..5 hold the neighbour slots (-1 none; a cell being created, -2, is no
-// leaf yet).  The slots are read from those lanes and every one of the twelve
-// loads is issued unconditionally (slot 0 in place of a missing neighbour,
-// its result discarded), so they travel in one round trip.
-__device__ inline void stage_layers(LeafLds& L, const SweepArgs& a, int lane, int32_t nb) {
-    const int i = lane >> 3, j = lane & 7;
-    uint8_t on[6];
-    float val[6];
-    uint64_t mw[6];
-    float nv[6];
-    int32_t n[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        n[k] = __builtin_amdgcn_readlane(nb, k);
-        const int f = (k & 1) ? 0 : 7;  // -side neighbour: its far layer 7; +side: layer 0
-        const int o = k < 2 ? ((f << 6) | (i << 3) | j) : (k < 4 ? ((i << 6) | (f << 3) | j) : ((i << 6) | (j << 3) | f));
-        const uint64_t ns = n[k] >= 0 ? (uint64_t)n[k] : 0;
-        mw[k] = a.masks[ns * 8 + (o >> 6)];
-        nv[k] = a.values[ns * 512 + o];
-    }
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const int f = (k & 1) ? 0 : 7;
-        const int o = k < 2 ? ((f << 6) | (i << 3) | j) : (k < 4 ? ((i << 6) | (f << 3) | j) : ((i << 6) | (j << 3) | f));
-        on[k] = n[k] >= 0 ? (uint8_t)((mw[k] >> (o & 63)) & 1ull) : (uint8_t)0;
-        val[k] = on[k] ? nv[k] : 0.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const int g = (k & 1) ? 8 : -1;  // the padding layer this maps to
-        const int po = k < 2 ? pidx(g, i, j) : (k < 4 ? pidx(i, g, j) : pidx(i, j, g));
-        L.st[po] = on[k];
-        L.val[po] = val[k];
-    }
-}
-
-// The staged leaf swept (the wavefront over its 22 voxel planes), written
-// back, and its pushes (fast_sweep.rs:186-273): the +direction face of each
-// axis; lanes 0..2 create the pushed neighbours of the three axes at once.
-// A created slot is published without a fence: in this plane a lookup of the
-// new leaf reads only its masks and values, which hold the empty leaf
-// already, and its origin is read only in a later plane.
-__device__ inline void sweep_and_finish(LeafLds& L, const SweepArgs& a, uint32_t slot, int4 org, uint32_t plane,
-                                        uint32_t n_planes, uint32_t start, uint32_t* created, OffsetState* st,
-                                        int lane) {
-    const int lx = lane >> 3, ly = lane & 7;
-    // voxel plane p holds the voxels u + v + w = p (u, v, w counted in the
-    // sweep direction); they are independent of each other, so lane (u, v)
-    // = (lx, ly) takes w = p - u - v when that is a voxel
-    const int pu = a.sx > 0 ? lx : 7 - lx, pv = a.sy > 0 ? ly : 7 - ly;
+// The wavefront over the leaf's 22 voxel planes (fast_sweep.rs:120-184 for each
+// voxel): plane p holds the voxels u + v + w = p (u, v, w the voxel's coordinates
+// counted along the sweep), which do not depend on each other; lane (u, v) takes
+// w = p - u - v.  A voxel reads the new values of its three upwind neighbours,
+// written on plane p - 1, and the old ones of the downwind neighbours, all
+// through one address that moves a word per plane.
+//
+// One wave issues an instruction every 4 to 5 cycles and a leaf is one wave, so
+// the march costs its instruction count: about 75 a plane of voxels (95 with two
+// signs), 4.8 us a leaf; 7.5 us with 150, from float compares, activity bytes and
+// the full range's square root.
+template <int KIND>
+__device__ inline void march(const SweepArgs& a, uint32_t* word, int lane, uint32_t frozen) {
+    const int x = lane >> 3, y = lane & 7;
+    const int first_w = -(a.sx > 0 ? x : 7 - x) - (a.sy > 0 ? y : 7 - y);
+    uint32_t* row = word + pidx(x, y, 0);
+    const float h = a.h, h_sq = h * h, two_h_sq = h_sq + h_sq, three_h_sq = two_h_sq + h_sq;
     for (int p = 0; p < 22; ++p) {
-        const int w = p - lx - ly;
-        if (w >= 0 && w < 8) sweep_voxel(L, a, pidx(pu, pv, a.sz > 0 ? w : 7 - w));
-        __syncthreads();
-    }
-    {
-        const int base = pidx(lx, ly, 0);
-        float4* vp = reinterpret_cast<float4*>(a.values + (uint64_t)slot * 512 + lane * 8);
-        vp[0] = make_float4(L.val[base + 0], L.val[base + 1], L.val[base + 2], L.val[base + 3]);
-        vp[1] = make_float4(L.val[base + 4], L.val[base + 5], L.val[base + 6], L.val[base + 7]);
-        uint32_t row = 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) row |= (uint32_t)(L.st[base + k] & 1) << k;
-        const uint64_t w = gather_word(row, ly);
-        if (ly == 0) a.masks[(uint64_t)slot * 8 + lx] = w;
-    }
-    bool push[3];
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-        const int dir = ax == 0 ? a.sx : (ax == 1 ? a.sy : a.sz);
-        const int f = dir > 0 ? 7 : 0;
-        const int i = lx, j = ly;
-        const int o = ax == 0 ? pidx(f, i, j) : (ax == 1 ? pidx(i, f, j) : pidx(i, j, f));
-        const float v = L.val[o];
-        const bool q = (L.st[o] & 1) && (int)(__float_as_uint(v) >> 31) == a.neg && fabsf(v) < a.limit_abs;
-        push[ax] = __ballot(q) != 0;
-    }
-    if (lane < 3 && (lane == 0 ? push[0] : (lane == 1 ? push[1] : push[2]))) {
-        const int ax = lane;
-        const int dir = ax == 0 ? a.sx : (ax == 1 ? a.sy : a.sz);
-        if (plane + 1 >= n_planes) atomicOr(&st->fail, 1u | 4u);
-        const int32_t nx = (org.x >> 3) + (ax == 0 ? dir : 0), ny = (org.y >> 3) + (ax == 1 ? dir : 0),
-                      nz = (org.z >> 3) + (ax == 2 ? dir : 0);
-        int32_t* cell = a.map.claim(nx, ny, nz, &st->fail);
-        if (cell) {
-            const uint32_t s = start + atomicAdd(&created[plane + 1], 1u);
-            if (s < a.capacity) {
-                a.origins[s] = make_int4(nx * 8, ny * 8, nz * 8, 0);
-                atomicExch(cell, (int32_t)s);
+        const int w = first_w + p;
+        if ((uint32_t)w < 8u) {
+            const int z = a.sz > 0 ? w : 7 - w;
+            uint32_t* c = row + z;
+            const uint32_t xp = c[PX], xm = c[-PX], yp = c[PY], ym = c[-PY], zp = c[1], zm = c[-1], own = c[0];
+            const bool fixed = (frozen >> z) & 1u;
+            if constexpr (KIND != MARCH_GENERAL) {
+                uint32_t bx, by, bz;  // the axes' neighbours
+                if constexpr (KIND == MARCH_ONE_SIGN) {
+                    bx = min(xp, xm), by = min(yp, ym), bz = min(zp, zm);
+                } else {
+                    auto pick = [](uint32_t plus, uint32_t minus) { return (minus | 1u) < (plus & ~1u) ? minus : plus; };
+                    bx = pick(xp, xm), by = pick(yp, ym), bz = pick(zp, zm);
+                }
+                const uint32_t mx = min(bx >> 1, FAR_BITS), my = min(by >> 1, FAR_BITS), mz = min(bz >> 1, FAR_BITS);
+                const uint32_t lo = min(min(mx, my), mz), hi = max(max(mx, my), mz),
+                               mid = max(min(mx, my), min(max(mx, my), mz));
+                const float d = solve_sorted<true>(__uint_as_float(lo), __uint_as_float(mid), __uint_as_float(hi), h,
+                                                   two_h_sq, three_h_sq);
+                const uint32_t first = KIND == MARCH_ONE_SIGN ? 0u : (bx < NONE ? bx : (by < NONE ? by : bz));
+                if (d < __uint_as_float(min(own >> 1, a.past_limit)) && !fixed && !(first & 1u))
+                    *c = __float_as_uint(d) << 1;
             } else {
-                atomicOr(&st->fail, 2u);  // pool overflow: retried with a larger pool
+                const uint32_t plus[3] = {xp, yp, zp}, minus[3] = {xm, ym, zm};
+                bool has[3];
+                uint32_t q[3];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const bool hp = plus[k] != NONE, hm = minus[k] != NONE;
+                    has[k] = hp || hm;
+                    q[k] = (hp && hm) ? (__uint_as_float(plus[k] >> 1) > __uint_as_float(minus[k] >> 1) ? minus[k] : plus[k])
+                                      : (hp ? plus[k] : minus[k]);
+                }
+                const uint32_t first = has[0] ? q[0] : (has[1] ? q[1] : q[2]);
+                float a1 = has[0] ? __uint_as_float(q[0] >> 1) : FS_FAR, a2 = has[1] ? __uint_as_float(q[1] >> 1) : FS_FAR,
+                      a3 = has[2] ? __uint_as_float(q[2] >> 1) : FS_FAR, t;
+                if (a1 > a3) t = a1, a1 = a3, a3 = t;
+                if (a1 > a2) t = a1, a1 = a2, a2 = t;
+                if (a2 > a3) t = a2, a2 = a3, a3 = t;
+                const float d = fabsf(solve_sorted<false>(a1, a2, a3, h, two_h_sq, three_h_sq));
+                const float old = own != NONE ? __uint_as_float(own >> 1) : FS_FAR;
+                if (!fixed && (has[0] || has[1] || has[2]) && !(first & 1u) && !(d > a.limit) && d < old)
+                    *c = __float_as_uint(d) << 1;
             }
         }
+        // the wave's LDS operations complete in order: the compiler alone must keep the next plane's reads below
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
-// One leaf plane of one sweep: the leaves of bucket [b0, b1) of `order` plus
-// the leaves created while the previous plane was swept.  starts[p + 1] is
-// the pool size when plane p begins and created[p + 1] the leaves plane p
-// creates (all on plane p + 1), so this plane sweeps the pool range
-// [starts[plane], starts[plane] + created[plane]) after its bucket and
-// allocates its own new leaves from starts[plane] + created[plane] on.
-// One 64-lane block per leaf, looping over the plane's leaves.
-__global__ __launch_bounds__(64) void k_sweep_plane(SweepArgs a, const uint32_t* __restrict__ order,
-                                                     const int4* __restrict__ org_order,
-                                                     const uint32_t* __restrict__ bucket_off, uint32_t plane,
-                                                     uint32_t n_planes, uint32_t* starts, uint32_t* created,
-                                                     OffsetState* st) {
-    __shared__ LeafLds L;
-    const uint32_t b0 = bucket_off[plane], b1 = bucket_off[plane + 1];
-    const uint32_t n_old = b1 - b0;
-    const uint32_t new_lo = starts[plane];
-    const uint32_t start = min(new_lo + created[plane], a.capacity);
+// Claims the missing neighbours that a leaf pushes: lanes 0..2, the sweep's
+// +direction face of each axis.  A created slot is published without a fence:
+// in this plane a lookup of the new leaf reads only its words, which hold the
+// empty leaf already, and its origin and work bits are read only in a later
+// plane.
+__device__ inline void push_neighbours(const SweepArgs& a, int4 org, uint32_t faces, uint32_t plane, uint32_t n_planes,
+                                       uint32_t start, uint2* counts, OffsetState* st, int lane, bool there) {
+    const int s = lane == 0 ? a.sx : (lane == 1 ? a.sy : a.sz);
+    if (lane >= 3 || !((faces >> (2 * lane + (s > 0 ? 2 : 1))) & 1u)) return;
+    if (plane + 1 >= n_planes) atomicOr(&st->fail, 1u | 4u);
+    if (there) return;
+    const int32_t nx = (org.x >> 3) + (lane == 0 ? s : 0), ny = (org.y >> 3) + (lane == 1 ? s : 0),
+                  nz = (org.z >> 3) + (lane == 2 ? s : 0);
+    int32_t* cell = a.map.claim(nx, ny, nz, &st->fail);
+    if (!cell) return;
+    const uint32_t slot = start + atomicAdd(&counts[plane + 1].y, 1u);
+    if (slot < a.capacity) {
+        a.origins[slot] = make_int4(nx * 8, ny * 8, nz * 8, 0);
+        a.work[slot] = WORK_SWEEP;
+        atomicExch(cell, (int32_t)slot);
+    } else {
+        atomicOr(&st->fail, 2u);  // pool overflow: retried with a larger pool
+    }
+}
+
+// a word with its sign bit on top: below INF_BITS exactly when the voxel is
+// active with the sweeps' sign
+__device__ inline uint32_t sign_first(uint32_t w) { return w >> 1 | w << 31; }
+
+// One leaf plane of one sweep: entries [b0, b0 + n_old) of `order` (origin and,
+// in w, pool slot) plus the leaves created while the previous plane was swept.
+// counts[p + 1] holds the pool size when plane p begins (x) and the leaves plane
+// p creates (y, all on plane p + 1), so this plane sweeps the pool range [x, x + y)
+// of counts[plane] after its bucket and allocates its own new leaves from x + y
+// on; the sweep's first plane has no leaves created before it and begins with
+// `pool` leaves.  One wavefront per leaf, looping over the plane's leaves.
+//
+// A sweep is a chain of these launches, so what counts is the time of one leaf
+// from end to end: three dependent rounds of loads (the leaf's entry; its
+// words, work bits and six map cells; the six neighbour layers), the march, the
+// write-back of what changed, and the pushes.  Code that runs once per leaf
+// costs most of its time in instruction fetch (a launch starts with a cold
+// instruction cache: about 15 cycles an instruction), so the pool holds words
+// that go to LDS as they are; from values and masks, coding and decoding
+// them took 2.5 us of a leaf's 11.5.
+__global__ __launch_bounds__(64) void k_sweep_plane(SweepArgs a, const int4* __restrict__ order, uint32_t b0,
+                                                     uint32_t n_old, uint32_t plane, uint32_t first,
+                                                     uint32_t n_planes, uint32_t pool, uint2* counts, OffsetState* st) {
+    __shared__ __align__(16) uint32_t word[PB * PX];
+    const int lane = threadIdx.x, x = lane >> 3, y = lane & 7;
+    int4 entry = order[b0 + min(blockIdx.x, max(n_old, 1u) - 1)];  // before the counts arrive
+    const uint2 before = counts[plane];
+    const uint32_t new_lo = plane == first ? pool : before.x;
+    const uint32_t start = plane == first ? pool : min(new_lo + before.y, a.capacity);
     const uint32_t n_new = start - new_lo;
-    const int lane = threadIdx.x;
-    if (blockIdx.x == 0 && lane == 0) starts[plane + 1] = start;
+    if (blockIdx.x == 0 && lane == 0) counts[plane + 1].x = start;
     for (uint32_t item = blockIdx.x; item < n_old + n_new; item += gridDim.x) {
-        // a bucket leaf's slot and origin in one round trip, a pushed one's origin
-        const uint32_t slot = item < n_old ? order[b0 + item] : new_lo + (item - n_old);
-        const int4 org = item < n_old ? org_order[b0 + item] : a.origins[slot];
-        LeafStage s;
-        stage_issue(a, slot, org, lane, s);
-        stage_store(L, s, lane);
-        stage_layers(L, a, lane, s.nb >= 0 ? s.nb : -1);  // the padding: no overlap with stage_store
+        if (item >= n_old) {
+            entry = a.origins[new_lo + (item - n_old)];
+            entry.w = (int32_t)(new_lo + (item - n_old));
+        } else if (item != blockIdx.x) {
+            entry = order[b0 + item];
+        }
+        const uint32_t slot = (uint32_t)entry.w;
+        const uint32_t work = a.work[slot];
+        uint4* mine = reinterpret_cast<uint4*>(a.words + (uint64_t)slot * 512 + lane * 8);
+        const uint4 w0 = mine[0], w1 = mine[1];
+        // byte y of a frozen word x holds row (x, y)
+        const uint32_t frozen = reinterpret_cast<const uint8_t*>(a.frozen)[(uint64_t)slot * 64 + lane];
+        // lanes 0..5: the neighbour slots (-1: none, or a leaf being created, which has no active voxel)
+        int32_t nb = -1;
+        if (lane < 6) {
+            const int ax = lane >> 1, dir = (lane & 1) ? 1 : -1;
+            nb = a.map.find((entry.x >> 3) + (ax == 0 ? dir : 0), (entry.y >> 3) + (ax == 1 ? dir : 0),
+                            (entry.z >> 3) + (ax == 2 ? dir : 0));
+        }
+        int32_t n[6];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) n[k] = __builtin_amdgcn_readlane(nb, k);
+        const bool there = (lane == 0 ? (a.sx > 0 ? n[1] : n[0])
+                                      : (lane == 1 ? (a.sy > 0 ? n[3] : n[2]) : (a.sz > 0 ? n[5] : n[4]))) >= 0;
+        if (!(work & WORK_SWEEP)) {
+            push_neighbours(a, entry, work, plane, n_planes, start, counts, st, lane, there);
+            continue;
+        }
+        // the six layers next to the leaf, a voxel per lane and face (slot 0 in place of a missing neighbour)
+        uint32_t f[6];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const int far = (k & 1) ? 0 : 7;  // -side neighbour: its layer 7; +side: layer 0
+            const int off = k < 2 ? (far << 6 | lane) : (k < 4 ? (x << 6 | far << 3 | y) : (lane << 3 | far));
+            f[k] = a.words[(n[k] >= 0 ? (uint64_t)n[k] : 0) * 512 + off];
+        }
+        uint4* own = reinterpret_cast<uint4*>(word + pidx(x, y, 0));
+        own[0] = w0;
+        own[1] = w1;
+        const uint32_t old[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+        uint32_t least = NONE, either = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) least = min(least, sign_first(old[k])), either |= old[k];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            f[k] = n[k] >= 0 ? f[k] : NONE;
+            least = min(least, sign_first(f[k])), either |= f[k];
+            const int g = (k & 1) ? 8 : -1;
+            word[k < 2 ? pidx(g, x, y) : (k < 4 ? pidx(x, g, y) : pidx(x, y, g))] = f[k];
+        }
         __syncthreads();
-        sweep_and_finish(L, a, slot, org, plane, n_planes, start, created, st, lane);
+        if (!a.normal)
+            march<MARCH_GENERAL>(a, word, lane, frozen);
+        else if (__ballot(least < INF_BITS)) {
+            if (__ballot(either & 1u))
+                march<MARCH_SIGNED>(a, word, lane, frozen);
+            else
+                march<MARCH_ONE_SIGN>(a, word, lane, frozen);
+        }  // else no voxel has the sweeps' sign: none is set, and none can be pushed
+        __syncthreads();
+        // what changed, what can be pushed
+        const uint4 r0 = own[0], r1 = own[1];
+        const uint32_t now[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+        uint32_t diff = 0;
+        least = NONE;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) diff |= now[k] ^ old[k], least = min(least, sign_first(now[k]));
+        const uint32_t limit_bits = __float_as_uint(a.limit);
+        const uint64_t FX0 = 0xFFull, FX7 = FX0 << 56, FY0 = 0x0101010101010101ull, FY7 = FY0 << 7;  // rows of the faces
+        const uint64_t can = __ballot(least < limit_bits);
+        uint32_t faces = (uint32_t)((can & FX0) != 0) << 1 | (uint32_t)((can & FX7) != 0) << 2 |
+                         (uint32_t)((can & FY0) != 0) << 3 | (uint32_t)((can & FY7) != 0) << 4 |
+                         (uint32_t)(__ballot(sign_first(now[0]) < limit_bits) != 0) << 5 |
+                         (uint32_t)(__ballot(sign_first(now[7]) < limit_bits) != 0) << 6 | (work & WORK_LIVE);
+        const uint64_t set = __ballot(diff != 0);
+        if (set) {
+            faces |= WORK_SWEEP | WORK_LIVE;
+            mine[0] = r0;
+            mine[1] = r1;
+            const uint32_t moved = (uint32_t)((set & FX0) != 0) | (uint32_t)((set & FX7) != 0) << 1 |
+                                   (uint32_t)((set & FY0) != 0) << 2 | (uint32_t)((set & FY7) != 0) << 3 |
+                                   (uint32_t)(__ballot(now[0] != old[0]) != 0) << 4 |
+                                   (uint32_t)(__ballot(now[7] != old[7]) != 0) << 5;
+            if (lane < 6 && nb >= 0 && (moved >> lane & 1u)) atomicOr(&a.work[nb], WORK_SWEEP);
+        }
+        if (lane == 0) a.work[slot] = faces;
+        push_neighbours(a, entry, faces, plane, n_planes, start, counts, st, lane, there);
         __syncthreads();
     }
 }
@@ -384,43 +480,58 @@ __global__ __launch_bounds__(64) void k_sweep_plane(SweepArgs a, const uint32_t*
 // Sort keys of the final pool: empty leaves (fast_sweep.rs:61-64
 // remove_empty_branches) sort last.
 __global__ __launch_bounds__(256) void k_final_keys(uint32_t n, const int4* __restrict__ origins,
-                                                     const uint64_t* __restrict__ masks, uint64_t* __restrict__ keys,
-                                                     uint32_t* __restrict__ idx, uint32_t* __restrict__ n_live) {
+                                                     const uint32_t* __restrict__ work, uint64_t* __restrict__ keys,
+                                                     uint32_t* __restrict__ idx, OffsetState* st) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t any = 0;
-#pragma unroll
-    for (int w = 0; w < 8; ++w) any |= masks[(uint64_t)i * 8 + w];
-    const int4 o = origins[i];
-    keys[i] = any ? leaf_key(o.x >> 3, o.y >> 3, o.z >> 3) : ~0ull;
-    idx[i] = i;
-    if (any) atomicAdd(n_live, 1u);
+    const bool live = i < n && (work[i] & WORK_LIVE);
+    if (i < n) {
+        const int4 o = origins[i];
+        keys[i] = live ? leaf_key(o.x >> 3, o.y >> 3, o.z >> 3) : ~0ull;
+        idx[i] = i;
+    }
+    const uint64_t b = __ballot(live);
+    if ((threadIdx.x & 63) == 0 && b) atomicAdd(&st->live, (uint32_t)__popcll(b));
 }
 
 // Gathers the live leaves in key order and applies v -= D to active values
-// (visitors/value_mut_visitor.rs:4-32 visits active values only).
-__global__ __launch_bounds__(256) void k_final_gather(uint64_t n_out, const uint32_t* __restrict__ src_idx,
-                                                       const int4* __restrict__ porigins,
-                                                       const uint64_t* __restrict__ pmasks,
-                                                       const float* __restrict__ pvalues, float distance,
+// (visitors/value_mut_visitor.rs:4-32 visits active values only): a frozen
+// voxel has its input value, a swept one its word's, an inactive one what the
+// input held (0 in a created leaf).
+__global__ __launch_bounds__(256) void k_final_gather(uint64_t n_out, const uint32_t* __restrict__ src_idx, SweepArgs a,
+                                                       uint32_t n_keep, const uint32_t* __restrict__ src,
+                                                       const float* __restrict__ in_values, float distance,
                                                        int4* __restrict__ origins, uint64_t* __restrict__ masks,
                                                        float* __restrict__ values) {
     const uint64_t leaf = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (leaf >= n_out) return;
     const int lane = threadIdx.x & 63;
     const uint32_t s = src_idx[leaf];
-    const uint64_t word = pmasks[(uint64_t)s * 8 + (lane >> 3)] >> ((lane & 7) * 8);
-    const float4* vp = reinterpret_cast<const float4*>(pvalues + (uint64_t)s * 512 + lane * 8);
-    const float4 q0 = vp[0], q1 = vp[1];
+    const uint4* wp = reinterpret_cast<const uint4*>(a.words + (uint64_t)s * 512 + lane * 8);
+    const uint4 w0 = wp[0], w1 = wp[1];
+    const uint32_t frozen = reinterpret_cast<const uint8_t*>(a.frozen)[(uint64_t)s * 64 + lane];
+    float4 q0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), q1 = q0;
+    if (s < n_keep) {
+        const float4* vp = reinterpret_cast<const float4*>(in_values + (uint64_t)src[s] * 512 + lane * 8);
+        q0 = vp[0];
+        q1 = vp[1];
+    }
+    const uint32_t w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
     float v[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+    uint32_t row = 0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-        if ((word >> k) & 1) v[k] = v[k] - distance;
+    for (int k = 0; k < 8; ++k) {
+        if (w[k] == NONE) continue;
+        row |= 1u << k;
+        if (!((frozen >> k) & 1u))
+            v[k] = __uint_as_float(__float_as_uint(__uint_as_float(w[k] >> 1) * a.unscale) | (uint32_t)a.neg << 31);
+        v[k] = v[k] - distance;
+    }
     float4* op = reinterpret_cast<float4*>(values + leaf * 512 + (uint64_t)lane * 8);
     op[0] = make_float4(v[0], v[1], v[2], v[3]);
     op[1] = make_float4(v[4], v[5], v[6], v[7]);
-    if (lane < 8) masks[leaf * 8 + lane] = pmasks[(uint64_t)s * 8 + lane];
-    if (lane == 0) origins[leaf] = porigins[s];
+    const uint64_t m = gather_word(row, lane & 7);
+    if ((lane & 7) == 0) masks[leaf * 8 + (lane >> 3)] = m;
+    if (lane == 0) origins[leaf] = a.origins[s];
 }
 
 constexpr int kDirs[8][3] = {{1, 1, 1},  {-1, 1, 1},  {1, -1, 1},  {-1, -1, 1},
@@ -441,25 +552,19 @@ void exclusive_scan_u32(bs_ctx* ctx, const uint32_t* in, uint32_t* out, uint64_t
     BS_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, in, out, (int)n, ctx->stream));
 }
 
-template <class T>
-T read_back(bs_ctx* ctx, const T* d) {
-    T h{};
-    BS_HIP(hipMemcpyAsync(&h, d, sizeof(T), hipMemcpyDeviceToHost, ctx->stream));
-    BS_HIP(hipStreamSynchronize(ctx->stream));
-    return h;
-}
-
-// Device buffers of one offset attempt (released on every exit path).
+// The large device buffers of one offset attempt, back to the pool on every
+// exit path once the stream is done with them.
 struct OffsetBuffers {
+    hipStream_t st;
     std::vector<void*> ptrs;
+    explicit OffsetBuffers(hipStream_t s) : st(s) { ptrs.reserve(4); }
     template <class T> T* alloc(uint64_t count) {
-        void* p = nullptr;
-        BS_HIP(hipMalloc(&p, std::max<uint64_t>(count, 1) * sizeof(T)));
-        ptrs.push_back(p);
-        return static_cast<T*>(p);
+        ptrs.push_back(alloc_block(std::max<uint64_t>(count, 1) * sizeof(T)));
+        return static_cast<T*>(ptrs.back());
     }
     ~OffsetBuffers() {
-        for (void* p : ptrs) (void)hipFree(p);
+        const bool done = hipStreamSynchronize(st) == hipSuccess;
+        for (void* p : ptrs) free_block(p, !done);
     }
 };
 
@@ -489,38 +594,34 @@ OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_
     const float limit_abs = fabsf(ext);
     const int neg = std::signbit(ext) ? 1 : 0;
 
-    OffsetBuffers B;
+    if (stats) stats->n_kept = 0;
+    if (n == 0) return res;
+    Scratch& S = ctx->scratch;
+    OffsetBuffers B(st);
     // remove_if and compaction of the surviving leaves
-    uint64_t* rm_masks = B.alloc<uint64_t>(8 * n);
-    uint32_t* keep = B.alloc<uint32_t>(n);
-    uint32_t* dst = B.alloc<uint32_t>(n);
-    if (n) {
-        k_remove_if<<<div_up(n, 4), 256, 0, st>>>(n, vol->masks, vol->values, two_h, rm_masks, keep);
-        BS_HIP(hipGetLastError());
-        exclusive_scan_u32(ctx, keep, dst, n);
-    }
-    res.keep.assign(n, 0);
-    std::vector<int32_t> o4(4 * n);
-    if (n) {
-        BS_HIP(hipMemcpyAsync(res.keep.data(), keep, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, st));
-        BS_HIP(hipMemcpyAsync(o4.data(), vol->origins, sizeof(int32_t) * 4 * n, hipMemcpyDeviceToHost, st));
-        BS_HIP(hipStreamSynchronize(st));
-    }
-    uint64_t n_keep = 0;
-    int32_t lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
-    for (uint64_t i = 0; i < n; ++i) {
-        if (!res.keep[i]) continue;
-        ++n_keep;
-        for (int k = 0; k < 3; ++k) {
-            lo[k] = std::min(lo[k], o4[4 * i + k] >> 3);
-            hi[k] = std::max(hi[k], o4[4 * i + k] >> 3);
-        }
-    }
+    uint64_t* rm_masks = S.as<uint64_t>(S_OFF_MASKS, 8 * n);
+    uint32_t* keep = S.as<uint32_t>(S_OFF_KEEP, n);
+    uint32_t* dst = S.as<uint32_t>(S_OFF_DST, n);
+    int32_t* dbox = S.as<int32_t>(S_LEAF_BOX, 6);
+    k_remove_if<<<div_up(n, 4), 256, 0, st>>>(n, vol->masks, vol->values, two_h, rm_masks, keep);
+    BS_HIP(hipGetLastError());
+    exclusive_scan_u32(ctx, keep, dst, n);
+    k_leaf_box_init<<<1, 64, 0, st>>>(dbox);
+    BS_HIP(hipGetLastError());
+    k_leaf_box<<<(unsigned)std::min<uint64_t>(div_up(n, 256), 256), 256, 0, st>>>(
+        n, reinterpret_cast<const int4*>(vol->origins), dbox, keep);
+    BS_HIP(hipGetLastError());
+    res.keep.resize(n);
+    int32_t box[6];
+    uint32_t last_dst = 0;
+    BS_HIP(hipMemcpyAsync(res.keep.data(), keep, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, st));
+    BS_HIP(hipMemcpyAsync(&last_dst, dst + n - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    BS_HIP(hipMemcpyAsync(box, dbox, sizeof(box), hipMemcpyDeviceToHost, st));
+    BS_HIP(hipStreamSynchronize(st));
+    const uint64_t n_keep = last_dst + res.keep[n - 1];
     if (stats) stats->n_kept = n_keep;
-    if (n_keep == 0) {
-        out.n_leaves = 0;
-        return res;
-    }
+    if (n_keep == 0) return res;
+    int32_t lo[3] = {box[0], box[1], box[2]}, hi[3] = {box[3], box[4], box[5]};
     BS_REQUIRE(capacity >= n_keep && capacity < (1ull << 31), BS_ERR_INVALID_ARG, "offset leaf pool too large");
 
     // Reach of the extension: a value grows by at least h/sqrt(3) per voxel
@@ -555,141 +656,126 @@ OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_
     SweepArgs a{};
     a.map = map;
     a.capacity = (uint32_t)capacity;
-    a.origins = B.alloc<int4>(capacity);
-    a.masks = B.alloc<uint64_t>(8 * capacity);
-    a.frozen = B.alloc<uint64_t>(8 * capacity);
-    a.values = B.alloc<float>(512 * capacity);
-    a.h = h;
-    a.limit_abs = limit_abs;
+    a.origins = S.as<int4>(S_OFF_ORIGINS, capacity);
+    a.frozen = S.as<uint64_t>(S_OFF_FROZEN, 8 * capacity);
+    a.work = S.as<uint32_t>(S_OFF_WORK, capacity);
+    a.words = B.alloc<uint32_t>(512 * capacity);
     a.neg = neg;
-    // leaves created by the sweep start empty, with 0.0 values (Leaf::empty)
-    BS_HIP(hipMemsetAsync(a.masks, 0, sizeof(uint64_t) * 8 * capacity, st));
-    BS_HIP(hipMemsetAsync(a.frozen, 0, sizeof(uint64_t) * 8 * capacity, st));
-    BS_HIP(hipMemsetAsync(a.values + 512 * n_keep, 0, sizeof(float) * 512 * (capacity - n_keep), st));
-    OffsetState* dstate = B.alloc<OffsetState>(1);
-    OffsetState init{(uint32_t)n_keep, 0};
-    BS_HIP(hipMemcpyAsync(dstate, &init, sizeof(init), hipMemcpyHostToDevice, st));
-    k_pool_init<<<div_up(n, 4), 256, 0, st>>>(n, keep, dst, vol->origins, rm_masks, vol->values, a, &dstate->fail);
+    // the words' units (see NONE): scaling up by a power of two is exact, and nothing overflows with h within
+    // 2^+-60 and the limit within 2^59 of it
+    int h_exp = 0;
+    std::frexp(h, &h_exp);
+    const bool in_range = h_exp >= -60 && h_exp <= 60 && limit_abs / h <= 5.0e17f;
+    const int up = in_range && h_exp < 1 ? 1 - h_exp : 0;
+    const float scale = std::ldexp(1.0f, up);
+    a.unscale = std::ldexp(1.0f, -up);
+    a.h = h * scale;
+    a.limit = limit_abs * scale;
+    const float past_limit = std::nextafter(a.limit, INFINITY);
+    std::memcpy(&a.past_limit, &past_limit, sizeof(float));
+    // leaves created by the sweep start empty (Leaf::empty)
+    BS_HIP(hipMemsetD32Async(a.words + 512 * n_keep, (int)NONE, 512 * (capacity - n_keep), st));
+    BS_HIP(hipMemsetAsync(a.frozen + 8 * n_keep, 0, sizeof(uint64_t) * 8 * (capacity - n_keep), st));
+    // the planes of the map box, as many in every direction; their leaf counts and bucket starts, the state (read
+    // back with the starts in one copy) and the pool counts
+    const uint32_t n_planes = (uint32_t)(hi[0] - lo[0] + hi[1] - lo[1] + hi[2] - lo[2] + 1);
+    constexpr uint32_t STATE_WORDS = sizeof(OffsetState) / sizeof(uint32_t);
+    uint32_t* hist = S.as<uint32_t>(S_OFF_PLANES, 4 * (uint64_t)(n_planes + 2) + STATE_WORDS + 2);
+    uint32_t* off = hist + n_planes + 1;
+    OffsetState* dstate = reinterpret_cast<OffsetState*>(off + n_planes + 1);
+    uint2* counts = reinterpret_cast<uint2*>(hist + (2 * (n_planes + 1) + STATE_WORDS + 1) / 2 * 2);
+    uint32_t* back = static_cast<uint32_t*>(pinned_words(ctx, n_planes + 1 + STATE_WORDS));
+    const uint32_t* hoff = back;
+    OffsetState cur{};
+    auto read_state = [&] { std::memcpy(&cur, back + n_planes + 1, sizeof(cur)); };
+    BS_HIP(hipMemsetAsync(dstate, 0, sizeof(OffsetState), st));
+    uint32_t* src = S.as<uint32_t>(S_OFF_SRC, n_keep);
+    k_pool_init<<<div_up(n, 4), 256, 0, st>>>(n, keep, dst, vol->origins, rm_masks, vol->values, scale, a, src, dstate);
     BS_HIP(hipGetLastError());
 
-    // plane range over the whole map box
-    uint32_t* order = B.alloc<uint32_t>(capacity);
-    int4* org_order = B.alloc<int4>(capacity);
-
-    uint64_t planes_total = 0, launches = 0, swept = 0;
+    // one entry more than leaves: a plane past the last bucket reads one that it does not use
+    int4* order = S.as<int4>(S_OFF_ORDER, capacity + 1);
+    uint64_t planes_total = 0, swept = 0;
     uint32_t pool = (uint32_t)n_keep;  // pool size at the start of the sweep
-    for (int s = 0; s < 8; ++s) {
-        a.sx = kDirs[s][0], a.sy = kDirs[s][1], a.sz = kDirs[s][2];
-        const OffsetState cur = read_back(ctx, dstate);
+    auto check = [&](int s) {
         BS_REQUIRE(!(cur.fail & 1u), BS_ERR_INTERNAL,
                    "offset: a pushed leaf left the reachable box (flags " + std::to_string(cur.fail) + ", sweep " +
                        std::to_string(s) + ", pool " + std::to_string(pool) + ")");
-        if (cur.fail) {
-            res.retry = true;
-            return res;
-        }
-        const uint32_t n_pool = pool;
-        if (s > 0) swept += n_pool;  // every leaf in the pool at the end of a sweep was swept in it
-        // planes of the map box in this direction
-        // planes of the reachable box (the leaves plus the extension margin)
-        int32_t kmin = 0, kmax = 0;
-        const int sgn[3] = {a.sx, a.sy, a.sz};
-        for (int k = 0; k < 3; ++k) {
-            kmin += sgn[k] > 0 ? lo[k] : -hi[k];
-            kmax += sgn[k] > 0 ? hi[k] : -lo[k];
-        }
-        const uint32_t n_planes = (uint32_t)(kmax - kmin + 1);
-        uint32_t* hist = B.alloc<uint32_t>(n_planes + 1);
-        uint32_t* off = B.alloc<uint32_t>(n_planes + 1);
+        return cur.fail == 0;
+    };
+    for (int s = 0; s < 8; ++s) {
+        a.sx = kDirs[s][0], a.sy = kDirs[s][1], a.sz = kDirs[s][2];
+        const int32_t kmin = (a.sx > 0 ? lo[0] : -hi[0]) + (a.sy > 0 ? lo[1] : -hi[1]) + (a.sz > 0 ? lo[2] : -hi[2]);
         BS_HIP(hipMemsetAsync(hist, 0, sizeof(uint32_t) * (n_planes + 1), st));
-        k_plane_hist<<<div_up(n_pool, 256), 256, 0, st>>>(n_pool, a.origins, a.sx, a.sy, a.sz, kmin, n_planes, hist,
-                                                         &dstate->fail);
+        BS_HIP(hipMemsetAsync(counts, 0, sizeof(uint2) * (n_planes + 1), st));
+        k_plane_hist<<<div_up(pool, PLANE_RUN), PLANE_BLOCK, 0, st>>>(pool, a.origins, a.sx, a.sy, a.sz, kmin, n_planes,
+                                                                      hist, &dstate->fail);
         BS_HIP(hipGetLastError());
         exclusive_scan_u32(ctx, hist, off, n_planes + 1);
-        BS_HIP(hipMemcpyAsync(hist, off, sizeof(uint32_t) * (n_planes + 1), hipMemcpyDeviceToDevice, st));
-        k_plane_scatter<<<div_up(n_pool, 256), 256, 0, st>>>(n_pool, a.origins, a.sx, a.sy, a.sz, kmin, n_planes, hist,
-                                                            order, org_order);
+        BS_HIP(hipMemcpyAsync(back, off, sizeof(uint32_t) * (n_planes + 1 + STATE_WORDS), hipMemcpyDeviceToHost, st));
+        k_plane_scatter<<<div_up(pool, PLANE_RUN), PLANE_BLOCK, 0, st>>>(pool, a.origins, a.sx, a.sy, a.sz, kmin,
+                                                                         n_planes, off, order);
         BS_HIP(hipGetLastError());
-        // host view of the bucket sizes: the first and last plane holding a leaf
-        std::vector<uint32_t> hoff(n_planes + 1);
-        BS_HIP(hipMemcpyAsync(hoff.data(), off, sizeof(uint32_t) * (n_planes + 1), hipMemcpyDeviceToHost, st));
         BS_HIP(hipStreamSynchronize(st));
-        uint32_t first = 0, last = 0, max_bucket = 0;
-        bool any = false;
-        for (uint32_t p = 0; p < n_planes; ++p) {
-            const uint32_t c = hoff[p + 1] - hoff[p];
-            if (!c) continue;
-            if (!any) first = p;
-            any = true;
-            last = p;
-            max_bucket = std::max(max_bucket, c);
-        }
-        if (!any) break;
-        // starts[p + 1], created[p + 1]: pool size when plane p begins, leaves it creates
-        uint32_t* starts = B.alloc<uint32_t>(n_planes + 2);
-        uint32_t* created = B.alloc<uint32_t>(n_planes + 2);
-        BS_HIP(hipMemsetAsync(created, 0, sizeof(uint32_t) * (n_planes + 2), st));
-        BS_HIP(hipMemcpyAsync(starts + first, &pool, sizeof(uint32_t), hipMemcpyHostToDevice, st));
-        uint32_t p_end = first;
-        for (uint32_t p = first; p < n_planes; ++p) {
-            const uint32_t bucket = hoff[p + 1] - hoff[p];
-            if (p > last) {
-                // past the last bucket: continue only while the previous plane created leaves
-                uint32_t c = 0;
-                BS_HIP(hipMemcpyAsync(&c, created + p, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-                BS_HIP(hipStreamSynchronize(st));
-                if (c == 0) break;
-            }
+        read_state();
+        res.retry = !check(s);
+        if (res.retry) return res;
+        a.normal = in_range && !cur.nan;
+        // the first and the last plane holding a leaf (the pool is never empty)
+        uint32_t first = 0, last = n_planes - 1;
+        while (hoff[first + 1] == 0) ++first;
+        while (hoff[last] == hoff[n_planes]) --last;
+        auto launch = [&](uint32_t p) {
             // enough blocks for the bucket and the leaves the previous plane may have created
-            const uint32_t prev = p > first ? hoff[p] - hoff[p - 1] : 0;
-            const unsigned grid = (unsigned)std::min<uint64_t>(std::max<uint64_t>((uint64_t)bucket + prev + 64, 64), 4096);
-            k_sweep_plane<<<grid, 64, 0, st>>>(a, order, org_order, off, p, n_planes, starts, created, dstate);
+            const uint32_t bucket = hoff[p + 1] - hoff[p], prev = p > first ? hoff[p] - hoff[p - 1] : 0;
+            const unsigned grid = (unsigned)std::min<uint64_t>((uint64_t)bucket + prev + 64, 4096);
+            k_sweep_plane<<<grid, 64, 0, st>>>(a, order, hoff[p], bucket, p, first, n_planes, pool, counts, dstate);
             BS_HIP(hipGetLastError());
             ++planes_total;
-            ++launches;
-            p_end = p;
+        };
+        uint32_t p = first;
+        while (p <= last) launch(p++);
+        // past the last bucket: on while the planes create leaves, a few planes for each look
+        uint32_t* tail = back + n_planes + 1;
+        for (;;) {
+            for (uint32_t e = std::min(n_planes, p + 4); p < e; ++p) launch(p);
+            BS_HIP(hipMemcpyAsync(tail, counts + p, sizeof(uint2), hipMemcpyDeviceToHost, st));
+            BS_HIP(hipStreamSynchronize(st));
+            if (p == n_planes || tail[1] == 0) break;
         }
-        // pool size after the last plane swept
-        uint32_t tail[2] = {0, 0};
-        BS_HIP(hipMemcpyAsync(&tail[0], starts + p_end + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        BS_HIP(hipMemcpyAsync(&tail[1], created + p_end + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        BS_HIP(hipStreamSynchronize(st));
-        pool = std::min<uint32_t>(tail[0] + tail[1], (uint32_t)capacity);
+        // the pool's size after the last plane swept
         if ((uint64_t)tail[0] + tail[1] > capacity) {
             res.retry = true;
             return res;
         }
-    }
-    const OffsetState fin = read_back(ctx, dstate);
-    BS_REQUIRE(!(fin.fail & 1u), BS_ERR_INTERNAL,
-               "offset: a pushed leaf left the reachable box (flags " + std::to_string(fin.fail) + ", after the sweeps)");
-    if (fin.fail) {
-        res.retry = true;
-        return res;
+        pool = tail[0] + tail[1];
+        swept += pool;  // every leaf in the pool at the end of a sweep was swept in it
     }
     const uint32_t n_pool = pool;
-    swept += n_pool;
     if (stats) {
         stats->n_swept = swept;
         stats->n_pool = n_pool;
         stats->n_planes = planes_total;
-        stats->n_launches = launches;
+        stats->n_launches = planes_total;
     }
 
     // empty leaves go, the rest sorted by origin, shifted by -D
-    uint64_t* keys = B.alloc<uint64_t>(n_pool);
-    uint64_t* keys_s = B.alloc<uint64_t>(n_pool);
-    uint32_t* idx = B.alloc<uint32_t>(n_pool);
-    uint32_t* idx_s = B.alloc<uint32_t>(n_pool);
-    uint32_t* n_live = B.alloc<uint32_t>(1);
-    BS_HIP(hipMemsetAsync(n_live, 0, sizeof(uint32_t), st));
-    k_final_keys<<<div_up(n_pool, 256), 256, 0, st>>>(n_pool, a.origins, a.masks, keys, idx, n_live);
+    uint64_t* keys = S.as<uint64_t>(S_KEYS, n_pool);
+    uint64_t* keys_s = S.as<uint64_t>(S_KEYS_SORTED, n_pool);
+    uint32_t* idx = S.as<uint32_t>(S_IDX, n_pool);
+    uint32_t* idx_s = S.as<uint32_t>(S_IDX_SORTED, n_pool);
+    k_final_keys<<<div_up(n_pool, 256), 256, 0, st>>>(n_pool, a.origins, a.work, keys, idx, dstate);
     BS_HIP(hipGetLastError());
+    BS_HIP(hipMemcpyAsync(back + n_planes + 1, dstate, sizeof(cur), hipMemcpyDeviceToHost, st));
     sort_pairs_u64(ctx, keys, keys_s, idx, idx_s, n_pool);
-    const uint32_t n_out = read_back(ctx, n_live);
+    BS_HIP(hipStreamSynchronize(st));
+    read_state();
+    res.retry = !check(8);
+    if (res.retry) return res;
+    const uint32_t n_out = cur.live;
     alloc_leaves(&out, n_out);
     if (n_out) {
-        k_final_gather<<<div_up(n_out, 4), 256, 0, st>>>(n_out, idx_s, a.origins, a.masks, a.values, distance,
+        k_final_gather<<<div_up(n_out, 4), 256, 0, st>>>(n_out, idx_s, a, (uint32_t)n_keep, src, vol->values, distance,
                                                          reinterpret_cast<int4*>(out.origins), out.masks, out.values);
         BS_HIP(hipGetLastError());
     }

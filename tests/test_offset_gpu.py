@@ -123,3 +123,35 @@ def test_offset_grows_into_new_blocks(gpu_ctx, oracle_lib, r, h, c, D, bx):
     gs, rs = g.signs_at(q), ref.signs_at(q)
     assert np.array_equal(gs, rs)
     assert gs.min() != gs.max()      # the grid holds inside and outside voxels
+
+
+@pytest.mark.parametrize("h,kind", [(0.05, "signs"), (3.0, "signs"), (0.05, "one sign"), (2.0 ** -70, "signs"),
+                                    (0.05, "nan"), (2.0 ** 40, "holes")])
+@pytest.mark.parametrize("D", [3.3, -2.0])
+def test_random_bands_match_oracle(gpu_ctx, oracle_lib, h, kind, D):
+    """Bands of random values across leaf borders: neighbours of both signs and
+    of equal magnitude (the + one counts), one sign only, holes, values beyond
+    the band, zeros of both signs, NaN, and voxel sizes that the fast marches
+    take scaled, unscaled and not at all."""
+    rng = np.random.default_rng(7)
+    n = 19
+    g = np.stack(np.meshgrid(*[np.arange(-7, n - 7)] * 3, indexing="ij"), -1).reshape(-1, 3).astype(np.int32)
+    near = np.abs(g - 2).sum(1) % 5 < 2
+    idx = g[near & (rng.random(g.shape[0]) < (0.4 if kind == "holes" else 0.8))]
+    mag = rng.choice([0.0, 0.25, 0.5, 1.0, 1.9, 2.5], idx.shape[0]) + (rng.random(idx.shape[0]) < 0.3) * 0.01
+    sign = np.where(rng.random(idx.shape[0]) < (0.0 if kind == "one sign" else 0.4), -1.0, 1.0) * np.sign(D)
+    val = (mag * sign * h).astype(np.float32)
+    if kind == "nan":
+        val[rng.random(idx.shape[0]) < 0.05] = np.nan
+    ref = oracle_lib.from_voxels(idx, val, h)
+    got = bs.volume_from_voxels(idx, val, h, gpu_ctx).offset(D * h)
+    want = ref.offset(D * h).export()
+    assert want.active().sum() > idx.shape[0]
+    if kind == "nan":
+        e = got.export()
+        assert np.array_equal(e.masks, want.masks)
+        assert np.array_equal(np.isnan(e.values), np.isnan(want.values))
+        ok = ~np.isnan(want.values)
+        assert np.array_equal(e.values[ok].view(np.uint32), want.values[ok].view(np.uint32))
+    else:
+        assert_same_volume(got.export(), want)
