@@ -300,13 +300,16 @@ bs_status bs_volume_clone(const bs_volume* v, bs_volume** out) {
         c->voxel_size = v->voxel_size;
         c->n_leaves = v->n_leaves;
         c->tiles = v->tiles;
-        if (v->topo) c->topo = v->topo->clone();
         try {
+            if (v->topo) c->topo = v->topo->clone();
+            if (v->tree) c->tree = clone_tree(*v->tree);
             if (v->n_leaves) {
                 alloc_leaves(c, v->n_leaves);
-                BS_HIP(hipMemcpy(c->origins, v->origins, sizeof(int32_t) * 4 * v->n_leaves, hipMemcpyDeviceToDevice));
-                BS_HIP(hipMemcpy(c->masks, v->masks, sizeof(uint64_t) * 8 * v->n_leaves, hipMemcpyDeviceToDevice));
-                BS_HIP(hipMemcpy(c->values, v->values, sizeof(float) * 512 * v->n_leaves, hipMemcpyDeviceToDevice));
+                BS_HIP(hipMemcpyAsync(c->origins, v->origins, sizeof(int32_t) * 4 * v->n_leaves, hipMemcpyDeviceToDevice));
+                BS_HIP(hipMemcpyAsync(c->masks, v->masks, sizeof(uint64_t) * 8 * v->n_leaves, hipMemcpyDeviceToDevice));
+                BS_HIP(hipMemcpyAsync(c->values, v->values, sizeof(float) * 512 * v->n_leaves, hipMemcpyDeviceToDevice));
+                // a device-to-device copy need not have ended when the call returns
+                BS_HIP(hipStreamSynchronize(nullptr));
             }
         } catch (...) {
             free_volume_arrays(c);

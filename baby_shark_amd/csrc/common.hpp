@@ -12,6 +12,7 @@
 
 #include "../../include/bs_voxel.h"
 #include "topology.hpp"
+#include "tree.hpp"
 
 namespace bs {
 
@@ -65,7 +66,10 @@ enum ScratchSlot : int {
     S_TD_PRIMS, S_TD_FR, S_TD_BINS, S_TD_TASKS, S_TD_TCNT, S_TD_SPLIT, S_TD_SMALL, S_TD_HIST,
     S_LEAF_MKEY, S_LEAF_MKEY_S, S_LEAF_IDS, S_LEAF_PERM,
     S_OFF_MASKS, S_OFF_KEEP, S_OFF_DST, S_OFF_ORIGINS, S_OFF_FROZEN, S_OFF_WORK, S_OFF_SRC, S_OFF_ORDER,
-    S_OFF_PLANES, S_COUNT
+    S_OFF_PLANES,
+    S_TREE_MARK, S_TREE_TILES, S_TREE_TILE_VAL, S_TREE_FLAGS, S_TREE_PAIRS, S_TREE_FLIPS, S_TREE_PARTNER, S_TREE_ZERO,
+    S_TREE_RANK, S_TREE_ROOTS, S_TREE_NODES, S_TREE_ITEMS, S_TREE_REFS, S_TREE_NODE_N, S_TREE_PLACE, S_MC_TILE_VAL,
+    S_COUNT
 };
 
 struct Scratch {
@@ -131,7 +135,9 @@ struct bs_volume {
     uint64_t* masks = nullptr;   // device, n_leaves*8
     float* values = nullptr;     // device, n_leaves*512
     std::vector<bs::TileRec> tiles;           // active internal tiles (host, few)
-    std::unique_ptr<bs::Topology> topo;       // upper levels; built from the leaves when absent
+    // upper levels, in one form or the other; built from the leaves and tiles when absent
+    std::unique_ptr<bs::Topology> topo;
+    std::unique_ptr<bs::DeviceTree> tree;
 };
 
 namespace bs {

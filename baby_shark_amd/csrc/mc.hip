@@ -745,11 +745,21 @@ void marching_cubes_device(bs_ctx* ctx, bs_volume* vol, float voxel_size, float*
     *n_tris = 0;
     BS_REQUIRE(vol->device == ctx->device, BS_ERR_INVALID_ARG, "volume lives on another device");
     if (stats) *stats = bs_dc_stats{};
-    Topology& topo = ensure_topology(ctx, vol);
-    std::vector<int64_t> units;
+    // the units in visit order, from the device's tree or, where that does not fit, the host's
+    std::vector<int64_t> host_units;
     std::vector<TileRec> tiles;
-    topo.visit_units(units, tiles);
-    const uint64_t n_units = units.size(), n = vol->n_leaves;
+    const int64_t* units = nullptr;
+    uint64_t n_units = 0;
+    if (const DeviceTree* t = ensure_tree(ctx, vol)) {
+        n_units = tree_units(ctx, *t, &units, tiles);
+    } else {
+        ensure_topology(ctx, vol).visit_units(host_units, tiles);
+        n_units = host_units.size();
+        int64_t* d = ctx->scratch.as<int64_t>(S_MC_UNITS, n_units);
+        if (n_units) BS_HIP(hipMemcpyAsync(d, host_units.data(), 8 * n_units, hipMemcpyHostToDevice, st));
+        units = d;
+    }
+    const uint64_t n = vol->n_leaves;
     if (!n_units) return;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (stats) {
@@ -813,18 +823,17 @@ void marching_cubes_device(bs_ctx* ctx, bs_volume* vol, float voxel_size, float*
     }
     std::copy(val8.begin(), val8.end(), tv.begin() + tiles.size());
     std::copy(val128.begin(), val128.end(), tv.begin() + tiles.size() + val8.size());
-    // units, tile records and tile values in one upload
-    const size_t b_units = 8 * n_units, b_torg = 16 * torg.size(), b_tv = 4 * tv.size();
-    std::vector<uint8_t> up(b_units + b_torg + b_tv);
-    std::memcpy(up.data(), units.data(), b_units);
-    std::memcpy(up.data() + b_units, torg.data(), b_torg);
-    std::memcpy(up.data() + b_units + b_torg, tv.data(), b_tv);
-    uint8_t* dup = ctx->scratch.as<uint8_t>(S_MC_UNITS, up.size());
+    // tile records and tile values in one upload
+    const size_t b_torg = 16 * torg.size(), b_tv = 4 * tv.size();
+    std::vector<uint8_t> up(b_torg + b_tv);
+    std::memcpy(up.data(), torg.data(), b_torg);
+    std::memcpy(up.data() + b_torg, tv.data(), b_tv);
+    uint8_t* dup = ctx->scratch.as<uint8_t>(S_MC_TILE_VAL, up.size());
     BS_HIP(hipMemcpyAsync(dup, up.data(), up.size(), hipMemcpyHostToDevice, st));
-    a.units = reinterpret_cast<const int64_t*>(dup);
+    a.units = units;
     a.n_units = n_units;
-    a.tile_org = reinterpret_cast<const int4*>(dup + b_units);
-    a.tile_val = reinterpret_cast<const float*>(dup + b_units + b_torg);
+    a.tile_org = reinterpret_cast<const int4*>(dup);
+    a.tile_val = reinterpret_cast<const float*>(dup + b_torg);
     a.t8_val = a.tile_val + tiles.size();
     a.t128_val = a.t8_val + val8.size();
     a.origins = reinterpret_cast<const int4*>(vol->origins);

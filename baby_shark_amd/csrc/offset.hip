@@ -576,7 +576,7 @@ namespace {
 
 struct OffsetResult {
     uint64_t n_out = 0;
-    std::vector<uint32_t> keep;  // per input leaf
+    const uint32_t* keep_dev = nullptr;  // per input leaf (context scratch)
     bool retry = false;
 };
 
@@ -611,14 +611,15 @@ OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_
     k_leaf_box<<<(unsigned)std::min<uint64_t>(div_up(n, 256), 256), 256, 0, st>>>(
         n, reinterpret_cast<const int4*>(vol->origins), dbox, keep);
     BS_HIP(hipGetLastError());
-    res.keep.resize(n);
-    int32_t box[6];
-    uint32_t last_dst = 0;
-    BS_HIP(hipMemcpyAsync(res.keep.data(), keep, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, st));
-    BS_HIP(hipMemcpyAsync(&last_dst, dst + n - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    BS_HIP(hipMemcpyAsync(box, dbox, sizeof(box), hipMemcpyDeviceToHost, st));
+    res.keep_dev = keep;
+    uint32_t* first = static_cast<uint32_t*>(pinned_words(ctx, 8));
+    BS_HIP(hipMemcpyAsync(first, dst + n - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    BS_HIP(hipMemcpyAsync(first + 1, keep + n - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    BS_HIP(hipMemcpyAsync(first + 2, dbox, 6 * sizeof(int32_t), hipMemcpyDeviceToHost, st));
     BS_HIP(hipStreamSynchronize(st));
-    const uint64_t n_keep = last_dst + res.keep[n - 1];
+    const uint64_t n_keep = (uint64_t)first[0] + first[1];
+    int32_t box[6];
+    std::memcpy(box, first + 2, sizeof(box));
     if (stats) stats->n_kept = n_keep;
     if (n_keep == 0) return res;
     int32_t lo[3] = {box[0], box[1], box[2]}, hi[3] = {box[3], box[4], box[5]};
@@ -793,7 +794,6 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
     EventPair ev;
     ev.start(ctx->stream);
     BS_REQUIRE(vol->device == ctx->device, BS_ERR_INVALID_ARG, "volume lives on another device");
-    Topology& topo = ensure_topology(ctx, vol);
     const float two_h = vol->voxel_size * 2.0f;
     // fast_sweep.rs:100 unwraps the leaf at every queued origin, and the queue
     // holds every active tile that survives remove_if: the reference panics.
@@ -816,14 +816,26 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
         BS_REQUIRE(attempt < 6, BS_ERR_INTERNAL, "offset: leaf pool kept overflowing");
         capacity *= 4;
     }
-    // topology: remove_if (tiles, emptied leaves, empty nodes), the new leaves, empty nodes again
-    std::vector<std::array<int32_t, 3>> out_origins(out.n_leaves);
-    if (out.n_leaves) {
-        std::vector<int32_t> o4(4 * out.n_leaves);
-        BS_HIP(hipMemcpy(o4.data(), out.origins, sizeof(int32_t) * o4.size(), hipMemcpyDeviceToHost));
-        for (uint64_t i = 0; i < out.n_leaves; ++i) out_origins[i] = {o4[4 * i], o4[4 * i + 1], o4[4 * i + 2]};
+    // the tree: remove_if (tiles, emptied leaves, empty nodes), the new leaves, empty nodes again.  A volume
+    // without one has the tree that its leaves give (no tile survives), and so has the result.
+    std::unique_ptr<Topology> t2;
+    std::unique_ptr<DeviceTree> d2;
+    if (vol->topo || vol->tree || !vol->tiles.empty()) {
+        if (const DeviceTree* d = ensure_tree(ctx, vol))
+            d2 = tree_after_offset(ctx, *d, reinterpret_cast<const int4*>(vol->origins), r.keep_dev, vol->n_leaves,
+                                   reinterpret_cast<const int4*>(out.origins), out.n_leaves);
+        if (!d2) {
+            std::vector<uint32_t> keep(vol->n_leaves);
+            std::vector<int32_t> o4(4 * out.n_leaves);
+            if (!keep.empty())
+                BS_HIP(hipMemcpy(keep.data(), r.keep_dev, sizeof(uint32_t) * keep.size(), hipMemcpyDeviceToHost));
+            if (!o4.empty())
+                BS_HIP(hipMemcpy(o4.data(), out.origins, sizeof(int32_t) * o4.size(), hipMemcpyDeviceToHost));
+            std::vector<std::array<int32_t, 3>> out_origins(out.n_leaves);
+            for (uint64_t i = 0; i < out.n_leaves; ++i) out_origins[i] = {o4[4 * i], o4[4 * i + 1], o4[4 * i + 2]};
+            t2 = ensure_topology(ctx, vol).after_offset(keep, out_origins, two_h);
+        }
     }
-    std::unique_ptr<Topology> t2 = topo.after_offset(r.keep, out_origins, two_h);
     free_leaves(vol);
     vol->n_leaves = out.n_leaves;
     vol->origins = out.origins;
@@ -834,6 +846,7 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
     out.values = nullptr;
     vol->tiles.clear();  // remove_if deactivated every tile (checked above)
     vol->topo = std::move(t2);
+    vol->tree = std::move(d2);
     ev.stop(ctx->stream);
     if (stats) {
         stats->n_out = out.n_leaves;

@@ -5,8 +5,9 @@
 // leaf) live in device memory and every pass over them is a streaming kernel
 // (one wavefront per leaf, 8 values per lane).  The upper tree levels are a
 // few hundred slot nodes per volume; their flood fill and CSG slot decisions
-// run on the host (topology.cpp) and produce, for each output leaf, a
-// reference to its source leaves and the combination to apply.
+// run on the device too (tree.hip), on the host (topology.cpp) for trees that do
+// not fit there, and produce, for each output leaf, a reference to its source
+// leaves and the combination to apply.
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -216,6 +217,11 @@ static std::vector<std::array<int32_t, 3>> leaf_origins(bs_ctx* ctx, const bs_vo
 
 Topology& ensure_topology(bs_ctx* ctx, bs_volume* v) {
     if (v->topo) return *v->topo;
+    if (v->tree) {
+        v->topo = download_tree(ctx, v);
+        v->tree.reset();
+        return *v->topo;
+    }
     v->topo = Topology::from_leaves(leaf_origins(ctx, v), v->tiles);
     BS_REQUIRE(v->topo->leaves.size() == v->n_leaves, BS_ERR_INTERNAL, "volume has two leaves at one origin");
     return *v->topo;
@@ -224,6 +230,8 @@ Topology& ensure_topology(bs_ctx* ctx, bs_volume* v) {
 // ensure_topology of two volumes, the second built on another host thread
 static void ensure_topologies(bs_ctx* ctx, bs_volume* a, bs_volume* b) {
     std::vector<std::array<int32_t, 3>> oa, ob;
+    if (a->tree) ensure_topology(ctx, a);
+    if (b->tree) ensure_topology(ctx, b);
     if (!a->topo) oa = leaf_origins(ctx, a);
     if (!b->topo) ob = leaf_origins(ctx, b);
     auto build_b = std::async(std::launch::async, [&] {
@@ -541,16 +549,23 @@ __global__ void k_gather_signs(uint64_t n, const uint64_t* __restrict__ q, const
 
 inline int32_t floor_div8(int64_t v) { return (int32_t)(v >= 0 ? v / 8 : -((-v + 7) / 8)); }
 
-// Runs the leaf flood fill of one volume on the device (values in place) and
-// records each leaf's first/last sign and emptiness in its topology.  The
-// caller synchronises before reading `flags_host`.
+// Runs the leaf flood fill of one volume on the device (values in place); each
+// leaf's first/last sign and emptiness in the returned device array.
+uint8_t* launch_leaf_flood_fill(bs_ctx* ctx, bs_volume* v, int slot) {
+    uint8_t* d_flags = ctx->scratch.as<uint8_t>(slot, v->n_leaves);
+    if (v->n_leaves)
+        k_leaf_flood_fill<<<div_up(v->n_leaves, WAVES_PER_BLOCK), 256, 0, ctx->stream>>>(v->n_leaves, v->masks, v->values,
+                                                                                       d_flags);
+    BS_HIP(hipGetLastError());
+    return d_flags;
+}
+
+// The same with the flags on the host: the caller synchronises before reading
+// `flags_host`.
 void launch_leaf_flood_fill(bs_ctx* ctx, bs_volume* v, int slot, std::vector<uint8_t>& flags_host) {
     flags_host.assign(v->n_leaves, 0);
     if (!v->n_leaves) return;
-    uint8_t* d_flags = ctx->scratch.as<uint8_t>(slot, v->n_leaves);
-    k_leaf_flood_fill<<<div_up(v->n_leaves, WAVES_PER_BLOCK), 256, 0, ctx->stream>>>(v->n_leaves, v->masks, v->values,
-                                                                                   d_flags);
-    BS_HIP(hipGetLastError());
+    const uint8_t* d_flags = launch_leaf_flood_fill(ctx, v, slot);
     BS_HIP(hipMemcpyAsync(flags_host.data(), d_flags, v->n_leaves, hipMemcpyDeviceToHost, ctx->stream));
 }
 
@@ -634,6 +649,71 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
         last = now;
         return ms;
     };
+    // the result in `a`; `plan` says where each leaf comes from
+    auto finish = [&](bs_volume& out, std::vector<TileRec>&& tiles) {
+        free_leaves(a);
+        free_leaves(b);
+        a->n_leaves = out.n_leaves;
+        a->origins = out.origins;
+        a->masks = out.masks;
+        a->values = out.values;
+        out.origins = nullptr;
+        out.masks = nullptr;
+        out.values = nullptr;
+        a->tiles = std::move(tiles);
+    };
+    auto assemble = [&](bs_volume& out, uint64_t n_out, const int4* refs, const int4* origins, EventPair& ev_asm) {
+        ev_asm.start(ctx->stream);
+        if (n_out) {
+            k_csg_assemble<<<div_up(n_out, WAVES_PER_BLOCK), 256, 0, ctx->stream>>>(
+                n_out, refs, origins, a->masks, a->values, b->masks, b->values, reinterpret_cast<int4*>(out.origins),
+                out.masks, out.values);
+            BS_HIP(hipGetLastError());
+        }
+        ev_asm.stop(ctx->stream);
+    };
+    // Both trees on the device, where they fit and the root's flood fill has no
+    // gap to close; the host's form of the tree otherwise.
+    DeviceTree* da = ensure_tree(ctx, a);
+    DeviceTree* db = da ? ensure_tree(ctx, b) : nullptr;
+    if (da && db && !tree_has_root_gap(*da) && !tree_has_root_gap(*db)) {
+        cs.ms_topology = lap();
+        EventPair ev_flood, ev_asm;
+        da->pending = db->pending = ctx->stream;
+        ev_flood.start(ctx->stream);
+        const uint8_t* fa = launch_leaf_flood_fill(ctx, a, S_FLAGS_A);
+        const uint8_t* fb = launch_leaf_flood_fill(ctx, b, S_FLAGS_B);
+        ev_flood.stop(ctx->stream);
+        tree_flood_fill(ctx, *da, fa);
+        tree_flood_fill(ctx, *db, fb);
+        TreeCsg plan = tree_csg(ctx, *da, *db, {reinterpret_cast<const int4*>(a->origins), fa, a->n_leaves},
+                                {reinterpret_cast<const int4*>(b->origins), fb, b->n_leaves}, op);
+        cs.ms_plan = lap();
+        cs.n_paired = plan.n_paired;
+        bs_volume out;
+        out.device = a->device;
+        try {
+            alloc_leaves(&out, plan.n_out);
+            cs.ms_memory = lap();
+            assemble(out, plan.n_out, plan.refs, plan.origins, ev_asm);
+            BS_HIP(hipStreamSynchronize(ctx->stream));
+        } catch (...) {
+            free_leaves(&out, ctx->stream);
+            throw;
+        }
+        cs.ms_flood = ev_flood.ms();
+        cs.ms_assemble = ev_asm.ms();
+        lap();
+        da->pending = db->pending = plan.tree->pending = nullptr;
+        finish(out, std::move(plan.tiles));
+        a->tree = std::move(plan.tree);
+        b->tree.reset();
+        cs.ms_memory += lap();
+        cs.n_out = a->n_leaves;
+        cs.ms_wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_wall).count();
+        ctx->last_csg = cs;
+        return;
+    }
     ensure_topologies(ctx, a, b);
     Topology& ta = *a->topo;
     Topology& tb = *b->topo;
@@ -755,16 +835,10 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
     try {
         alloc_leaves(&out, n_out);
         cs.ms_memory = lap();
-        ev_asm.start(ctx->stream);
-        if (n_out) {
-            int4* d_host = ctx->scratch.as<int4>(S_CSG_PLAN, 2 * n_out);
+        int4* d_host = ctx->scratch.as<int4>(S_CSG_PLAN, 2 * n_out);
+        if (n_out)
             BS_HIP(hipMemcpyAsync(d_host, host.data(), sizeof(int4) * host.size(), hipMemcpyHostToDevice, ctx->stream));
-            k_csg_assemble<<<div_up(n_out, WAVES_PER_BLOCK), 256, 0, ctx->stream>>>(
-                n_out, d_host, d_host + n_out, a->masks, a->values, b->masks, b->values,
-                reinterpret_cast<int4*>(out.origins), out.masks, out.values);
-            BS_HIP(hipGetLastError());
-        }
-        ev_asm.stop(ctx->stream);
+        assemble(out, n_out, d_host, d_host + n_out, ev_asm);
         BS_HIP(hipStreamSynchronize(ctx->stream));
         cs.ms_assemble = ev_asm.ms();
     } catch (...) {
@@ -772,17 +846,8 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
         throw;
     }
     lap();
-    free_leaves(a);
-    free_leaves(b);
+    finish(out, std::move(tiles));
     cs.ms_memory += lap();
-    a->n_leaves = out.n_leaves;
-    a->origins = out.origins;
-    a->masks = out.masks;
-    a->values = out.values;
-    out.origins = nullptr;
-    out.masks = nullptr;
-    out.values = nullptr;
-    a->tiles = std::move(tiles);
     a->topo = ta.compact(new_index);
     cs.ms_compact = lap();
     cs.n_out = n_out;

@@ -121,12 +121,13 @@ typedef struct {
     double ms_assemble;       /* result assembly kernel (events)              */
     double ms_wall;           /* the whole call on the host clock             */
     /* host-clock parts of ms_wall: building the operands' upper levels from
-     * their leaves (when they carry none), the upper-level flood fill, CSG
-     * and output plan, device allocation and release, and the result's
-     * upper levels */
+     * their leaves (when they carry none), the flood fill, upper-level CSG
+     * and output plan, device allocation and release, and (trees in the
+     * host's form only) the result's upper levels */
     double ms_topology, ms_plan, ms_memory, ms_compact;
-    /* ms_plan split: flags and upper-level flood fill, the tree CSG with the
-     * collection of the result's leaves, the output order and plan */
+    /* ms_plan split, trees in the host's form only: flags and upper-level
+     * flood fill, the tree CSG with the collection of the result's leaves,
+     * the output order and plan */
     double ms_plan_fill, ms_plan_tree, ms_plan_order;
 } bs_csg_stats;
 

@@ -203,3 +203,68 @@ def test_csg_with_empty_and_self(gpu_ctx, oracle_lib):
         c.union(c)
     with pytest.raises(ValueError):
         a.union(c)                                       # a was consumed above
+
+
+@pytest.mark.parametrize("extra", ["none", "far in x", "gap in z", "next root in z"])
+def test_chain_keeps_the_tree(gpu_ctx, oracle_lib, extra):
+    """Every step of a chain of CSG, offset, sign and meshing calls against the
+    oracle, with the upper levels on the device (alone, and over a root border)
+    and in the host's form (a far voxel: too many blocks between; a gap between
+    two root blocks on one z line), carried from step to step and through
+    clones: leaves, masks, values, tiles, signs and the marching-cubes soup."""
+    h = 0.05
+    B = bs.VolumeBuilder(gpu_ctx, h)
+    at = {"none": None, "far in x": (7000000, 3, 5), "gap in z": (0, 0, 8192 + 40), "next root in z": (2, 1, 4096 + 9)}[extra]
+
+    def pair(kind, *args):
+        return getattr(B, kind)(*args), getattr(oracle_lib, kind)(*args, h)
+
+    def extra_pair(neg):
+        idx = np.array([at, (at[0] + 1, at[1], at[2])], np.int32)
+        val = np.array([-0.02 if neg else 0.02, 0.03], np.float32)
+        return bs.volume_from_voxels(idx, val, h, gpu_ctx), oracle_lib.from_voxels(idx, val, h)
+
+    ax = np.arange(-60, 60, 7, dtype=np.int32)
+    q = np.stack(np.meshgrid(ax, ax, ax, indexing="ij"), -1).reshape(-1, 3)
+    if at:
+        q = np.concatenate([q, np.array(at, np.int32) + ax[:, None] * np.array([0, 0, 3], np.int32)])
+
+    def same(g, r, signs):
+        assert_same_volume(g.export(), r.export())
+        if signs:
+            assert np.array_equal(g.signs_at(q), r.signs_at(q))
+
+    g, r = pair("sphere", 2.0, (0.1, -0.2, 0.3))
+    if at:
+        e = extra_pair(True)
+        g, r = g.union(e[0]), r.union(e[1])
+        same(g, r, False)
+    b = pair("sphere", 1.1, (1.6, 0.2, 0.0))
+    g, r = g.union(b[0]), r.union(b[1])
+    same(g, r, False)
+    b = pair("sphere", 0.9, (-0.4, 0.0, 0.2))          # inside: tiles
+    g, r = g.clone().union(b[0]), r.union(b[1])
+    same(g, r, True)
+    b = pair("cuboid", (-3.0, -3.0, 0.4), (3.0, 3.0, 3.0))
+    g, r = g.subtract(b[0]), r.subtract(b[1])
+    same(g, r, False)
+    got = bs.MarchingCubesMesher(gpu_ctx).with_voxel_size(h).mesh(g)
+    want = r.marching_cubes(h)
+    assert got.shape == want.shape and np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    if g.export().tile_values.size == 0 or np.all(np.abs(g.export().tile_values) > 2 * h):
+        g, r = g.offset(-0.2), r.offset(-0.2)
+        same(g, r, False)
+    b = pair("sphere", 1.5, (0.0, 0.9, 0.0))
+    if at:
+        e = extra_pair(False)
+        b = b[0].union(e[0]), b[1].union(e[1])
+    g, r = g.intersect(b[0]), r.intersect(b[1])
+    same(g, r, True)
+    g.flood_fill()
+    r.flood_fill()
+    b = pair("sphere", 0.7, (0.0, 0.2, -0.3))
+    g, r = g.subtract(b[0]), r.subtract(b[1])
+    same(g, r, True)
+    got = bs.MarchingCubesMesher(gpu_ctx).with_voxel_size(h).mesh(g)
+    want = r.marching_cubes(h)
+    assert got.shape == want.shape and np.array_equal(got.view(np.uint32), want.view(np.uint32))
