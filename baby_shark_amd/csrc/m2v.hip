@@ -227,7 +227,7 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_subtri_setup(const float* __res
         const F3 nn = {e0.y * ec.z - e0.z * ec.y, e0.z * ec.x - e0.x * ec.z, e0.x * ec.y - e0.y * ec.x};
         const float nl2 = nn.x * nn.x + nn.y * nn.y + nn.z * nn.z;
         const float l0sq = e0.x * e0.x + e0.y * e0.y + e0.z * e0.z;
-        const bool degenerate = !(nl2 > 0.0f) || !(l0sq > 0.0f);
+        bool degenerate = !(nl2 > 0.0f) || !(l0sq > 0.0f);
         if (!degenerate) {
             const float l0 = sqrtf(l0sq), inl = 1.0f / sqrtf(nl2);
             const F3 U = {e0.x / l0, e0.y / l0, e0.z / l0};
@@ -236,23 +236,26 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_subtri_setup(const float* __res
             r.U[0] = U.x; r.U[1] = U.y; r.U[2] = U.z;
             r.V[0] = V.x; r.V[1] = V.y; r.V[2] = V.z;
             r.N[0] = N.x; r.N[1] = N.y; r.N[2] = N.z;
+            const float cu = U.x * ec.x + U.y * ec.y + U.z * ec.z;
+            const float cv = V.x * ec.x + V.y * ec.y + V.z * ec.z;
+            const float fx = cu - l0;
             r.L0 = l0;
-            r.inv0 = 1.0f / l0;
-            r.cu = U.x * ec.x + U.y * ec.y + U.z * ec.z;
-            r.cv = V.x * ec.x + V.y * ec.y + V.z * ec.z;
-            r.e1x = r.cu - l0;
-            r.e1y = r.cv;
-            const float l1 = r.e1x * r.e1x + r.e1y * r.e1y;
-            const float l2 = r.cu * r.cu + r.cv * r.cv;
-            r.inv1 = l1 > 0.0f ? 1.0f / l1 : 0.0f;
-            r.inv2 = l2 > 0.0f ? 1.0f / l2 : 0.0f;
+            r.L1 = sqrtf(fx * fx + cv * cv);
+            r.L2 = sqrtf(cu * cu + cv * cv);
+            // c on b or on a within rounding: no direction to project on
+            degenerate = !(r.L1 > 0.0f) || !(r.L2 > 0.0f);
+            r.e1x = fx / r.L1;
+            r.e1y = cv / r.L1;
+            r.e2x = cu / r.L2;
+            r.e2y = cv / r.L2;
             r.flags = 0;
-        } else {
+        }
+        if (degenerate) {
             for (int k = 0; k < 3; ++k) r.U[k] = r.V[k] = r.N[k] = 0.0f;
-            r.L0 = r.inv0 = r.cu = r.cv = r.e1x = r.e1y = r.inv1 = r.inv2 = 0.0f;
+            r.L0 = r.e1x = r.e1y = r.L1 = r.e2x = r.e2y = r.L2 = 0.0f;
             r.flags = 1;
         }
-        r.pad = 0;
+        r.pad[0] = r.pad[1] = 0;
         for (int k = 0; k < 3; ++k) { r.box[k] = lo[k]; r.box[3 + k] = hi[k]; }
         recs[t] = r;
         uint32_t nl = 1;
@@ -502,9 +505,13 @@ __global__ __launch_bounds__(DIST_BLOCK) void k_distance(const int32_t* __restri
             const int s = (int)(__umul24((uint32_t)lane, m_yz) >> 16);
             const int rr = lane - (int)__umul24((uint32_t)s, (uint32_t)nyz);
             const int yq = (int)(__umul24((uint32_t)rr, m_z) >> 16);
-            const int y = y0 + yq, z = z0 + (rr - (int)__umul24((uint32_t)yq, (uint32_t)nz));
-            const int loff = ((y - oy) << 3) | (z - oz);
-            const float py = (float)y * h, pz = (float)z * h;
+            const int zq = rr - (int)__umul24((uint32_t)yq, (uint32_t)nz);
+            const float py = (float)(y0 + yq) * h, pz = (float)(z0 + zq) * h;
+            // the lane's first voxel in the leaf; a step in x is spp slices on
+            int vo = ((x0 - ox) << 6) + ((y0 - oy) << 3) + (z0 - oz) + (s << 6) + (yq << 3) + zq;
+            // x runs as a float: whole numbers below 2^24, so every step is exact
+            float x = (float)(x0 + s);
+            const float xe = (float)x1, xs = (float)spp;
             if (s < spp) {
                 if (r.flags == 0) {
                     const float dy = py - r.a[1], dz = pz - r.a[2];
@@ -514,23 +521,24 @@ __global__ __launch_bounds__(DIST_BLOCK) void k_distance(const int32_t* __restri
                     // the fields the x loop reads, in scalar registers before it
                     // starts (else their loads sink into the loop body)
                     const PlaneRec q = plane_rec(r);
-                    for (int x = x0 + s; x <= x1; x += spp) {
-                        const float dx = (float)x * h - q.a0;
+                    unsigned long long* slot = best + vo;
+                    for (; x <= xe; x += xs, slot += spp << 6) {
+                        const float dx = x * h - q.a0;
                         const float pu = __builtin_fmaf(q.U0, dx, bu);
                         const float pv = __builtin_fmaf(q.V0, dx, bv);
                         const float pw = __builtin_fmaf(q.N0, dx, bw);
                         const float d2 = __builtin_fmaf(pw, pw, plane_dist2(q, pu, pv));
                         const unsigned long long key = ((unsigned long long)__float_as_uint(d2) << 32) | t;
-                        atomicMin(&best[((x - ox) << 6) | loff], key);
+                        atomicMin(slot, key);
                     }
                 } else {
                     const float* v = sub + 9 * (uint64_t)t;
-                    for (int x = x0 + s; x <= x1; x += spp) {
+                    for (; x <= xe; x += xs, vo += spp << 6) {
                         const float d = ericson_distance({v[0], v[1], v[2]}, {v[3], v[4], v[5]}, {v[6], v[7], v[8]},
-                                                         {(float)x * h, py, pz});
+                                                         {x * h, py, pz});
                         if (d == d) {  // a NaN distance never enters the field (`dist < cur` is false)
                             const unsigned long long key = ((unsigned long long)__float_as_uint(d * d) << 32) | t;
-                            atomicMin(&best[((x - ox) << 6) | loff], key);
+                            atomicMin(&best[vo], key);
                         }
                     }
                 }

@@ -85,19 +85,20 @@ __device__ inline float ericson_distance(F3 A, F3 B, F3 C, F3 p) {
 // Per sub-triangle record for the distance kernel (112 B, read wave-uniformly
 // through scalar loads).  The triangle is expressed in its own frame: origin
 // a, axes U = (b-a)/|b-a|, V = N x U, N = unit normal; there b = (L0, 0) and
-// c = (cu, cv) with cv > 0.  A degenerate sub-triangle (zero area or a zero
-// first edge) has flags = 1 and is evaluated with the reference's own
-// closest-point arithmetic instead.
+// c = (cu, cv) with cv > 0.  The edges b->c and a->c are unit vectors and
+// lengths: a point's coordinates along and across an edge are then two
+// multiply-adds each, and the clamp takes the length, not a division.  A
+// degenerate sub-triangle (zero area or an edge of no length) has flags = 1 and
+// is evaluated with the reference's own closest-point arithmetic instead.
 struct alignas(16) DistRec {
     float a[3];
     float U[3], V[3], N[3];
-    float L0, inv0;       // |b-a|, 1/|b-a|
-    float cu, cv;         // c in the frame
-    float e1x, e1y, inv1; // c-b in the frame, 1/|c-b|^2
-    float inv2;           // 1/|a-c|^2
-    int box[6];           // dilated voxel box lo.xyz, hi.xyz (inclusive)
+    float L0;           // |b-a|
+    float e1x, e1y, L1; // (c-b)/|c-b| in the frame, |c-b|
+    float e2x, e2y, L2; // (c-a)/|c-a| in the frame, |c-a|
+    int box[6];         // dilated voxel box lo.xyz, hi.xyz (inclusive)
     int flags;
-    int pad;
+    int pad[2];
 };
 static_assert(sizeof(DistRec) == 112, "DistRec layout");
 
@@ -105,44 +106,44 @@ static_assert(sizeof(DistRec) == 112, "DistRec layout");
 // of the record's loads are issued before it, one wait for the lot.
 __device__ inline void pin_dist_rec(const DistRec& r) {
     asm volatile("" ::"s"(r.a[0]), "s"(r.a[1]), "s"(r.a[2]), "s"(r.U[0]), "s"(r.U[1]), "s"(r.U[2]), "s"(r.V[0]),
-                 "s"(r.V[1]), "s"(r.V[2]), "s"(r.N[0]), "s"(r.N[1]), "s"(r.N[2]), "s"(r.L0), "s"(r.inv0), "s"(r.cu),
-                 "s"(r.cv), "s"(r.e1x), "s"(r.e1y), "s"(r.inv1), "s"(r.inv2), "s"(r.box[0]), "s"(r.box[1]),
-                 "s"(r.box[2]), "s"(r.box[3]), "s"(r.box[4]), "s"(r.box[5]), "s"(r.flags));
+                 "s"(r.V[1]), "s"(r.V[2]), "s"(r.N[0]), "s"(r.N[1]), "s"(r.N[2]), "s"(r.L0), "s"(r.e1x), "s"(r.e1y),
+                 "s"(r.L1), "s"(r.e2x), "s"(r.e2y), "s"(r.L2), "s"(r.box[0]), "s"(r.box[1]), "s"(r.box[2]),
+                 "s"(r.box[3]), "s"(r.box[4]), "s"(r.box[5]), "s"(r.flags));
 }
 
 // The fields of a DistRec that the per-voxel step reads, held in scalar
 // registers: plane_rec's empty asm takes each as an SGPR operand, so their
 // loads are all issued (and waited for) once per candidate.
 struct PlaneRec {
-    float a0, U0, V0, N0, L0, inv0, cu, cv, e1x, e1y, inv1, inv2;
+    float a0, U0, V0, N0, L0, e1x, e1y, L1, e2x, e2y, L2;
 };
 
 __device__ inline PlaneRec plane_rec(const DistRec& r) {
-    PlaneRec q{r.a[0], r.U[0], r.V[0], r.N[0], r.L0, r.inv0, r.cu, r.cv, r.e1x, r.e1y, r.inv1, r.inv2};
-    asm volatile("" ::"s"(q.a0), "s"(q.U0), "s"(q.V0), "s"(q.N0), "s"(q.L0), "s"(q.inv0), "s"(q.cu), "s"(q.cv),
-                 "s"(q.e1x), "s"(q.e1y), "s"(q.inv1), "s"(q.inv2));
+    PlaneRec q{r.a[0], r.U[0], r.V[0], r.N[0], r.L0, r.e1x, r.e1y, r.L1, r.e2x, r.e2y, r.L2};
+    asm volatile("" ::"s"(q.a0), "s"(q.U0), "s"(q.V0), "s"(q.N0), "s"(q.L0), "s"(q.e1x), "s"(q.e1y), "s"(q.L1),
+                 "s"(q.e2x), "s"(q.e2y), "s"(q.L2));
     return q;
 }
 
 // In-plane squared distance from (pu, pv) to the frame triangle (0,0), (L0,0),
-// (cu,cv): 0 inside, else the nearest clamped edge projection.  The three edge
-// terms are computed for every lane (the empty asm keeps them out of a branch
-// on `inside`, which would cost more in mask handling than it saves).
+// (cu,cv): 0 inside, else the nearest of the three edges.  For an edge, s runs
+// along it and n across it (positive on the inner side); the squared distance is
+// n^2 plus the square of what s lies outside [0, L].  The three edge terms are
+// computed for every lane (the empty asm keeps them out of a branch on `inside`,
+// which would cost more in mask handling than it saves).
 __device__ inline float plane_dist2(const PlaneRec& r, float pu, float pv) {
-    const float t0 = __builtin_amdgcn_fmed3f(pu * r.inv0, 0.0f, 1.0f);
-    const float qx = __builtin_fmaf(-t0, r.L0, pu);
-    const float d0 = __builtin_fmaf(qx, qx, pv * pv);
+    const float q0 = pu - __builtin_amdgcn_fmed3f(pu, 0.0f, r.L0);
+    const float d0 = __builtin_fmaf(q0, q0, pv * pv);
     const float rx = pu - r.L0;
-    const float t1 = __builtin_amdgcn_fmed3f(__builtin_fmaf(rx, r.e1x, pv * r.e1y) * r.inv1, 0.0f, 1.0f);
-    const float sx = __builtin_fmaf(-t1, r.e1x, rx), sy = __builtin_fmaf(-t1, r.e1y, pv);
-    const float d1 = __builtin_fmaf(sx, sx, sy * sy);
-    const float wx = pu - r.cu, wy = pv - r.cv;
-    const float t2 = __builtin_amdgcn_fmed3f(-__builtin_fmaf(wx, r.cu, wy * r.cv) * r.inv2, 0.0f, 1.0f);
-    const float ux = __builtin_fmaf(t2, r.cu, wx), uy = __builtin_fmaf(t2, r.cv, wy);
-    const float d2 = __builtin_fmaf(ux, ux, uy * uy);
-    const float f1 = __builtin_fmaf(r.e1x, pv, -r.e1y * rx);   // cross(c-b, q-b)
-    const float f2 = __builtin_fmaf(r.cv, wx, -r.cu * wy);     // cross(a-c, q-c)
-    const bool inside = fminf(fminf(pv, f1), f2) >= 0.0f;
+    const float s1 = __builtin_fmaf(rx, r.e1x, pv * r.e1y);
+    const float n1 = __builtin_fmaf(r.e1x, pv, -(r.e1y * rx));
+    const float q1 = s1 - __builtin_amdgcn_fmed3f(s1, 0.0f, r.L1);
+    const float d1 = __builtin_fmaf(q1, q1, n1 * n1);
+    const float s2 = __builtin_fmaf(pu, r.e2x, pv * r.e2y);
+    const float n2 = __builtin_fmaf(r.e2y, pu, -(r.e2x * pv));
+    const float q2 = s2 - __builtin_amdgcn_fmed3f(s2, 0.0f, r.L2);
+    const float d2 = __builtin_fmaf(q2, q2, n2 * n2);
+    const bool inside = fminf(fminf(pv, n1), n2) >= 0.0f;
     float m = fminf(fminf(d0, d1), d2);
     asm volatile("" : "+v"(m));
     return inside ? 0.0f : m;
