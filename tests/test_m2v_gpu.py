@@ -336,3 +336,32 @@ def test_tiny_meshes(gpu_ctx, oracle_lib, n):
     levels): the first n faces of a level-1 icosphere, open, against the oracle."""
     soup = mg.sphere_soup(1, radius=0.5)[:n]
     check_case(gpu_ctx, oracle_lib, soup, 0.05, 2, closed=False)
+
+
+@pytest.mark.parametrize("accuracy,level,h,band", [
+    (2.0, 2, 0.4, 0),    # a handful of voxels: the last chunk not full, its ball as wide as the mesh
+    (2.0, 4, 0.03, 1),   # thin band: chunks of partly active blocks
+    (2.0, 5, 0.011, 3),  # full chunks, most of the tree summed per chunk
+    (8.0, 4, 0.03, 2),   # longer lists
+    (64.0, 4, 0.03, 2),  # nothing far nearby: lists outgrow their room, voxels walk from the root
+])
+@pytest.mark.parametrize("open_mesh", [False, True])
+def test_chunk_far_field_signs(gpu_ctx, oracle_lib, accuracy, level, h, band, open_mesh):
+    """Signs against exact winding numbers, wherever these are further from the
+    threshold than the order-2 approximation error (0.1, as in the open-cap
+    test): chunks with a far-field polynomial and without one, short and
+    overflowing node lists."""
+    soup = mg.displaced_icosphere(level, radius=0.7, seed=4)
+    if open_mesh:
+        soup = soup[soup.mean(axis=1)[:, 2] > -0.2]
+    m = bs.MeshToVolume(gpu_ctx).with_voxel_size(h).with_narrow_band_width(band)
+    m.params.wn_accuracy = accuracy
+    ge = m.convert(soup).export()
+    li, off = np.nonzero(ge.active())
+    pick = RNG.permutation(li.size)[:4000]
+    li, off = li[pick], off[pick]
+    pts = voxel_points(ge.origins, li, off, h)
+    w = oracle_lib.winding_numbers(soup, pts, 2.0, exact=True)[2].astype(np.float64)
+    sure = (np.abs(w - 0.2) >= WN_AMBIGUITY) & ~on_surface(ge.values[li, off], pts, h)
+    assert sure.sum() > 0.5 * len(pick)
+    assert np.array_equal(np.signbit(ge.values[li, off])[sure], ~(w < 0.2)[sure])
