@@ -44,7 +44,7 @@ struct DeviceTree {
 
 // The volume's tree on the device, made from its leaves (and tiles) or from its
 // Topology, which it replaces; nullptr when it does not fit: more than 2^24
-// 128^3 blocks in the box of the leaves, 4096 root blocks in it or 2^16 nodes.
+// 128^3 blocks in the box of the leaves, 256 root blocks in it or 2^16 nodes.
 DeviceTree* ensure_tree(bs_ctx* ctx, bs_volume* v);
 std::unique_ptr<DeviceTree> clone_tree(const DeviceTree& t);
 // The host's form of a volume's device tree.
