@@ -23,10 +23,10 @@ sys.path.insert(0, ROOT)
 
 PEAK_FP32_TFLOPS = 157.3  # MI355X dense FP32 vector, published
 PEAK_HBM_GBS = 8000.0
-# HBM bytes per k_winding launch at the default workload, from the FETCH_SIZE
-# (x2.0 calibration) and WRITE_SIZE counters of `bench.py --traffic-probe`
-# under rocprofv3 --pmc
-WINDING_TRAFFIC_BYTES = 1.015e9
+# HBM bytes per launch at the default workload, from the FETCH_SIZE (x2.0
+# calibration) and WRITE_SIZE counters of `bench.py --traffic-probe` under
+# rocprofv3 --pmc; the winding pass is k_far_field and k_winding
+TRAFFIC_BYTES = {"k_distance": 4.74e9, "k_winding": 1.63e9}
 
 
 def traffic_probe():
@@ -485,7 +485,8 @@ def main():
 
     # work: the winding kernel's visit counters (one step with the counting
     # variant); kernel durations: HIP events on the library stream around each
-    # phase of the production (non-counting) kernels
+    # phase of the production (non-counting) kernels.  The winding phase holds
+    # k_far_field too, whose operations are not counted
     ctx.set_profiling(True, counters=True)
     v = m2v.convert(dev)
     v.free()
@@ -511,7 +512,7 @@ def main():
     # FP32 (VALU), priced against MI355X's published FP32 peak
     roof = {"bound": "mfma", "bound_detail": "compute, vector FP32 (VALU); no matrix-shaped work", "kernel": dom, "achieved": round(kernels[dom]["tflops"], 3),
             "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": round(kernels[dom]["tflops"] / PEAK_FP32_TFLOPS, 4),
-            "traffic": WINDING_TRAFFIC_BYTES if dom == "k_winding" else None,
+            "traffic": TRAFFIC_BYTES[dom],
             "traffic_source": "profiles/m2v_icosphere_L8_traffic.md (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE)"}
 
     out = {
