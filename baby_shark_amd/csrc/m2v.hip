@@ -3265,7 +3265,8 @@ void mesh_to_volume_device(bs_ctx* ctx, const float* d_tris, uint64_t n, const b
         FarChunk* chunks = nullptr;
         uint32_t* far_list = nullptr;
         float* coef = nullptr;
-        if (wn_list == act) {
+        // the polynomials are in voxel units: 1 / h^3 has to be a normal float
+        if (wn_list == act && h > 1e-12f && h < 1e12f) {
             const uint32_t n_chunks = (uint32_t)div_up(n_wn, 64);
             const uint32_t pool = (uint32_t)std::min<uint64_t>((uint64_t)n_chunks * FF_POOL, 1u << 30);
             chunks = S.as<FarChunk>(S_WN_CHUNKS, n_chunks);
