@@ -80,7 +80,8 @@ struct Scratch {
         if (cap[slot] < bytes) {
             if (ptr[slot]) BS_HIP(hipFree(ptr[slot]));
             ptr[slot] = nullptr;
-            size_t b = bytes + bytes / 4 + 256;
+            cap[slot] = 0;  // when the new buffer cannot be had, nothing is left
+            const size_t b = bytes + bytes / 4 + 256;
             BS_HIP(device_malloc(&ptr[slot], b));
             cap[slot] = b;
         }
