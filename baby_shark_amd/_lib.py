@@ -136,6 +136,7 @@ def load():
             "bs_volume_clone": (C.c_int, [vp, pp]),
             "bs_volume_free": (None, [vp]),
             "bs_release_cached_memory": (None, []),
+            "bs_refuse_allocations": (C.c_uint64, [C.c_uint64, C.c_uint64]),
             "bs_volume_info_get": (C.c_int, [vp, C.POINTER(VolumeInfo)]),
             "bs_volume_export": (C.c_int, [vp, i32p, u64p, f32p]),
             "bs_volume_export_tiles": (C.c_int, [vp, i32p, i32p, f32p]),

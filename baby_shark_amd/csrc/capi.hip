@@ -33,6 +33,7 @@ void marching_cubes_device(bs_ctx* ctx, bs_volume* vol, float voxel_size, float*
                            bs_dc_stats* stats);
 void volume_from_voxels(bs_ctx* ctx, const int32_t* idx, const float* values, uint64_t n, float h, bs_volume** out);
 void volume_signs_at(bs_ctx* ctx, bs_volume* v, const int32_t* idx, uint64_t n, uint8_t* out_neg);
+uint64_t refuse_allocations(uint64_t first, uint64_t count);
 
 template <class F>
 static bs_status guarded(F&& f) {
@@ -300,6 +301,7 @@ bs_status bs_volume_clone(const bs_volume* v, bs_volume** out) {
         c->voxel_size = v->voxel_size;
         c->n_leaves = v->n_leaves;
         c->tiles = v->tiles;
+        c->tree_lost = v->tree_lost;
         try {
             if (v->topo) c->topo = v->topo->clone();
             if (v->tree) c->tree = clone_tree(*v->tree);
@@ -321,6 +323,8 @@ bs_status bs_volume_clone(const bs_volume* v, bs_volume** out) {
 }
 
 void bs_release_cached_memory(void) { release_cached_memory(); }
+
+uint64_t bs_refuse_allocations(uint64_t first, uint64_t count) { return refuse_allocations(first, count); }
 
 void bs_volume_free(bs_volume* v) {
     if (!v) return;

@@ -40,6 +40,9 @@ void set_last_error(const std::string& msg);
 // hipMalloc on the current device; when memory runs out, the library's pools
 // are emptied and it tries once more.
 hipError_t device_malloc(void** p, uint64_t bytes);
+// True when bs_refuse_allocations has this request of the thread fail; every
+// request for device memory asks once.
+bool allocation_refused();
 
 // Device blocks from a per-device pool of released ones (device_pool.hip).
 // free_block takes any device pointer (one that the pool did not hand out goes
@@ -139,6 +142,9 @@ struct bs_volume {
     // upper levels, in one form or the other; built from the leaves and tiles when absent
     std::unique_ptr<bs::Topology> topo;
     std::unique_ptr<bs::DeviceTree> tree;
+    // a call that works on the host's form in place failed part-way: the leaves are whole, but what the
+    // upper levels held beyond them is lost
+    bool tree_lost = false;
 };
 
 namespace bs {

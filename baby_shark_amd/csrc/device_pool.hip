@@ -58,9 +58,10 @@ void free_blocks(const std::vector<DeviceBlock>& blocks) {
     }
 }
 
-}  // namespace
+// bs_refuse_allocations: requests of this thread so far, and the ones to refuse
+thread_local uint64_t t_requests = 0, t_refuse_from = 0, t_refuse_to = 0;
 
-hipError_t device_malloc(void** p, uint64_t bytes) {
+hipError_t malloc_or_empty_pools(void** p, uint64_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
@@ -74,8 +75,29 @@ hipError_t device_malloc(void** p, uint64_t bytes) {
     return e;
 }
 
+}  // namespace
+
+bool allocation_refused() {
+    ++t_requests;
+    return t_requests >= t_refuse_from && t_requests < t_refuse_to;
+}
+
+uint64_t refuse_allocations(uint64_t first, uint64_t count) {
+    const uint64_t seen = t_requests;
+    t_requests = 0;
+    t_refuse_from = first;
+    t_refuse_to = first ? first + count : 0;
+    return seen;
+}
+
+hipError_t device_malloc(void** p, uint64_t bytes) {
+    *p = nullptr;
+    return allocation_refused() ? hipErrorOutOfMemory : malloc_or_empty_pools(p, bytes);
+}
+
 void* alloc_block(uint64_t bytes) {
     if (!bytes) bytes = 256;
+    if (allocation_refused()) BS_HIP(hipErrorOutOfMemory);
     int dev = -1;
     BS_HIP(hipGetDevice(&dev));
     BlockPool& P = block_pool();
@@ -95,7 +117,7 @@ void* alloc_block(uint64_t bytes) {
         }
     }
     void* p = nullptr;
-    BS_HIP(device_malloc(&p, bytes));
+    BS_HIP(malloc_or_empty_pools(&p, bytes));
     try {
         std::lock_guard<std::mutex> lk(P.mu);
         P.live.emplace(p, DeviceBlock{p, bytes, dev});

@@ -794,6 +794,7 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
     EventPair ev;
     ev.start(ctx->stream);
     BS_REQUIRE(vol->device == ctx->device, BS_ERR_INVALID_ARG, "volume lives on another device");
+    require_tree(vol);
     const float two_h = vol->voxel_size * 2.0f;
     // fast_sweep.rs:100 unwraps the leaf at every queued origin, and the queue
     // holds every active tile that survives remove_if: the reference panics.

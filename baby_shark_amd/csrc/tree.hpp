@@ -35,7 +35,7 @@ struct DeviceTree {
     std::map<Topology::Key, int32_t> root;  // -> 32^3 node
     TreeView v{};
     void* block = nullptr;
-    hipStream_t pending = nullptr;  // a stream that may still work on it (a call that failed part-way)
+    hipStream_t pending = nullptr;  // a stream that may still work on it, within a call
     DeviceTree() = default;
     DeviceTree(const DeviceTree&) = delete;
     DeviceTree& operator=(const DeviceTree&) = delete;
@@ -46,6 +46,8 @@ struct DeviceTree {
 // Topology, which it replaces; nullptr when it does not fit: more than 2^24
 // 128^3 blocks in the box of the leaves, 256 root blocks in it or 2^16 nodes.
 DeviceTree* ensure_tree(bs_ctx* ctx, bs_volume* v);
+// Throws for a volume whose upper levels a failed call lost.
+void require_tree(const bs_volume* v);
 std::unique_ptr<DeviceTree> clone_tree(const DeviceTree& t);
 // The host's form of a volume's device tree.
 std::unique_ptr<Topology> download_tree(bs_ctx* ctx, const bs_volume* v);
@@ -58,8 +60,9 @@ bool tree_has_root_gap(const DeviceTree& t);
 void tree_flood_fill(bs_ctx* ctx, const DeviceTree& t, const uint8_t* leaf_flags);
 
 // CSG of two flood-filled trees (root_node/csg.rs:9-58, internal_node/csg.rs:
-// 68-162) with `a` as self; both are spent.  The result's leaves in origin order:
-// refs[i] = (leaf of a, leaf of b, LEAF_* | negate << 8, 0), origins[i].
+// 68-162) with `a` as self.  The slot rules work on copies, so that a call that
+// fails leaves both operands' trees as they were.  The result's leaves in origin
+// order: refs[i] = (leaf of a, leaf of b, LEAF_* | negate << 8, 0), origins[i].
 struct TreeOperand {
     const int4* origins;
     const uint8_t* flags;  // bit 2: mask empty
@@ -67,11 +70,13 @@ struct TreeOperand {
 };
 struct TreeCsg {
     std::unique_ptr<DeviceTree> tree;
-    std::vector<TileRec> tiles;  // active tiles in tree order
+    std::unique_ptr<DeviceTree> work_a, work_b;  // the copies, read until the stream is done
+    std::vector<TileRec> tiles;                  // active tiles in tree order
     uint64_t n_out = 0, n_paired = 0;
     const int4 *refs = nullptr, *origins = nullptr;  // context scratch
 };
-TreeCsg tree_csg(bs_ctx* ctx, DeviceTree& a, DeviceTree& b, const TreeOperand& la, const TreeOperand& lb, CsgOp op);
+TreeCsg tree_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, const TreeOperand& la, const TreeOperand& lb,
+                 CsgOp op);
 
 // The tree after Volume::offset (see Topology::after_offset) of a volume whose
 // tree is `old`: the nodes of the result's leaves, with the tile values of the

@@ -90,6 +90,7 @@ void alloc_leaves(bs_volume* v, uint64_t n) {
     v->masks = nullptr;
     v->values = nullptr;
     if (!n) return;
+    if (allocation_refused()) BS_HIP(hipErrorOutOfMemory);
     LeafPool& P = leaf_pool();
     const int dev = v->device;
     if (dev >= 0 && dev < POOL_DEVICES) {
@@ -216,6 +217,7 @@ static std::vector<std::array<int32_t, 3>> leaf_origins(bs_ctx* ctx, const bs_vo
 }
 
 Topology& ensure_topology(bs_ctx* ctx, bs_volume* v) {
+    require_tree(v);
     if (v->topo) return *v->topo;
     if (v->tree) {
         v->topo = download_tree(ctx, v);
@@ -230,6 +232,8 @@ Topology& ensure_topology(bs_ctx* ctx, bs_volume* v) {
 // ensure_topology of two volumes, the second built on another host thread
 static void ensure_topologies(bs_ctx* ctx, bs_volume* a, bs_volume* b) {
     std::vector<std::array<int32_t, 3>> oa, ob;
+    require_tree(a);
+    require_tree(b);
     if (a->tree) ensure_topology(ctx, a);
     if (b->tree) ensure_topology(ctx, b);
     if (!a->topo) oa = leaf_origins(ctx, a);
@@ -679,32 +683,36 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
     if (da && db && !tree_has_root_gap(*da) && !tree_has_root_gap(*db)) {
         cs.ms_topology = lap();
         EventPair ev_flood, ev_asm;
-        da->pending = db->pending = ctx->stream;
-        ev_flood.start(ctx->stream);
-        const uint8_t* fa = launch_leaf_flood_fill(ctx, a, S_FLAGS_A);
-        const uint8_t* fb = launch_leaf_flood_fill(ctx, b, S_FLAGS_B);
-        ev_flood.stop(ctx->stream);
-        tree_flood_fill(ctx, *da, fa);
-        tree_flood_fill(ctx, *db, fb);
-        TreeCsg plan = tree_csg(ctx, *da, *db, {reinterpret_cast<const int4*>(a->origins), fa, a->n_leaves},
-                                {reinterpret_cast<const int4*>(b->origins), fb, b->n_leaves}, op);
-        cs.ms_plan = lap();
-        cs.n_paired = plan.n_paired;
         bs_volume out;
         out.device = a->device;
+        TreeCsg plan;
         try {
+            ev_flood.start(ctx->stream);
+            const uint8_t* fa = launch_leaf_flood_fill(ctx, a, S_FLAGS_A);
+            const uint8_t* fb = launch_leaf_flood_fill(ctx, b, S_FLAGS_B);
+            ev_flood.stop(ctx->stream);
+            tree_flood_fill(ctx, *da, fa);
+            tree_flood_fill(ctx, *db, fb);
+            plan = tree_csg(ctx, *da, *db, {reinterpret_cast<const int4*>(a->origins), fa, a->n_leaves},
+                            {reinterpret_cast<const int4*>(b->origins), fb, b->n_leaves}, op);
+            cs.ms_plan = lap();
+            cs.n_paired = plan.n_paired;
             alloc_leaves(&out, plan.n_out);
             cs.ms_memory = lap();
             assemble(out, plan.n_out, plan.refs, plan.origins, ev_asm);
             BS_HIP(hipStreamSynchronize(ctx->stream));
+            cs.ms_flood = ev_flood.ms();
+            cs.ms_assemble = ev_asm.ms();
         } catch (...) {
-            free_leaves(&out, ctx->stream);
+            // the operands are the caller's again, flood filled and otherwise as they were: no kernel may still
+            // read them when they are freed
+            (void)hipStreamSynchronize(ctx->stream);
+            free_leaves(&out);
             throw;
         }
-        cs.ms_flood = ev_flood.ms();
-        cs.ms_assemble = ev_asm.ms();
         lap();
-        da->pending = db->pending = plan.tree->pending = nullptr;
+        plan.tree->pending = plan.work_a->pending = nullptr;
+        if (plan.work_b) plan.work_b->pending = nullptr;
         finish(out, std::move(plan.tiles));
         a->tree = std::move(plan.tree);
         b->tree.reset();
@@ -745,6 +753,19 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
     }
     cs.ms_plan_fill = split();
 
+    // The plan is made in the operands' trees themselves: a call that fails from here on loses them.
+    struct LoseTrees {
+        bs_ctx* ctx;
+        bs_volume *a, *b;
+        bool done = false;
+        ~LoseTrees() {
+            if (done) return;
+            (void)hipStreamSynchronize(ctx->stream);
+            a->topo.reset();
+            b->topo.reset();
+            a->tree_lost = b->tree_lost = true;
+        }
+    } lose{ctx, a, b};
     std::unique_ptr<Topology> tb_owned = std::move(b->topo);
     ta.csg(std::move(*tb_owned), op);
     tb_owned.reset();
@@ -832,6 +853,7 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
     cs.ms_plan = lap();
     bs_volume out;
     out.device = a->device;
+    std::unique_ptr<Topology> compacted;
     try {
         alloc_leaves(&out, n_out);
         cs.ms_memory = lap();
@@ -841,15 +863,17 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
         assemble(out, n_out, d_host, d_host + n_out, ev_asm);
         BS_HIP(hipStreamSynchronize(ctx->stream));
         cs.ms_assemble = ev_asm.ms();
+        lap();
+        compacted = ta.compact(new_index);
+        cs.ms_compact = lap();
     } catch (...) {
         free_leaves(&out, ctx->stream);
         throw;
     }
-    lap();
+    lose.done = true;
     finish(out, std::move(tiles));
+    a->topo = std::move(compacted);
     cs.ms_memory += lap();
-    a->topo = ta.compact(new_index);
-    cs.ms_compact = lap();
     cs.n_out = n_out;
     cs.ms_wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_wall).count();
     ctx->last_csg = cs;

@@ -210,6 +210,12 @@ void bs_volume_free(bs_volume* v);
  * once): for callers that need the device memory back for other work. */
 void bs_release_cached_memory(void);
 
+/* For tests of what a call leaves behind when device memory runs out: of the
+ * calling thread's requests for device memory from now on, numbers first (1 is
+ * the next one) to first + count - 1 fail; first 0 refuses none.  Returns the
+ * thread's requests since the last call of this function. */
+uint64_t bs_refuse_allocations(uint64_t first, uint64_t count);
+
 /* Volume::voxel_size and sizes. */
 bs_status bs_volume_info_get(const bs_volume* v, bs_volume_info* out);
 

@@ -1,0 +1,90 @@
+"""Calls that run out of device memory part-way: each request for memory of a
+call is refused in turn (bs_refuse_allocations) on a context without scratch,
+and the volumes it was given must then be what they were."""
+import contextlib
+
+import numpy as np
+import pytest
+
+import baby_shark_amd as bs
+from baby_shark_amd import _lib
+
+pytestmark = pytest.mark.gpu
+H = 0.05
+AX = np.arange(-60, 60, 9, dtype=np.int32)
+Q = np.stack(np.meshgrid(AX, AX, AX, indexing="ij"), -1).reshape(-1, 3)
+
+
+@contextlib.contextmanager
+def refusing(first, count=1 << 40):
+    _lib.load().bs_refuse_allocations(first, count)
+    try:
+        yield
+    finally:
+        _lib.load().bs_refuse_allocations(0, 0)
+
+
+def same_volume(g, r):
+    for f in ("origins", "masks", "tile_origins", "tile_sizes"):
+        assert np.array_equal(getattr(g, f), getattr(r, f)), f
+    for f in ("values", "tile_values"):
+        assert np.array_equal(getattr(g, f).view(np.uint32), getattr(r, f).view(np.uint32)), f
+
+
+def operands(ctx, gap):
+    """Two volumes with tiles and upper levels; with a gap between two root
+    blocks on a z line, so that those are in the host's form."""
+    B = bs.VolumeBuilder(ctx, H)
+
+    def far():
+        return bs.volume_from_voxels(np.array([[0, 0, 8192 + 40], [1, 0, 8192 + 40]], np.int32),
+                                     np.array([-0.02, 0.03], np.float32), H, ctx)
+    a = B.sphere(2.0, (0.1, -0.2, 0.3)).union(B.sphere(0.9, (-0.4, 0.0, 0.2)))
+    b = B.sphere(1.5, (1.6, 0.2, 0.0)).union(B.sphere(0.6, (1.5, 0.1, 0.0)))
+    return (a.union(far()), b.union(far())) if gap else (a, b)
+
+
+def on_context(v, ctx):
+    c = v.clone()
+    c._ctx = ctx
+    return c
+
+
+def mesh(ctx, v):
+    return bs.MarchingCubesMesher(ctx).with_voxel_size(H).mesh(v).view(np.uint32)
+
+
+@pytest.mark.parametrize("op", ["union", "subtract", "intersect"])
+@pytest.mark.parametrize("gap", [False, True])
+def test_csg_that_fails_keeps_its_operands(gpu_ctx, op, gap):
+    a0, b0 = operands(gpu_ctx, gap)
+    soups = mesh(gpu_ctx, a0.clone()), mesh(gpu_ctx, b0.clone())
+    r = getattr(a0.clone(), op)(b0.clone())
+    want, signs = r.export(), r.signs_at(Q)
+    failed = lost = 0
+    for first in range(1, 100):
+        print(f"  {op} gap={gap} refused from request {first}", flush=True)
+        ctx = bs.Context(0)
+        a, b = on_context(a0, ctx), on_context(b0, ctx)
+        try:
+            with refusing(first):
+                r = getattr(a, op)(b)
+            break
+        except bs.BSError:
+            failed += 1
+        try:
+            got = mesh(ctx, a), mesh(ctx, b)
+            assert np.array_equal(got[0], soups[0]) and np.array_equal(got[1], soups[1])
+            r = getattr(a, op)(b)
+        except bs.BSError as e:  # only where the plan was made in the host's form
+            assert gap and "upper levels" in str(e)
+            assert np.array_equal(a.export().origins, a0.export().origins)
+            lost += 1
+            continue
+        same_volume(r.export(), want)
+        assert np.array_equal(r.signs_at(Q), signs)
+    else:
+        pytest.fail("still refused")
+    assert failed > 2 and bool(lost) == gap
+    same_volume(r.export(), want)
+    assert np.array_equal(r.signs_at(Q), signs)
