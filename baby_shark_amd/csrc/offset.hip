@@ -803,16 +803,17 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
                    "offset: an active tile lies within the band; the reference panics (fast_sweep.rs:100)");
     if (stats) *stats = bs_offset_stats{};
     uint64_t capacity = std::max<uint64_t>(4 * vol->n_leaves + 4096, 8192);
-    bs_volume out;
+    // the result's leaf arrays, given back unless they have moved into the volume
+    struct Result {
+        hipStream_t st;
+        bs_volume v;
+        ~Result() { free_leaves(&v, st); }
+    } result{ctx->stream, {}};
+    bs_volume& out = result.v;
     out.device = vol->device;
     OffsetResult r;
     for (int attempt = 0;; ++attempt) {
-        try {
-            r = offset_attempt(ctx, vol, distance, capacity, (ctx->paths & BS_PATH_FORCE_HASH) != 0, out, stats);
-        } catch (...) {
-            free_leaves(&out, ctx->stream);
-            throw;
-        }
+        r = offset_attempt(ctx, vol, distance, capacity, (ctx->paths & BS_PATH_FORCE_HASH) != 0, out, stats);
         if (!r.retry) break;
         BS_REQUIRE(attempt < 6, BS_ERR_INTERNAL, "offset: leaf pool kept overflowing");
         capacity *= 4;
@@ -837,8 +838,9 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
             t2 = ensure_topology(ctx, vol).after_offset(keep, out_origins, two_h);
         }
     }
+    const uint64_t n_out = out.n_leaves;
     free_leaves(vol);
-    vol->n_leaves = out.n_leaves;
+    vol->n_leaves = n_out;
     vol->origins = out.origins;
     vol->masks = out.masks;
     vol->values = out.values;
@@ -850,7 +852,7 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
     vol->tree = std::move(d2);
     ev.stop(ctx->stream);
     if (stats) {
-        stats->n_out = out.n_leaves;
+        stats->n_out = n_out;
         stats->ms_device = ev.ms();
         stats->ms_wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_wall).count();
     }

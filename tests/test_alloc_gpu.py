@@ -31,14 +31,14 @@ def same_volume(g, r):
         assert np.array_equal(getattr(g, f).view(np.uint32), getattr(r, f).view(np.uint32)), f
 
 
-def operands(ctx, gap):
+def operands(ctx, gap, h=H):
     """Two volumes with tiles and upper levels; with a gap between two root
     blocks on a z line, so that those are in the host's form."""
-    B = bs.VolumeBuilder(ctx, H)
+    B = bs.VolumeBuilder(ctx, h)
 
     def far():
         return bs.volume_from_voxels(np.array([[0, 0, 8192 + 40], [1, 0, 8192 + 40]], np.int32),
-                                     np.array([-0.02, 0.03], np.float32), H, ctx)
+                                     np.array([-0.02, 0.03], np.float32), h, ctx)
     a = B.sphere(2.0, (0.1, -0.2, 0.3)).union(B.sphere(0.9, (-0.4, 0.0, 0.2)))
     b = B.sphere(1.5, (1.6, 0.2, 0.0)).union(B.sphere(0.6, (1.5, 0.1, 0.0)))
     return (a.union(far()), b.union(far())) if gap else (a, b)
@@ -88,3 +88,51 @@ def test_csg_that_fails_keeps_its_operands(gpu_ctx, op, gap):
     assert failed > 2 and bool(lost) == gap
     same_volume(r.export(), want)
     assert np.array_equal(r.signs_at(Q), signs)
+
+
+@pytest.mark.parametrize("gap", [False, True])
+def test_offset_that_fails_keeps_its_volume_and_no_memory(gpu_ctx, gap):
+    import torch
+    h = H / 2
+    v0, _ = operands(gpu_ctx, gap, h)
+    v0 = v0.subtract(bs.VolumeBuilder(gpu_ctx, h).sphere(0.9, (0.3, 0.0, 0.2)))
+    before = v0.export()
+    r = v0.clone().offset(1.0)
+    want, signs = r.export(), r.signs_at(Q)
+    result_bytes = 2128 * want.origins.shape[0]
+    assert result_bytes > 8 << 20
+    r.free()
+
+    def free_bytes():
+        bs.release_cached_memory()
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    for _ in range(5):  # the runtime's own memory for kernels, streams and their queues
+        ctx = bs.Context(0)
+        on_context(v0, ctx).offset(1.0).free()
+        ctx.close()
+    start = free_bytes()
+    failed = 0
+    for first in range(1, 100):
+        print(f"  gap={gap} refused from request {first}", flush=True)
+        ctx = bs.Context(0)
+        v = on_context(v0, ctx)
+        try:
+            with refusing(first):
+                v.offset(1.0)
+            break
+        except bs.BSError:
+            failed += 1
+        same_volume(v.export(), before)
+        if failed % 4 == 0:
+            r = v.offset(1.0)
+            same_volume(r.export(), want)
+            assert np.array_equal(r.signs_at(Q), signs)
+            r.free()
+        v.free()
+        ctx.close()
+        assert start - free_bytes() < result_bytes // 2
+    else:
+        pytest.fail("still refused")
+    assert failed > 10
