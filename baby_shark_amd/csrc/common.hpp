@@ -68,7 +68,6 @@ enum ScratchSlot : int {
     S_PLOC_BOX, S_PLOC_INFO, S_PLOC_C0, S_PLOC_C1, S_PLOC_NN, S_PLOC_KEEP, S_PLOC_POS, S_PLOC_RING,
     S_TD_PRIMS, S_TD_FR, S_TD_BINS, S_TD_TASKS, S_TD_TCNT, S_TD_SPLIT, S_TD_SMALL, S_TD_HIST,
     S_LEAF_MKEY, S_LEAF_MKEY_S, S_LEAF_IDS, S_LEAF_PERM, S_WN_CHUNKS, S_WN_LIST, S_WN_COEF,
-    S_OFF_MASKS, S_OFF_KEEP, S_OFF_DST, S_OFF_ORIGINS, S_OFF_FROZEN, S_OFF_WORK, S_OFF_SRC, S_OFF_ORDER,
     S_OFF_PLANES,
     S_TREE_MARK, S_TREE_TILES, S_TREE_TILE_VAL, S_TREE_FLAGS, S_TREE_PAIRS, S_TREE_FLIPS, S_TREE_PARTNER, S_TREE_ZERO,
     S_TREE_RANK, S_TREE_ROOTS, S_TREE_NODES, S_TREE_ITEMS, S_TREE_REFS, S_TREE_NODE_N, S_TREE_PLACE, S_MC_TILE_VAL,

@@ -552,15 +552,24 @@ void exclusive_scan_u32(bs_ctx* ctx, const uint32_t* in, uint32_t* out, uint64_t
     BS_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, in, out, (int)n, ctx->stream));
 }
 
-// The large device buffers of one offset attempt, back to the pool on every
-// exit path once the stream is done with them.
+// Device buffers of an offset, back to the pool on every exit path once the
+// stream is done with them.  All that grows with the volume or the leaf pool is
+// here (2.2 KB per pool leaf), so that nothing of that size stays with the
+// context.
 struct OffsetBuffers {
     hipStream_t st;
     std::vector<void*> ptrs;
-    explicit OffsetBuffers(hipStream_t s) : st(s) { ptrs.reserve(4); }
+    explicit OffsetBuffers(hipStream_t s) : st(s) { ptrs.reserve(8); }
     template <class T> T* alloc(uint64_t count) {
         ptrs.push_back(alloc_block(std::max<uint64_t>(count, 1) * sizeof(T)));
         return static_cast<T*>(ptrs.back());
+    }
+    // several arrays in one block: f lays them out from p on (see take), first from null to find the size
+    template <class F> void carve(F&& f) {
+        uint8_t* p = nullptr;
+        f(p);
+        p = alloc<uint8_t>((uint64_t)(uintptr_t)p);
+        f(p);
     }
     ~OffsetBuffers() {
         const bool done = hipStreamSynchronize(st) == hipSuccess;
@@ -574,16 +583,27 @@ Topology& ensure_topology(bs_ctx* ctx, bs_volume* v);
 
 namespace {
 
+// An array at p on a 256-byte border; p moves past it.
+template <class T> void take(uint8_t*& p, T*& array, uint64_t count) {
+    array = reinterpret_cast<T*>(p);
+    p += (count * sizeof(T) + 255) / 256 * 256;
+}
+
+// What remove_if leaves of the volume, the same for every attempt.
+struct KeptLeaves {
+    uint64_t* masks = nullptr;  // per input leaf: 8 words
+    uint32_t *keep = nullptr, *dst = nullptr;
+};
+
 struct OffsetResult {
     uint64_t n_out = 0;
-    const uint32_t* keep_dev = nullptr;  // per input leaf (context scratch)
     bool retry = false;
 };
 
 // One attempt with a pool of `capacity` leaves; retry = the pool or the leaf
 // map was too small (nothing of `vol` was modified).
 OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_t capacity, bool force_hash,
-                            bs_volume& out, bs_offset_stats* stats) {
+                            const KeptLeaves& kept, bs_volume& out, bs_offset_stats* stats) {
     hipStream_t st = ctx->stream;
     OffsetResult res;
     const uint64_t n = vol->n_leaves;
@@ -599,9 +619,8 @@ OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_
     Scratch& S = ctx->scratch;
     OffsetBuffers B(st);
     // remove_if and compaction of the surviving leaves
-    uint64_t* rm_masks = S.as<uint64_t>(S_OFF_MASKS, 8 * n);
-    uint32_t* keep = S.as<uint32_t>(S_OFF_KEEP, n);
-    uint32_t* dst = S.as<uint32_t>(S_OFF_DST, n);
+    uint64_t* rm_masks = kept.masks;
+    uint32_t *keep = kept.keep, *dst = kept.dst;
     int32_t* dbox = S.as<int32_t>(S_LEAF_BOX, 6);
     k_remove_if<<<div_up(n, 4), 256, 0, st>>>(n, vol->masks, vol->values, two_h, rm_masks, keep);
     BS_HIP(hipGetLastError());
@@ -611,7 +630,6 @@ OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_
     k_leaf_box<<<(unsigned)std::min<uint64_t>(div_up(n, 256), 256), 256, 0, st>>>(
         n, reinterpret_cast<const int4*>(vol->origins), dbox, keep);
     BS_HIP(hipGetLastError());
-    res.keep_dev = keep;
     uint32_t* first = static_cast<uint32_t*>(pinned_words(ctx, 8));
     BS_HIP(hipMemcpyAsync(first, dst + n - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     BS_HIP(hipMemcpyAsync(first + 1, keep + n - 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
@@ -657,9 +675,15 @@ OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_
     SweepArgs a{};
     a.map = map;
     a.capacity = (uint32_t)capacity;
-    a.origins = S.as<int4>(S_OFF_ORIGINS, capacity);
-    a.frozen = S.as<uint64_t>(S_OFF_FROZEN, 8 * capacity);
-    a.work = S.as<uint32_t>(S_OFF_WORK, capacity);
+    int4* order = nullptr;
+    uint32_t* src = nullptr;
+    B.carve([&](uint8_t*& p) {
+        take(p, a.origins, capacity);
+        take(p, a.frozen, 8 * capacity);
+        take(p, a.work, capacity);
+        take(p, order, capacity + 1);  // a plane past the last bucket reads an entry that it does not use
+        take(p, src, n_keep);
+    });
     a.words = B.alloc<uint32_t>(512 * capacity);
     a.neg = neg;
     // the words' units (see NONE): scaling up by a power of two is exact, and nothing overflows with h within
@@ -690,12 +714,9 @@ OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_
     OffsetState cur{};
     auto read_state = [&] { std::memcpy(&cur, back + n_planes + 1, sizeof(cur)); };
     BS_HIP(hipMemsetAsync(dstate, 0, sizeof(OffsetState), st));
-    uint32_t* src = S.as<uint32_t>(S_OFF_SRC, n_keep);
     k_pool_init<<<div_up(n, 4), 256, 0, st>>>(n, keep, dst, vol->origins, rm_masks, vol->values, scale, a, src, dstate);
     BS_HIP(hipGetLastError());
 
-    // one entry more than leaves: a plane past the last bucket reads one that it does not use
-    int4* order = S.as<int4>(S_OFF_ORDER, capacity + 1);
     uint64_t planes_total = 0, swept = 0;
     uint32_t pool = (uint32_t)n_keep;  // pool size at the start of the sweep
     auto check = [&](int s) {
@@ -761,10 +782,14 @@ OffsetResult offset_attempt(bs_ctx* ctx, bs_volume* vol, float distance, uint64_
     }
 
     // empty leaves go, the rest sorted by origin, shifted by -D
-    uint64_t* keys = S.as<uint64_t>(S_KEYS, n_pool);
-    uint64_t* keys_s = S.as<uint64_t>(S_KEYS_SORTED, n_pool);
-    uint32_t* idx = S.as<uint32_t>(S_IDX, n_pool);
-    uint32_t* idx_s = S.as<uint32_t>(S_IDX_SORTED, n_pool);
+    uint64_t *keys = nullptr, *keys_s = nullptr;
+    uint32_t *idx = nullptr, *idx_s = nullptr;
+    B.carve([&](uint8_t*& p) {
+        take(p, keys, n_pool);
+        take(p, keys_s, n_pool);
+        take(p, idx, n_pool);
+        take(p, idx_s, n_pool);
+    });
     k_final_keys<<<div_up(n_pool, 256), 256, 0, st>>>(n_pool, a.origins, a.work, keys, idx, dstate);
     BS_HIP(hipGetLastError());
     BS_HIP(hipMemcpyAsync(back + n_planes + 1, dstate, sizeof(cur), hipMemcpyDeviceToHost, st));
@@ -811,9 +836,16 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
     } result{ctx->stream, {}};
     bs_volume& out = result.v;
     out.device = vol->device;
+    OffsetBuffers kept_block(ctx->stream);
+    KeptLeaves kept;
+    kept_block.carve([&](uint8_t*& p) {
+        take(p, kept.masks, 8 * vol->n_leaves);
+        take(p, kept.keep, vol->n_leaves);
+        take(p, kept.dst, vol->n_leaves);
+    });
     OffsetResult r;
     for (int attempt = 0;; ++attempt) {
-        r = offset_attempt(ctx, vol, distance, capacity, (ctx->paths & BS_PATH_FORCE_HASH) != 0, out, stats);
+        r = offset_attempt(ctx, vol, distance, capacity, (ctx->paths & BS_PATH_FORCE_HASH) != 0, kept, out, stats);
         if (!r.retry) break;
         BS_REQUIRE(attempt < 6, BS_ERR_INTERNAL, "offset: leaf pool kept overflowing");
         capacity *= 4;
@@ -824,13 +856,13 @@ void volume_offset(bs_ctx* ctx, bs_volume* vol, float distance, bs_offset_stats*
     std::unique_ptr<DeviceTree> d2;
     if (vol->topo || vol->tree || !vol->tiles.empty()) {
         if (const DeviceTree* d = ensure_tree(ctx, vol))
-            d2 = tree_after_offset(ctx, *d, reinterpret_cast<const int4*>(vol->origins), r.keep_dev, vol->n_leaves,
+            d2 = tree_after_offset(ctx, *d, reinterpret_cast<const int4*>(vol->origins), kept.keep, vol->n_leaves,
                                    reinterpret_cast<const int4*>(out.origins), out.n_leaves);
         if (!d2) {
             std::vector<uint32_t> keep(vol->n_leaves);
             std::vector<int32_t> o4(4 * out.n_leaves);
             if (!keep.empty())
-                BS_HIP(hipMemcpy(keep.data(), r.keep_dev, sizeof(uint32_t) * keep.size(), hipMemcpyDeviceToHost));
+                BS_HIP(hipMemcpy(keep.data(), kept.keep, sizeof(uint32_t) * keep.size(), hipMemcpyDeviceToHost));
             if (!o4.empty())
                 BS_HIP(hipMemcpy(o4.data(), out.origins, sizeof(int32_t) * o4.size(), hipMemcpyDeviceToHost));
             std::vector<std::array<int32_t, 3>> out_origins(out.n_leaves);

@@ -44,6 +44,13 @@ def operands(ctx, gap, h=H):
     return (a.union(far()), b.union(far())) if gap else (a, b)
 
 
+def free_bytes():
+    import torch
+    bs.release_cached_memory()
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
 def on_context(v, ctx):
     c = v.clone()
     c._ctx = ctx
@@ -92,7 +99,6 @@ def test_csg_that_fails_keeps_its_operands(gpu_ctx, op, gap):
 
 @pytest.mark.parametrize("gap", [False, True])
 def test_offset_that_fails_keeps_its_volume_and_no_memory(gpu_ctx, gap):
-    import torch
     h = H / 2
     v0, _ = operands(gpu_ctx, gap, h)
     v0 = v0.subtract(bs.VolumeBuilder(gpu_ctx, h).sphere(0.9, (0.3, 0.0, 0.2)))
@@ -102,11 +108,6 @@ def test_offset_that_fails_keeps_its_volume_and_no_memory(gpu_ctx, gap):
     result_bytes = 2128 * want.origins.shape[0]
     assert result_bytes > 8 << 20
     r.free()
-
-    def free_bytes():
-        bs.release_cached_memory()
-        torch.cuda.synchronize()
-        return torch.cuda.mem_get_info()[0]
 
     for _ in range(5):  # the runtime's own memory for kernels, streams and their queues
         ctx = bs.Context(0)
@@ -136,3 +137,25 @@ def test_offset_that_fails_keeps_its_volume_and_no_memory(gpu_ctx, gap):
     else:
         pytest.fail("still refused")
     assert failed > 10
+
+
+def test_offset_leaves_no_arrays_with_its_context(gpu_ctx):
+    """After an offset and release_cached_memory a context holds nothing that
+    grew with the leaf pool but the sort's scratch (12 B per pool leaf and side
+    buffers): at most 48 B, where the pool's own arrays are 100 B beside the
+    values."""
+    v0 = bs.VolumeBuilder(gpu_ctx, H / 10).sphere(2.0, (0.1, -0.2, 0.3))
+    contexts = []
+
+    def offset():
+        contexts.append(bs.Context(0))
+        on_context(v0, contexts[-1]).offset(H / 5).free()
+        return contexts[-1].last_offset_stats()["n_capacity"]
+
+    for _ in range(5):  # the runtime's own memory for kernels, streams and their queues
+        offset()
+        contexts[-1].close()
+    start = free_bytes()
+    pool = offset()
+    assert start - free_bytes() < 48 * pool
+    contexts[-1].close()
