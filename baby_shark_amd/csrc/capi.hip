@@ -303,8 +303,11 @@ bs_status bs_volume_clone(const bs_volume* v, bs_volume** out) {
         c->tiles = v->tiles;
         c->tree_lost = v->tree_lost;
         try {
-            if (v->topo) c->topo = v->topo->clone();
-            if (v->tree) c->tree = clone_tree(*v->tree);
+            {
+                std::lock_guard<std::mutex> lk(v->forms);
+                if (v->tree) c->tree = clone_tree(*v->tree);
+                else if (v->topo) c->topo = v->topo->clone();
+            }
             if (v->n_leaves) {
                 alloc_leaves(c, v->n_leaves);
                 BS_HIP(hipMemcpyAsync(c->origins, v->origins, sizeof(int32_t) * 4 * v->n_leaves, hipMemcpyDeviceToDevice));

@@ -10,6 +10,8 @@
 #include <memory>
 #include <vector>
 
+#include <mutex>
+
 #include "../../include/bs_voxel.h"
 #include "topology.hpp"
 #include "tree.hpp"
@@ -138,9 +140,13 @@ struct bs_volume {
     uint64_t* masks = nullptr;   // device, n_leaves*8
     float* values = nullptr;     // device, n_leaves*512
     std::vector<bs::TileRec> tiles;           // active internal tiles (host, few)
-    // upper levels, in one form or the other; built from the leaves and tiles when absent
+    // upper levels, in the host's form, the device's or both (the same tree); made from each other, or from the
+    // leaves and tiles, when a call needs a form that is absent.  Calls that only read the volume add a form, under
+    // `forms`, and never take one away, so several threads may read one volume; a call that changes the tree leaves
+    // only the forms that it changed.
     std::unique_ptr<bs::Topology> topo;
     std::unique_ptr<bs::DeviceTree> tree;
+    mutable std::mutex forms;
     // a call that works on the host's form in place failed part-way: the leaves are whole, but what the
     // upper levels held beyond them is lost
     bool tree_lost = false;

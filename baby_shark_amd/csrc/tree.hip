@@ -155,8 +155,17 @@ __global__ void k_put_tiles(uint32_t n, const int4* __restrict__ tiles, const fl
     }
 }
 
+bool root_gap(const Topology::Key& a, const Topology::Key& b) {  // of two keys next to each other in order
+    return a[0] == b[0] && a[1] == b[1] && b[2] != a[2] + SPAN1;
+}
+bool has_root_gap(const std::map<Topology::Key, int32_t>& root) {
+    return std::adjacent_find(root.begin(), root.end(), [](const auto& a, const auto& b) {
+               return root_gap(a.first, b.first);
+           }) != root.end();
+}
+
 std::unique_ptr<DeviceTree> tree_from_leaves(bs_ctx* ctx, const int4* origins, uint64_t n,
-                                             const std::vector<TileRec>& tiles) {
+                                             const std::vector<TileRec>& tiles, bool no_gap = false) {
     hipStream_t st = ctx->stream;
     Scratch& S = ctx->scratch;
     if (!n && tiles.empty()) return new_tree(ctx, 0, 0);
@@ -213,6 +222,7 @@ std::unique_ptr<DeviceTree> tree_from_leaves(bs_ctx* ctx, const int4* origins, u
         keys.push_back({((int32_t)(r / g.NZ / g.NY) + g.X0) * SPAN1, ((int32_t)(r / g.NZ % g.NY) + g.Y0) * SPAN1,
                         ((int32_t)(r % g.NZ) + g.Z0) * SPAN1});
     }
+    if (no_gap && std::adjacent_find(keys.begin(), keys.end(), root_gap) != keys.end()) return nullptr;
     auto t = new_tree(ctx, (uint32_t)keys.size(), n2);
     std::vector<int4> org1;
     for (size_t i = 0; i < keys.size(); ++i) {
@@ -702,16 +712,22 @@ void require_tree(const bs_volume* v) {
     BS_REQUIRE(!v->tree_lost, BS_ERR_INTERNAL, "an earlier operation that failed left this volume without its upper levels");
 }
 
-DeviceTree* ensure_tree(bs_ctx* ctx, bs_volume* v) {
+bool known_root_gap(const bs_volume* v) {
+    std::lock_guard<std::mutex> lk(v->forms);
+    return v->tree ? has_root_gap(v->tree->root) : v->topo && has_root_gap(v->topo->root);
+}
+
+DeviceTree* ensure_tree(bs_ctx* ctx, bs_volume* v, bool no_gap) {
     require_tree(v);
+    if (no_gap && known_root_gap(v)) return nullptr;
+    std::lock_guard<std::mutex> lk(v->forms);
     if (v->tree) return v->tree.get();
     std::unique_ptr<DeviceTree> t =
         v->topo ? upload_tree(ctx, *v->topo)
-                : tree_from_leaves(ctx, reinterpret_cast<const int4*>(v->origins), v->n_leaves, v->tiles);
+                : tree_from_leaves(ctx, reinterpret_cast<const int4*>(v->origins), v->n_leaves, v->tiles, no_gap);
     if (!t) return nullptr;
     t->pending = nullptr;  // both return with the stream's work done
     v->tree = std::move(t);
-    v->topo.reset();
     return v->tree.get();
 }
 
@@ -756,15 +772,6 @@ std::unique_ptr<Topology> download_tree(bs_ctx* ctx, const bs_volume* v) {
     LeafVec& recs = t->leaves.seg[0];
     for (uint64_t i = 0; i < v->n_leaves; ++i) recs[i] = leaf_ref(org[i].x, org[i].y, org[i].z, (int32_t)i);
     return t;
-}
-
-bool tree_has_root_gap(const DeviceTree& t) {
-    const Topology::Key* last = nullptr;
-    for (const auto& kv : t.root) {
-        if (last && (*last)[0] == kv.first[0] && (*last)[1] == kv.first[1] && kv.first[2] != (*last)[2] + SPAN1) return true;
-        last = &kv.first;
-    }
-    return false;
 }
 
 void tree_flood_fill(bs_ctx* ctx, const DeviceTree& t, const uint8_t* leaf_flags) {

@@ -43,18 +43,20 @@ struct DeviceTree {
 };
 
 // The volume's tree on the device, made from its leaves (and tiles) or from its
-// Topology, which it replaces; nullptr when it does not fit: more than 2^24
-// 128^3 blocks in the box of the leaves, 256 root blocks in it or 2^16 nodes.
-DeviceTree* ensure_tree(bs_ctx* ctx, bs_volume* v);
+// Topology; nullptr when it does not fit: more than 2^24 128^3 blocks in the box
+// of the leaves, 256 root blocks in it or 2^16 nodes.  With `no_gap` nullptr also,
+// and nothing is made, where the root's flood fill may close a gap on a z line
+// between two root entries (root_node/flood_fill.rs:14-41), which is left to
+// Topology.
+DeviceTree* ensure_tree(bs_ctx* ctx, bs_volume* v, bool no_gap = false);
+// A volume that has a form of its tree, with such a gap in its root.
+bool known_root_gap(const bs_volume* v);
 // Throws for a volume whose upper levels a failed call lost.
 void require_tree(const bs_volume* v);
 std::unique_ptr<DeviceTree> clone_tree(const DeviceTree& t);
 // The host's form of a volume's device tree.
 std::unique_ptr<Topology> download_tree(bs_ctx* ctx, const bs_volume* v);
 
-// Two root entries on one z line with a gap between them: the root's flood fill
-// may close it (root_node/flood_fill.rs:14-41), which is left to Topology.
-bool tree_has_root_gap(const DeviceTree& t);
 // Flood fill of both internal levels (internal_node/flood_fill.rs:17-75);
 // leaf_flags: bit 0 first value negative, bit 1 last value negative.
 void tree_flood_fill(bs_ctx* ctx, const DeviceTree& t, const uint8_t* leaf_flags);

@@ -218,10 +218,10 @@ static std::vector<std::array<int32_t, 3>> leaf_origins(bs_ctx* ctx, const bs_vo
 
 Topology& ensure_topology(bs_ctx* ctx, bs_volume* v) {
     require_tree(v);
+    std::lock_guard<std::mutex> lk(v->forms);
     if (v->topo) return *v->topo;
     if (v->tree) {
         v->topo = download_tree(ctx, v);
-        v->tree.reset();
         return *v->topo;
     }
     v->topo = Topology::from_leaves(leaf_origins(ctx, v), v->tiles);
@@ -597,12 +597,19 @@ void apply_flags(Topology& t, const std::vector<uint8_t>& flags) {
 
 // FloodFill::flood_fill of a whole grid (root_node/flood_fill.rs:8-42).
 void volume_flood_fill(bs_ctx* ctx, bs_volume* v) {
-    Topology& t = ensure_topology(ctx, v);
-    std::vector<uint8_t> flags;
-    launch_leaf_flood_fill(ctx, v, S_FLAGS_A, flags);
+    // each form that the volume has is filled; a gap in the root is closed in the host's alone
+    const bool on_device = v->tree && ensure_tree(ctx, v, true);
+    if (!on_device) ensure_topology(ctx, v);
+    const uint8_t* d_flags = launch_leaf_flood_fill(ctx, v, S_FLAGS_A);
+    std::vector<uint8_t> flags(v->n_leaves);
+    if (on_device) tree_flood_fill(ctx, *v->tree, d_flags);
+    if (v->topo && v->n_leaves)
+        BS_HIP(hipMemcpyAsync(flags.data(), d_flags, v->n_leaves, hipMemcpyDeviceToHost, ctx->stream));
     BS_HIP(hipStreamSynchronize(ctx->stream));
-    apply_flags(t, flags);
-    t.flood_fill_upper();
+    if (!on_device) v->tree.reset();
+    if (!v->topo) return;
+    apply_flags(*v->topo, flags);
+    v->topo->flood_fill_upper();
 }
 
 // sign_at for a batch of voxel indices (root_node/flood_fill.rs:56-63): tile
@@ -678,9 +685,11 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
     };
     // Both trees on the device, where they fit and the root's flood fill has no
     // gap to close; the host's form of the tree otherwise.
-    DeviceTree* da = ensure_tree(ctx, a);
-    DeviceTree* db = da ? ensure_tree(ctx, b) : nullptr;
-    if (da && db && !tree_has_root_gap(*da) && !tree_has_root_gap(*db)) {
+    DeviceTree* da = known_root_gap(b) ? nullptr : ensure_tree(ctx, a, true);
+    DeviceTree* db = da ? ensure_tree(ctx, b, true) : nullptr;
+    if (da && db) {
+        a->topo.reset();  // the device's form is flood filled
+        b->topo.reset();
         cs.ms_topology = lap();
         EventPair ev_flood, ev_asm;
         bs_volume out;
@@ -723,6 +732,8 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
         return;
     }
     ensure_topologies(ctx, a, b);
+    a->tree.reset();  // the host's form is flood filled
+    b->tree.reset();
     Topology& ta = *a->topo;
     Topology& tb = *b->topo;
     cs.ms_topology = lap();
@@ -1022,6 +1033,7 @@ void volume_densify_tiles(bs_ctx* ctx, bs_volume* v) {
     out.values = nullptr;
     v->tiles.clear();
     v->topo = t.compact(new_index);
+    v->tree.reset();
 }
 
 // The index box of Volume::from_fn (volume/mod.rs:49-51): floor(min / h) ..=
