@@ -21,7 +21,8 @@ namespace bs {
 // ---------------------------------------------------------------- errors
 struct Error : std::runtime_error {
     bs_status status;
-    Error(bs_status s, const std::string& m) : std::runtime_error(m), status(s) {}
+    bool out_of_memory;  // of the device
+    Error(bs_status s, const std::string& m, bool oom = false) : std::runtime_error(m), status(s), out_of_memory(oom) {}
 };
 
 void set_last_error(const std::string& msg);
@@ -31,7 +32,8 @@ void set_last_error(const std::string& msg);
         hipError_t e_ = (call);                                                                        \
         if (e_ != hipSuccess)                                                                          \
             throw ::bs::Error(BS_ERR_HIP, std::string(#call) + ": " + hipGetErrorString(e_) + " at " + \
-                                              __FILE__ + ":" + std::to_string(__LINE__));              \
+                                              __FILE__ + ":" + std::to_string(__LINE__),               \
+                              e_ == hipErrorOutOfMemory);                                              \
     } while (0)
 
 #define BS_REQUIRE(cond, status, msg)                          \

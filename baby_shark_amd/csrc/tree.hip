@@ -229,7 +229,8 @@ std::unique_ptr<DeviceTree> tree_from_leaves(bs_ctx* ctx, const int4* origins, u
         t->root[keys[i]] = (int32_t)i;
         org1.push_back(make_int4(keys[i][0], keys[i][1], keys[i][2], 0));
     }
-    // kinds, tile values and children of all slots: empty, 0, -1 (never followed)
+    // kinds, tile values and children of all slots: empty, 0, 0 (a child of a slot that is no branch is never
+    // followed)
     BS_HIP(hipMemsetAsync(t->block, 0, (uint64_t)((uint8_t*)t->v.org2 - (uint8_t*)t->block), st));
     BS_HIP(hipMemcpyAsync(root_id, ids, sizeof(uint32_t) * g.N, hipMemcpyHostToDevice, st));
     BS_HIP(hipMemcpyAsync(t->v.org1, org1.data(), sizeof(int4) * org1.size(), hipMemcpyHostToDevice, st));
@@ -722,9 +723,14 @@ DeviceTree* ensure_tree(bs_ctx* ctx, bs_volume* v, bool no_gap) {
     if (no_gap && known_root_gap(v)) return nullptr;
     std::lock_guard<std::mutex> lk(v->forms);
     if (v->tree) return v->tree.get();
-    std::unique_ptr<DeviceTree> t =
-        v->topo ? upload_tree(ctx, *v->topo)
-                : tree_from_leaves(ctx, reinterpret_cast<const int4*>(v->origins), v->n_leaves, v->tiles, no_gap);
+    std::unique_ptr<DeviceTree> t;
+    try {
+        t = v->topo ? upload_tree(ctx, *v->topo)
+                    : tree_from_leaves(ctx, reinterpret_cast<const int4*>(v->origins), v->n_leaves, v->tiles, no_gap);
+    } catch (const Error& e) {
+        if (!e.out_of_memory) throw;
+        (void)hipStreamSynchronize(ctx->stream);
+    }
     if (!t) return nullptr;
     t->pending = nullptr;  // both return with the stream's work done
     v->tree = std::move(t);
@@ -781,8 +787,8 @@ void tree_flood_fill(bs_ctx* ctx, const DeviceTree& t, const uint8_t* leaf_flags
     BS_HIP(hipGetLastError());
 }
 
-TreeCsg tree_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, const TreeOperand& la, const TreeOperand& lb,
-                 CsgOp op) {
+static void plan_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, const TreeOperand& la, const TreeOperand& lb,
+                     CsgOp op, TreeCsg& r) {
     hipStream_t st = ctx->stream;
     Scratch& S = ctx->scratch;
     // the root's rules (root_node/csg.rs:9-54): nodes that both hold are combined, the others stay or move in
@@ -798,10 +804,10 @@ TreeCsg tree_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, const Tr
             if (!a.root.count(kv.first)) res[kv.first] = -1 - kv.second;
     std::vector<int32_t> nodes;
     for (const auto& kv : res) nodes.push_back(kv.second);
+    if (nodes.size() > MAX_ROOTS) return;
 
     // 40 MB per copy at 570 k leaves; b's slots are written by a subtraction alone (k_csg_flip).  Working in place
     // a subtraction of that size takes 3.40 ms instead of 3.45, a union of 1,400 leaves 0.54 instead of 0.55.
-    TreeCsg r;
     r.work_a = copy_slots(ctx, a);
     if (op == CSG_SUBTRACT) r.work_b = copy_slots(ctx, b);
     const TreeView av = r.work_a->v, bv = r.work_b ? r.work_b->v : b.v;
@@ -861,15 +867,16 @@ TreeCsg tree_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, const Tr
     BS_HIP(hipMemcpyAsync(back, w.counts, sizeof(CsgCounts), hipMemcpyDeviceToHost, st));
     BS_HIP(hipStreamSynchronize(st));
     const CsgCounts c = *back;
+    if (c.n2 > MAX_N2) return;
     r.n_out = c.out;
     r.n_paired = c.paired;
     r.refs = plan;
     r.origins = plan + leaves;
-    r.tree = new_tree(ctx, (uint32_t)nodes.size(), c.n2);
+    auto tree = new_tree(ctx, (uint32_t)nodes.size(), c.n2);
     int32_t i1 = 0;
-    for (const auto& kv : res) r.tree->root[kv.first] = i1++;
-    if (n_items) k_copy_nodes1<<<blocks(n_items), 256, 0, st>>>(av, bv, n_items, d_nodes, at, r.tree->v);
-    if (c.n2) k_copy_nodes2<<<c.n2, 256, 0, st>>>(av, bv, w.n_a, refs2, place, r.tree->v);
+    for (const auto& kv : res) tree->root[kv.first] = i1++;
+    if (n_items) k_copy_nodes1<<<blocks(n_items), 256, 0, st>>>(av, bv, n_items, d_nodes, at, tree->v);
+    if (c.n2) k_copy_nodes2<<<c.n2, 256, 0, st>>>(av, bv, w.n_a, refs2, place, tree->v);
     BS_HIP(hipGetLastError());
     if (c.tiles) {
         int4* tile_org = S.as<int4>(S_TREE_TILES, c.tiles);
@@ -879,29 +886,47 @@ TreeCsg tree_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, const Tr
         BS_HIP(hipGetLastError());
         r.tiles = read_tiles(ctx, tile_org, tile_val, c.tiles);
     }
+    r.tree = std::move(tree);
+}
+
+TreeCsg tree_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, const TreeOperand& la, const TreeOperand& lb,
+                 CsgOp op) {
+    TreeCsg r;
+    try {
+        plan_csg(ctx, a, b, la, lb, op, r);
+    } catch (const Error& e) {
+        if (!e.out_of_memory) throw;
+    }
     return r;
 }
 
 std::unique_ptr<DeviceTree> tree_after_offset(bs_ctx* ctx, const DeviceTree& old, const int4* old_origins,
                                               const uint32_t* keep, uint64_t n_old, const int4* origins, uint64_t n) {
     hipStream_t st = ctx->stream;
-    auto t = tree_from_leaves(ctx, origins, n, {});
-    if (!t) return nullptr;
-    std::vector<int2> match;
-    for (const auto& kv : t->root) {
-        const auto it = old.root.find(kv.first);
-        if (it != old.root.end()) match.push_back(make_int2(kv.second, it->second));
-    }
-    if (!match.empty() && n_old) {
-        const int2* d_match = upload(ctx, S_TREE_ROOTS, match);
-        uint32_t* kept = ctx->scratch.as<uint32_t>(S_TREE_ZERO, (uint64_t)old.v.n1 + old.v.n2);
-        uint32_t* kept2 = kept + old.v.n1;
-        BS_HIP(hipMemsetAsync(kept, 0, sizeof(uint32_t) * ((uint64_t)old.v.n1 + old.v.n2), st));
-        k_node_kept<<<blocks(n_old), 256, 0, st>>>(n_old, old_origins, keep, old.v, d_match, (uint32_t)match.size(), kept,
-                                                   kept2);
-        k_keep_tiles<<<(unsigned)match.size() * (N1_SLOTS / 256), 256, 0, st>>>(old.v, d_match, kept, kept2, t->v);
-        BS_HIP(hipGetLastError());
-        BS_HIP(hipStreamSynchronize(st));
+    std::unique_ptr<DeviceTree> t;
+    try {
+        t = tree_from_leaves(ctx, origins, n, {});
+        if (!t) return nullptr;
+        std::vector<int2> match;
+        for (const auto& kv : t->root) {
+            const auto it = old.root.find(kv.first);
+            if (it != old.root.end()) match.push_back(make_int2(kv.second, it->second));
+        }
+        if (!match.empty() && n_old) {
+            const int2* d_match = upload(ctx, S_TREE_ROOTS, match);
+            uint32_t* kept = ctx->scratch.as<uint32_t>(S_TREE_ZERO, (uint64_t)old.v.n1 + old.v.n2);
+            uint32_t* kept2 = kept + old.v.n1;
+            BS_HIP(hipMemsetAsync(kept, 0, sizeof(uint32_t) * ((uint64_t)old.v.n1 + old.v.n2), st));
+            k_node_kept<<<blocks(n_old), 256, 0, st>>>(n_old, old_origins, keep, old.v, d_match, (uint32_t)match.size(),
+                                                       kept, kept2);
+            k_keep_tiles<<<(unsigned)match.size() * (N1_SLOTS / 256), 256, 0, st>>>(old.v, d_match, kept, kept2, t->v);
+            BS_HIP(hipGetLastError());
+            BS_HIP(hipStreamSynchronize(st));
+        }
+    } catch (const Error& e) {
+        if (!e.out_of_memory) throw;
+        (void)hipStreamSynchronize(st);
+        return nullptr;
     }
     t->pending = nullptr;
     return t;

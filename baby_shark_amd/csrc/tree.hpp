@@ -44,7 +44,7 @@ struct DeviceTree {
 
 // The volume's tree on the device, made from its leaves (and tiles) or from its
 // Topology; nullptr when it does not fit: more than 2^24 128^3 blocks in the box
-// of the leaves, 256 root blocks in it or 2^16 nodes.  With `no_gap` nullptr also,
+// of the leaves, 256 root blocks in it, 2^16 nodes, or device memory.  With `no_gap` nullptr also,
 // and nothing is made, where the root's flood fill may close a gap on a z line
 // between two root entries (root_node/flood_fill.rs:14-41), which is left to
 // Topology.
@@ -65,6 +65,8 @@ void tree_flood_fill(bs_ctx* ctx, const DeviceTree& t, const uint8_t* leaf_flags
 // 68-162) with `a` as self.  The slot rules work on copies, so that a call that
 // fails leaves both operands' trees as they were.  The result's leaves in origin
 // order: refs[i] = (leaf of a, leaf of b, LEAF_* | negate << 8, 0), origins[i].
+// No tree when the result has more than 256 root blocks or 2^16 nodes, or when
+// device memory runs out.
 struct TreeOperand {
     const int4* origins;
     const uint8_t* flags;  // bit 2: mask empty
@@ -82,7 +84,8 @@ TreeCsg tree_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, const Tr
 
 // The tree after Volume::offset (see Topology::after_offset) of a volume whose
 // tree is `old`: the nodes of the result's leaves, with the tile values of the
-// nodes that kept a leaf (keep: per leaf of the old volume).
+// nodes that kept a leaf (keep: per leaf of the old volume); nullptr when it does
+// not fit (see ensure_tree).
 std::unique_ptr<DeviceTree> tree_after_offset(bs_ctx* ctx, const DeviceTree& old, const int4* old_origins,
                                               const uint32_t* keep, uint64_t n_old, const int4* origins, uint64_t n);
 

@@ -705,13 +705,15 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
             plan = tree_csg(ctx, *da, *db, {reinterpret_cast<const int4*>(a->origins), fa, a->n_leaves},
                             {reinterpret_cast<const int4*>(b->origins), fb, b->n_leaves}, op);
             cs.ms_plan = lap();
-            cs.n_paired = plan.n_paired;
-            alloc_leaves(&out, plan.n_out);
-            cs.ms_memory = lap();
-            assemble(out, plan.n_out, plan.refs, plan.origins, ev_asm);
+            if (plan.tree) {
+                cs.n_paired = plan.n_paired;
+                alloc_leaves(&out, plan.n_out);
+                cs.ms_memory = lap();
+                assemble(out, plan.n_out, plan.refs, plan.origins, ev_asm);
+            }
             BS_HIP(hipStreamSynchronize(ctx->stream));
             cs.ms_flood = ev_flood.ms();
-            cs.ms_assemble = ev_asm.ms();
+            if (plan.tree) cs.ms_assemble = ev_asm.ms();
         } catch (...) {
             // the operands are the caller's again, flood filled and otherwise as they were: no kernel may still
             // read them when they are freed
@@ -720,20 +722,36 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
             throw;
         }
         lap();
-        plan.tree->pending = plan.work_a->pending = nullptr;
-        if (plan.work_b) plan.work_b->pending = nullptr;
-        finish(out, std::move(plan.tiles));
-        a->tree = std::move(plan.tree);
-        b->tree.reset();
-        cs.ms_memory += lap();
-        cs.n_out = a->n_leaves;
-        cs.ms_wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_wall).count();
-        ctx->last_csg = cs;
-        return;
+        for (DeviceTree* t : {plan.tree.get(), plan.work_a.get(), plan.work_b.get()})
+            if (t) t->pending = nullptr;
+        if (plan.tree) {
+            finish(out, std::move(plan.tiles));
+            a->tree = std::move(plan.tree);
+            b->tree.reset();
+            cs.ms_memory += lap();
+            cs.n_out = a->n_leaves;
+            cs.ms_wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_wall).count();
+            ctx->last_csg = cs;
+            return;
+        }
     }
+    // The host's forms are flood filled and then become the plan: a call that
+    // fails leaves the device's forms where there are any; else, from the plan on,
+    // the upper levels are lost.
+    struct HostForms {
+        bs_ctx* ctx;
+        bs_volume *a, *b;
+        bool planned = false, done = false;
+        ~HostForms() {
+            if (done) return;
+            (void)hipStreamSynchronize(ctx->stream);
+            for (bs_volume* v : {a, b}) {
+                if (!v->tree && planned) v->tree_lost = true;
+                if (v->tree || planned) v->topo.reset();
+            }
+        }
+    } forms{ctx, a, b};
     ensure_topologies(ctx, a, b);
-    a->tree.reset();  // the host's form is flood filled
-    b->tree.reset();
     Topology& ta = *a->topo;
     Topology& tb = *b->topo;
     cs.ms_topology = lap();
@@ -764,19 +782,7 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
     }
     cs.ms_plan_fill = split();
 
-    // The plan is made in the operands' trees themselves: a call that fails from here on loses them.
-    struct LoseTrees {
-        bs_ctx* ctx;
-        bs_volume *a, *b;
-        bool done = false;
-        ~LoseTrees() {
-            if (done) return;
-            (void)hipStreamSynchronize(ctx->stream);
-            a->topo.reset();
-            b->topo.reset();
-            a->tree_lost = b->tree_lost = true;
-        }
-    } lose{ctx, a, b};
+    forms.planned = true;
     std::unique_ptr<Topology> tb_owned = std::move(b->topo);
     ta.csg(std::move(*tb_owned), op);
     tb_owned.reset();
@@ -881,9 +887,11 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
         free_leaves(&out, ctx->stream);
         throw;
     }
-    lose.done = true;
+    forms.done = true;
     finish(out, std::move(tiles));
     a->topo = std::move(compacted);
+    a->tree.reset();
+    b->tree.reset();
     cs.ms_memory += lap();
     cs.n_out = n_out;
     cs.ms_wall = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_wall).count();

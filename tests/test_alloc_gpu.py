@@ -62,15 +62,17 @@ def mesh(ctx, v):
 
 
 @pytest.mark.parametrize("op", ["union", "subtract", "intersect"])
-@pytest.mark.parametrize("gap", [False, True])
-def test_csg_that_fails_keeps_its_operands(gpu_ctx, op, gap):
-    a0, b0 = operands(gpu_ctx, gap)
+@pytest.mark.parametrize("form", ["device", "device, gap", "host, gap"])
+def test_csg_that_fails_keeps_its_operands(gpu_ctx, op, form):
+    a0, b0 = operands(gpu_ctx, form != "device")
+    if form == "host, gap":
+        a0, b0 = a0.clone().union(b0.clone()), b0.subtract(a0)
     soups = mesh(gpu_ctx, a0.clone()), mesh(gpu_ctx, b0.clone())
     r = getattr(a0.clone(), op)(b0.clone())
     want, signs = r.export(), r.signs_at(Q)
     failed = lost = 0
     for first in range(1, 100):
-        print(f"  {op} gap={gap} refused from request {first}", flush=True)
+        print(f"  {op} {form} refused from request {first}", flush=True)
         ctx = bs.Context(0)
         a, b = on_context(a0, ctx), on_context(b0, ctx)
         try:
@@ -83,8 +85,8 @@ def test_csg_that_fails_keeps_its_operands(gpu_ctx, op, gap):
             got = mesh(ctx, a), mesh(ctx, b)
             assert np.array_equal(got[0], soups[0]) and np.array_equal(got[1], soups[1])
             r = getattr(a, op)(b)
-        except bs.BSError as e:  # only where the plan was made in the host's form
-            assert gap and "upper levels" in str(e)
+        except bs.BSError as e:  # only where the plan was made in the one form that there was
+            assert form == "host, gap" and "upper levels" in str(e)
             assert np.array_equal(a.export().origins, a0.export().origins)
             lost += 1
             continue
@@ -92,9 +94,64 @@ def test_csg_that_fails_keeps_its_operands(gpu_ctx, op, gap):
         assert np.array_equal(r.signs_at(Q), signs)
     else:
         pytest.fail("still refused")
-    assert failed > 2 and bool(lost) == gap
+    assert failed > 2 and bool(lost) == (form == "host, gap")
     same_volume(r.export(), want)
     assert np.array_equal(r.signs_at(Q), signs)
+
+
+@pytest.mark.parametrize("op", ["union", "subtract", "intersect", "offset"])
+def test_without_memory_for_the_device_tree(gpu_ctx, op):
+    """One request alone is refused: where that is for the upper levels on the
+    device, the host's form serves."""
+    a0, b0 = operands(gpu_ctx, False)
+    a0 = bs.MeshToVolume(gpu_ctx).with_voxel_size(H).with_narrow_band_width(2).convert(mesh(gpu_ctx, a0).view(np.float32))
+
+    def call(a, b):
+        return a.offset(0.2) if op == "offset" else getattr(a, op)(b)
+
+    if op == "offset":
+        a0 = a0.subtract(b0.clone())
+    r = call(a0.clone(), b0.clone())
+    want, signs = r.export(), r.signs_at(Q)
+    done = failed = 0
+    for first in range(1, 100):
+        print(f"  {op} refused: request {first}", flush=True)
+        ctx = bs.Context(0)
+        a, b = on_context(a0, ctx), on_context(b0, ctx)
+        _lib.load().bs_refuse_allocations(first, 1)
+        try:
+            r = call(a, b)
+            done += 1
+        except bs.BSError:
+            failed += 1
+            r = call(a, b)
+        made = _lib.load().bs_refuse_allocations(0, 0)
+        same_volume(r.export(), want)
+        assert np.array_equal(r.signs_at(Q), signs)
+        assert np.array_equal(mesh(ctx, r), mesh(gpu_ctx, r))
+        if made < first:
+            break
+    # refused for good: the operands' flags and the result's leaves, or what the sweeps need
+    assert done > (4 if op == "offset" else 15) and 1 <= failed <= (12 if op == "offset" else 4)
+
+
+def test_a_result_with_too_many_root_blocks_is_in_the_host_form(gpu_ctx, oracle_lib):
+    """256 root blocks are the device form's limit: two operands of 200, their
+    union of 400."""
+    def line(x0):
+        x = x0 + 4096 * np.arange(200)
+        idx = np.stack([np.concatenate([x, x + 1]), np.full(400, 3), np.full(400, 5)], 1).astype(np.int32)
+        val = np.where(np.arange(400) < 200, -0.02, 0.03).astype(np.float32)
+        return bs.volume_from_voxels(idx, val, H, gpu_ctx), oracle_lib.from_voxels(idx, val, H)
+    (g, r), (g2, r2) = line(-4096 * 300), line(4096 * 40)
+    g, r = g.union(g2), r.union(r2)
+    same_volume(g.export(), r.export())
+    _lib.load().bs_refuse_allocations(0, 0)
+    c = g.clone()
+    assert _lib.load().bs_refuse_allocations(0, 0) == 1  # the leaves, and no tree
+    g2, r2 = line(-4096 * 300 + 8)
+    g, r = c.subtract(g2), r.subtract(r2)
+    same_volume(g.export(), r.export())
 
 
 @pytest.mark.parametrize("gap", [False, True])
@@ -136,7 +193,7 @@ def test_offset_that_fails_keeps_its_volume_and_no_memory(gpu_ctx, gap):
         assert start - free_bytes() < result_bytes // 2
     else:
         pytest.fail("still refused")
-    assert failed > 10
+    assert failed > 6  # the blocks and scratch of the sweeps, the leaves
 
 
 def test_offset_leaves_no_arrays_with_its_context(gpu_ctx):
