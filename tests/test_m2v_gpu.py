@@ -365,3 +365,50 @@ def test_chunk_far_field_signs(gpu_ctx, oracle_lib, accuracy, level, h, band, op
     sure = (np.abs(w - 0.2) >= WN_AMBIGUITY) & ~on_surface(ge.values[li, off], pts, h)
     assert sure.sum() > 0.5 * len(pick)
     assert np.array_equal(np.signbit(ge.values[li, off])[sure], ~(w < 0.2)[sure])
+
+
+def _far_field_mesh(name):
+    if name == "box":  # large flat triangles, each cut into many
+        c = np.array([[x, y, z] for x in (-0.6, 0.6) for y in (-0.5, 0.5) for z in (-0.4, 0.4)], np.float32)
+        q = [(0, 1, 3, 2), (4, 6, 7, 5), (0, 4, 5, 1), (2, 3, 7, 6), (0, 2, 6, 4)]  # the +z face is missing
+        return np.array([c[[i, j, k]] for a, b, d, e in q for i, j, k in ((a, b, d), (a, d, e))])
+    soup = mg.torus(1.0, 0.35, 96, 48, 0.01, seed=3) if name == "torus" else mg.displaced_icosphere(5, 0.7, seed=4)
+    mid = soup.mean(axis=1)
+    if name == "patches":  # holes all over the surface
+        return soup[np.sin(9 * mid[:, 0]) * np.sin(8 * mid[:, 1] + 1) * np.sin(7 * mid[:, 2] + 2) < 0.25]
+    return soup[mid[:, 0] > -0.3]
+
+
+def _signs(ctx, soup, h, accuracy, fp64_band, threshold=0.2, band=3):
+    m = bs.MeshToVolume(ctx).with_voxel_size(h).with_narrow_band_width(band)
+    m.params.wn_accuracy = accuracy
+    m.params.fp64_band = fp64_band
+    m.params.sign_threshold = threshold
+    e = m.convert(soup).export()
+    return np.signbit(e.values)[e.active()]
+
+
+@pytest.mark.parametrize("accuracy", [1.0, 2.0, 5.0, 64.0])
+@pytest.mark.parametrize("name", ["cap", "patches", "torus", "box"])
+def test_open_mesh_signs_are_the_root_walk_s(gpu_ctx, name, accuracy):
+    """Open meshes, where winding numbers of all sizes occur.  With the default
+    re-check band the signs are those of a band one float narrower, with which
+    every voxel walks the tree from the root.  A band over everything gives the
+    FP64 walk's signs: the default band must give the same ones, and a band of
+    nothing too, wherever the walk is 1e-4 (a hundred times the rounding of its
+    sums in 32 bits) from the threshold.  (Not for the box, on whose planes
+    voxels lie: there a sum in 32 bits jumps where the one in 64 bits does not.)"""
+    soup = _far_field_mesh(name).astype(np.float32)
+    h = 0.011 if name != "box" else 0.02
+    signs = _signs(gpu_ctx, soup, h, accuracy, 0.1)
+    assert signs.any() and not signs.all()
+    assert np.array_equal(_signs(gpu_ctx, soup, h, accuracy, float(np.nextafter(np.float32(0.1), np.float32(0)))), signs)
+    if name == "box":
+        return
+    walk = _signs(gpu_ctx, soup, h, accuracy, 1e3)
+    assert np.array_equal(signs, walk)
+    sure = (_signs(gpu_ctx, soup, h, accuracy, 1e3, 0.2 - 1e-4) == walk) & \
+        (_signs(gpu_ctx, soup, h, accuracy, 1e3, 0.2 + 1e-4) == walk)
+    assert sure.mean() > 0.99
+    for _ in range(2):
+        assert np.array_equal(_signs(gpu_ctx, soup, h, accuracy, 0.0)[sure], walk[sure])
