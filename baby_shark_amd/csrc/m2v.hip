@@ -31,7 +31,7 @@ constexpr int WN_BLOCK = 256;
 
 enum Counter : int {
     C_ERR = 0, C_LEAVES, C_RECHECK, C_NEAR_INTERNAL, C_FAR, C_LEAF_VISITS, C_LEAF_TRIS, C_BOX_LO, C_BOX_HI = C_BOX_LO + 3,
-    C_PAIRS = C_BOX_HI + 3, C_SG_TILES, C_SG_CULLED, C_SG_MISS, C_SG_FALLBACK, C_WN_LIST, C_COUNT
+    C_PAIRS = C_BOX_HI + 3, C_SG_TILES, C_SG_CULLED, C_SG_MISS, C_SG_FALLBACK, C_COUNT
 };
 enum ErrBits : unsigned { E_RANGE = 1, E_TOO_MANY_SUBS = 2, E_STACK = 4, E_HASH = 8, E_TREE = 16 };
 
@@ -2119,9 +2119,11 @@ constexpr uint32_t WN_CHUNK = 512;
 // the cut-off terms below those that the order-2 term leaves out.  Everything
 // else ends in the chunk's list: k_winding visits the listed nodes per voxel.
 // A node near for every voxel, or still outside kappa * rho, is opened here, so
-// the list holds what the voxels have to look at themselves.  A chunk whose list
-// or stack outgrows its share of LDS, or the pool, lists the root instead and
-// has no polynomial: its voxels walk the whole tree.
+// the list holds what the voxels have to look at themselves.  A workgroup's lists
+// lie in its own part of the list memory, one behind the other; a chunk whose list
+// reaches past that part, or whose list or stack outgrows its share of LDS, has
+// no polynomial and no list: its voxels walk the whole tree.  Which chunks these
+// are depends on the mesh alone, not on the order in which workgroups run.
 //
 // 16 lanes per chunk: a tree level leaves about 15 nodes to look at, one per
 // lane, so four chunks keep a wave busy where one would leave three lanes of
@@ -2136,7 +2138,7 @@ constexpr int FF_BLOCK = 256;
 constexpr int FF_LANES = 16;                     // lanes per chunk
 constexpr int FF_CHUNKS = FF_BLOCK / FF_LANES;   // chunks per workgroup
 constexpr int FF_STACK = 192, FF_LIST = 128;     // LDS entries per chunk
-constexpr uint32_t FF_POOL = 64;                 // list entries per chunk in the pool, on average
+constexpr uint32_t FF_PART = 64 * FF_CHUNKS;     // a workgroup's list entries
 constexpr int FF_COEF = 24;                      // floats per chunk: centre, then 20 coefficients
 
 struct FarChunk {
@@ -2224,15 +2226,14 @@ struct FarSum {
 __global__ __launch_bounds__(FF_BLOCK) void k_far_field(const uint32_t* __restrict__ act, uint32_t n_act,
                                                         uint32_t n_chunks, const int32_t* __restrict__ origins, float h,
                                                         float inv_h, float kappa, const NodeRec* __restrict__ nodes,
-                                                        int n_nodes, uint32_t pool, uint32_t* __restrict__ list,
-                                                        FarChunk* __restrict__ chunks, float* __restrict__ coef,
-                                                        unsigned long long* counters) {
+                                                        int n_nodes, uint32_t* __restrict__ list,
+                                                        FarChunk* __restrict__ chunks, float* __restrict__ coef) {
     __shared__ int s_stack[FF_CHUNKS][FF_STACK];
     __shared__ uint32_t s_list[FF_CHUNKS][FF_LIST];
-    __shared__ uint32_t s_cnt[FF_CHUNKS], s_base;
+    __shared__ uint32_t s_cnt[FF_CHUNKS];
     const int grp = threadIdx.x / FF_LANES, gl = threadIdx.x % FF_LANES, sh = threadIdx.x & 48;
     // a workgroup covers FF_CHUNKS / 4 workgroups of k_winding: the same runs on the same XCD
-    const uint32_t chunk = xcd_workgroup(WN_CHUNK * (WN_BLOCK / 64) / FF_CHUNKS) * FF_CHUNKS + grp;
+    const uint32_t group = xcd_workgroup(WN_CHUNK * (WN_BLOCK / 64) / FF_CHUNKS), chunk = group * FF_CHUNKS + grp;
     const bool valid = chunk < n_chunks;
     // the chunk's voxels, four per lane; past the end of the list the last one again
     int v[4][3], lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
@@ -2319,24 +2320,15 @@ __global__ __launch_bounds__(FF_BLOCK) void k_far_field(const uint32_t* __restri
             cnt += n_list;
         }
     }
-    // the workgroup's share of the pool
+    // the chunk's place in the workgroup's part of the list memory
     if (gl == 0) s_cnt[grp] = bad || !valid ? 0u : cnt;
     __syncthreads();
-    uint32_t before = 0, total = 0;
-#pragma unroll
-    for (int g = 0; g < FF_CHUNKS; ++g) {
-        const uint32_t c = s_cnt[g];
-        before += g < grp ? c : 0u;
-        total += c;
-    }
-    if (threadIdx.x == 0) {
-        const unsigned long long at = atomicAdd(&counters[C_WN_LIST], (unsigned long long)total);
-        s_base = at + total <= pool ? (uint32_t)at : 0xFFFFFFFFu;
-    }
-    __syncthreads();
     if (!valid) return;
-    const uint32_t base = s_base;
-    if (bad || base == 0xFFFFFFFFu) {
+    uint32_t before = 0;
+#pragma unroll
+    for (int g = 0; g < FF_CHUNKS; ++g) before += g < grp ? s_cnt[g] : 0u;
+    const uint32_t base = group * FF_PART;
+    if (bad || before + cnt > FF_PART) {
         if (gl == 0) chunks[chunk] = FarChunk{0u, 0xFFFFFFFFu};
         return;
     }
@@ -3279,13 +3271,12 @@ void mesh_to_volume_device(bs_ctx* ctx, const float* d_tris, uint64_t n, const b
         // the polynomials are in voxel units: 1 / h^3 has to be a normal float
         if (wn_list == act && prm.wn_accuracy >= WN_FAR_ACCURACY && prm.fp64_band >= WN_FAR_BAND && h > 1e-12f && h < 1e12f) {
             const uint32_t n_chunks = (uint32_t)div_up(n_wn, 64);
-            const uint32_t pool = (uint32_t)std::min<uint64_t>((uint64_t)n_chunks * FF_POOL, 1u << 30);
+            const unsigned groups = div_up(n_chunks, FF_CHUNKS);
             chunks = S.as<FarChunk>(S_WN_CHUNKS, n_chunks);
-            far_list = S.as<uint32_t>(S_WN_LIST, pool);
+            far_list = S.as<uint32_t>(S_WN_LIST, (uint64_t)groups * FF_PART);
             coef = S.as<float>(S_WN_COEF, (uint64_t)n_chunks * FF_COEF);
-            k_far_field<<<(unsigned)div_up(n_chunks, FF_CHUNKS), FF_BLOCK, 0, st>>>(
-                act, n_act, n_chunks, vol->origins, h, inv_h, wn_kappa(prm.wn_accuracy), nodes, n_rec, pool, far_list,
-                chunks, coef, counters);
+            k_far_field<<<groups, FF_BLOCK, 0, st>>>(act, n_act, n_chunks, vol->origins, h, inv_h,
+                                                     wn_kappa(prm.wn_accuracy), nodes, n_rec, far_list, chunks, coef);
         }
         kern<<<div_up(n_wn, WN_BLOCK), WN_BLOCK, 0, st>>>(wn_list, n_wn, vol->origins, h, nodes, n_rec, btris,
                                                           prm.sign_threshold, prm.fp64_band, chunks, far_list, coef,

@@ -412,3 +412,20 @@ def test_open_mesh_signs_are_the_root_walk_s(gpu_ctx, name, accuracy):
     assert sure.mean() > 0.99
     for _ in range(2):
         assert np.array_equal(_signs(gpu_ctx, soup, h, accuracy, 0.0)[sure], walk[sure])
+
+
+@pytest.mark.parametrize("accuracy,level,h", [(4.0, 4, 0.02), (4.0, 6, 0.02), (5.0, 7, 0.02)])
+def test_chunk_lists_do_not_depend_on_the_run(gpu_ctx, accuracy, level, h):
+    """Lists of more than their part of the list memory on average: which chunks
+    walk from the root instead, and with that the visits, is the same each time."""
+    soup = mg.displaced_icosphere(level, radius=0.7, seed=4)
+    ctx = bs.Context(0)
+    ctx.set_profiling(True)
+    m = bs.MeshToVolume(ctx).with_voxel_size(h).with_narrow_band_width(2)
+    m.params.wn_accuracy = accuracy
+    seen = set()
+    for _ in range(6):
+        m.convert(soup).free()
+        s = ctx.last_stats()
+        seen.add(tuple(s[k] for k in ("wn_node_visits", "wn_far_evals", "wn_leaf_visits", "wn_leaf_tris")))
+    assert len(seen) == 1, seen
