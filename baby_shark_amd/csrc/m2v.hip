@@ -3272,11 +3272,16 @@ void mesh_to_volume_device(bs_ctx* ctx, const float* d_tris, uint64_t n, const b
         if (wn_list == act && prm.wn_accuracy >= WN_FAR_ACCURACY && prm.fp64_band >= WN_FAR_BAND && h > 1e-12f && h < 1e12f) {
             const uint32_t n_chunks = (uint32_t)div_up(n_wn, 64);
             const unsigned groups = div_up(n_chunks, FF_CHUNKS);
-            chunks = S.as<FarChunk>(S_WN_CHUNKS, n_chunks);
-            far_list = S.as<uint32_t>(S_WN_LIST, (uint64_t)groups * FF_PART);
-            coef = S.as<float>(S_WN_COEF, (uint64_t)n_chunks * FF_COEF);
-            k_far_field<<<groups, FF_BLOCK, 0, st>>>(act, n_act, n_chunks, vol->origins, h, inv_h,
-                                                     wn_kappa(prm.wn_accuracy), nodes, n_rec, far_list, chunks, coef);
+            try {  // 5.6 B a voxel, which the walk from the root does without
+                far_list = S.as<uint32_t>(S_WN_LIST, (uint64_t)groups * FF_PART);
+                coef = S.as<float>(S_WN_COEF, (uint64_t)n_chunks * FF_COEF);
+                chunks = S.as<FarChunk>(S_WN_CHUNKS, n_chunks);
+            } catch (const Error& e) {
+                if (!e.out_of_memory) throw;
+            }
+            if (chunks)
+                k_far_field<<<groups, FF_BLOCK, 0, st>>>(act, n_act, n_chunks, vol->origins, h, inv_h,
+                                                         wn_kappa(prm.wn_accuracy), nodes, n_rec, far_list, chunks, coef);
         }
         kern<<<div_up(n_wn, WN_BLOCK), WN_BLOCK, 0, st>>>(wn_list, n_wn, vol->origins, h, nodes, n_rec, btris,
                                                           prm.sign_threshold, prm.fp64_band, chunks, far_list, coef,

@@ -216,3 +216,32 @@ def test_offset_leaves_no_arrays_with_its_context(gpu_ctx):
     pool = offset()
     assert start - free_bytes() < 48 * pool
     contexts[-1].close()
+
+
+def test_conversion_without_memory_for_the_far_field(gpu_ctx):
+    """One request alone is refused: the three buffers of the far field are not
+    needed, and the signs are the same without them."""
+    from baby_shark_amd import meshgen as mg
+    soup = mg.displaced_icosphere(5, radius=0.7, seed=4)
+    soup = soup[soup.mean(axis=1)[:, 0] > -0.3]
+
+    def convert(ctx):
+        return bs.MeshToVolume(ctx).with_voxel_size(0.02).with_narrow_band_width(2).convert(soup)
+
+    want = convert(gpu_ctx).export()
+    done = failed = 0
+    for first in range(1, 200):
+        ctx = bs.Context(0)
+        _lib.load().bs_refuse_allocations(first, 1)
+        try:
+            v = convert(ctx)
+            done += 1
+        except bs.BSError:
+            failed += 1
+            v = convert(ctx)
+        made = _lib.load().bs_refuse_allocations(0, 0)
+        same_volume(v.export(), want)
+        if made < first:
+            break
+    print(f"  {done} calls made, {failed} failed", flush=True)
+    assert done - 1 == 3 and failed > 20  # the last call had nothing refused
