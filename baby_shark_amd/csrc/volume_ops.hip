@@ -984,7 +984,10 @@ __global__ __launch_bounds__(256) void k_densify_assemble(uint64_t n_out, const 
 // tiles, dual_contouring.rs:146).
 void volume_densify_tiles(bs_ctx* ctx, bs_volume* v) {
     if (v->tiles.empty()) return;
-    Topology& t = ensure_topology(ctx, v);
+    // the tree that receives the leaves; the volume keeps a form of its own until they are there
+    ensure_topology(ctx, v);
+    const std::unique_ptr<Topology> work = v->tree ? std::move(v->topo) : v->topo->clone();
+    Topology& t = *work;
     const uint64_t n_old = v->n_leaves;
     const std::vector<TileRec> made = t.densify_tiles();
     const uint64_t n_out = n_old + made.size();
@@ -1015,6 +1018,7 @@ void volume_densify_tiles(bs_ctx* ctx, bs_volume* v) {
             rec[i] = make_int2(-1, bits);
         }
     }
+    std::unique_ptr<Topology> compacted;
     bs_volume out;
     out.device = v->device;
     try {
@@ -1023,6 +1027,7 @@ void volume_densify_tiles(bs_ctx* ctx, bs_volume* v) {
         int4* d_org = ctx->scratch.as<int4>(S_MISC1, n_out);
         BS_HIP(hipMemcpyAsync(d_rec, rec.data(), sizeof(int2) * n_out, hipMemcpyHostToDevice, ctx->stream));
         BS_HIP(hipMemcpyAsync(d_org, org.data(), sizeof(int4) * n_out, hipMemcpyHostToDevice, ctx->stream));
+        compacted = t.compact(new_index);
         k_densify_assemble<<<div_up(n_out, WAVES_PER_BLOCK), 256, 0, ctx->stream>>>(
             n_out, d_rec, d_org, v->masks, v->values, reinterpret_cast<int4*>(out.origins), out.masks, out.values);
         BS_HIP(hipGetLastError());
@@ -1040,7 +1045,7 @@ void volume_densify_tiles(bs_ctx* ctx, bs_volume* v) {
     out.masks = nullptr;
     out.values = nullptr;
     v->tiles.clear();
-    v->topo = t.compact(new_index);
+    v->topo = std::move(compacted);
     v->tree.reset();
 }
 

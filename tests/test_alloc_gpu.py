@@ -39,8 +39,9 @@ def operands(ctx, gap, h=H):
     def far():
         return bs.volume_from_voxels(np.array([[0, 0, 8192 + 40], [1, 0, 8192 + 40]], np.int32),
                                      np.array([-0.02, 0.03], np.float32), h, ctx)
-    a = B.sphere(2.0, (0.1, -0.2, 0.3)).union(B.sphere(0.9, (-0.4, 0.0, 0.2)))
-    b = B.sphere(1.5, (1.6, 0.2, 0.0)).union(B.sphere(0.6, (1.5, 0.1, 0.0)))
+    a = B.sphere(0.9, (-0.4, 0.0, 0.2)).union(B.sphere(2.0, (0.1, -0.2, 0.3)))
+    b = B.sphere(0.6, (1.5, 0.1, 0.0)).union(B.sphere(1.5, (1.6, 0.2, 0.0)))
+    assert a.info()["n_tiles"] and b.info()["n_tiles"]
     return (a.union(far()), b.union(far())) if gap else (a, b)
 
 
@@ -245,3 +246,29 @@ def test_conversion_without_memory_for_the_far_field(gpu_ctx):
             break
     print(f"  {done} calls made, {failed} failed", flush=True)
     assert done - 1 == 3 and failed > 20  # the last call had nothing refused
+
+
+@pytest.mark.parametrize("form", ["device", "host, gap"])
+def test_densify_that_fails_keeps_its_volume(gpu_ctx, form):
+    v0, b = operands(gpu_ctx, form != "device")
+    if form == "host, gap":
+        v0 = v0.union(b)
+    before, soup, signs = v0.export(), mesh(gpu_ctx, v0.clone()), v0.clone().signs_at(Q)
+    r = v0.clone().densify_tiles()
+    want, want_soup = r.export(), mesh(gpu_ctx, r)
+    failed = 0
+    for first in range(1, 20):
+        ctx = bs.Context(0)
+        v = on_context(v0, ctx)
+        try:
+            with refusing(first):
+                v.densify_tiles()
+            break
+        except bs.BSError:
+            failed += 1
+        same_volume(v.export(), before)
+        assert np.array_equal(mesh(ctx, v), soup) and np.array_equal(v.signs_at(Q), signs)
+        v.densify_tiles()
+        same_volume(v.export(), want)
+        assert np.array_equal(mesh(ctx, v), want_soup)
+    assert 3 <= failed < 19
