@@ -2737,7 +2737,14 @@ uint32_t next_pow2(uint64_t v) {
 // 478,748 with none; at accuracy 1, where terms are taken a node's radius from the
 // node, some still did with 0.3.  So the far field is for the default accuracy
 // and band upwards; below either, every voxel walks from the root.
-constexpr float WN_FAR_BAND = 0.1f, WN_FAR_ACCURACY = 2.0f;
+//
+// Upwards to an accuracy of 4: the lists grow with its square, and from 5 on most
+// chunks have none and their time is lost.  Conversions of 42 M, 3.5 M, 14 M and
+// 0.7 M voxels with and without: 19.0 / 26.6, 2.7 / 3.2, 6.3 / 8.2 and 1.08 / 1.08 ms
+// at 2, 54 / 60, 5.1 / 6.1, 11.6 / 15.8 and 1.69 / 1.61 at 4, 83 / 83, 7.9 / 8.1,
+// 22.3 / 21.1 and 2.08 / 1.90 at 5, 115 / 110, 10.9 / 10.4, 27.8 / 26.9 and 2.43 / 2.28
+// at 6.
+constexpr float WN_FAR_BAND = 0.1f, WN_FAR_ACCURACY = 2.0f, WN_FAR_ACCURACY_MAX = 4.0f;
 float wn_kappa(float accuracy) { return sqrtf(2.0f * accuracy); }
 
 }  // namespace
@@ -3269,7 +3276,8 @@ void mesh_to_volume_device(bs_ctx* ctx, const float* d_tris, uint64_t n, const b
         uint32_t* far_list = nullptr;
         float* coef = nullptr;
         // the polynomials are in voxel units: 1 / h^3 has to be a normal float
-        if (wn_list == act && prm.wn_accuracy >= WN_FAR_ACCURACY && prm.fp64_band >= WN_FAR_BAND && h > 1e-12f && h < 1e12f) {
+        if (wn_list == act && prm.wn_accuracy >= WN_FAR_ACCURACY && prm.wn_accuracy <= WN_FAR_ACCURACY_MAX &&
+            prm.fp64_band >= WN_FAR_BAND && h > 1e-12f && h < 1e12f) {
             const uint32_t n_chunks = (uint32_t)div_up(n_wn, 64);
             const unsigned groups = div_up(n_chunks, FF_CHUNKS);
             try {  // 5.6 B a voxel, which the walk from the root does without

@@ -48,11 +48,10 @@ typedef struct {
     float voxel_size;     /* with_voxel_size; default 1.0                         */
     int64_t band;         /* with_narrow_band_width; default 0                    */
     float wn_accuracy;    /* accuracy scale of approximate(); reference: 2.0;
-                           * below it no far field is shared by neighbouring
-                           * voxels (slower)                                    */
+                           * from it to 4 neighbouring voxels share a far field */
     float sign_threshold; /* wn < threshold => outside; reference: 0.2            */
     float fp64_band;      /* |wn - threshold| < fp64_band is re-evaluated in FP64;
-                           * below 0.1, the default, no far field is shared     */
+                           * below 0.1, the default, no far field (slower)      */
     int32_t sign_mode;    /* BS_SIGN_PER_VOXEL (the reference) or BS_SIGN_SHARED  */
 } bs_m2v_params;
 

@@ -414,18 +414,33 @@ def test_open_mesh_signs_are_the_root_walk_s(gpu_ctx, name, accuracy):
         assert np.array_equal(_signs(gpu_ctx, soup, h, accuracy, 0.0)[sure], walk[sure])
 
 
-@pytest.mark.parametrize("accuracy,level,h", [(4.0, 4, 0.02), (4.0, 6, 0.02), (5.0, 7, 0.02)])
-def test_chunk_lists_do_not_depend_on_the_run(gpu_ctx, accuracy, level, h):
+def _visit_counts(soup, h, accuracy, fp64_band, band=2):
+    """Winding-number visit counts of a conversion on a context of its own."""
+    ctx = bs.Context(0)
+    ctx.set_profiling(True)
+    _signs(ctx, soup, h, accuracy, fp64_band, band=band)
+    s = ctx.last_stats()
+    return tuple(s[k] for k in ("wn_node_visits", "wn_far_evals", "wn_leaf_visits", "wn_leaf_tris"))
+
+
+@pytest.mark.parametrize("accuracy,level,h", [(4.0, 4, 0.02), (4.0, 5, 0.03), (4.0, 6, 0.02)])
+def test_chunk_lists_do_not_depend_on_the_run(accuracy, level, h):
     """Lists of more than their part of the list memory on average: which chunks
     walk from the root instead, and with that the visits, is the same each time."""
     soup = mg.displaced_icosphere(level, radius=0.7, seed=4)
-    ctx = bs.Context(0)
-    ctx.set_profiling(True)
-    m = bs.MeshToVolume(ctx).with_voxel_size(h).with_narrow_band_width(2)
-    m.params.wn_accuracy = accuracy
-    seen = set()
-    for _ in range(6):
-        m.convert(soup).free()
-        s = ctx.last_stats()
-        seen.add(tuple(s[k] for k in ("wn_node_visits", "wn_far_evals", "wn_leaf_visits", "wn_leaf_tris")))
+    seen = {_visit_counts(soup, h, accuracy, 0.1) for _ in range(6)}
     assert len(seen) == 1, seen
+
+
+@pytest.mark.parametrize("accuracy,level,h,shared", [
+    (2.0, 5, 0.011, True), (4.0, 5, 0.011, True),
+    (1.99, 5, 0.011, False), (4.01, 5, 0.011, False),  # outside the range that it serves
+])
+def test_where_voxels_share_a_far_field(gpu_ctx, accuracy, level, h, shared):
+    """Seen in the visits: those of a walk from the root (a re-check band just
+    below the default's) or fewer.  The signs are the same."""
+    soup = mg.displaced_icosphere(level, radius=0.7, seed=4)
+    narrow = float(np.nextafter(np.float32(0.1), np.float32(0)))
+    far, walk = _visit_counts(soup, h, accuracy, 0.1, 0), _visit_counts(soup, h, accuracy, narrow, 0)
+    assert (far[0] < walk[0]) if shared else (far == walk)
+    assert np.array_equal(_signs(gpu_ctx, soup, h, accuracy, 0.1, band=0), _signs(gpu_ctx, soup, h, accuracy, narrow, band=0))
