@@ -98,9 +98,23 @@ static void check_pool() {
     CHECK(g_live.empty());
 }
 
+// A block given back twice: the second time it is the pool's, which keeps it.
+static void check_second_release() {
+    void* a = alloc_block(1 << 20);
+    free_block(a);
+    free_block(a);
+    CHECK(g_live.count(a) == 1);
+    void* b = alloc_block(1 << 20);
+    CHECK(g_live.count(b) == 1);
+    free_block(b);
+    release_cached_memory();
+    CHECK(g_live.empty());
+}
+
 int main() {
     check_scratch();
     check_pool();
+    check_second_release();
     if (g_bad) return 1;
     std::puts("allocation checks passed");
     return 0;

@@ -138,6 +138,9 @@ void free_block(void* p, bool wait) {
         if (it != P.live.end()) {
             b = it->second;
             P.live.erase(it);
+        } else {
+            for (const DeviceBlock& parked : P.idle)
+                if (parked.p == p) return;  // given back before: the pool's, and not the driver's to free
         }
     }
     if (!b.p) {  // not one of the pool's
