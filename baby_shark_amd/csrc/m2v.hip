@@ -2732,10 +2732,11 @@ uint32_t next_pow2(uint64_t v) {
 // How far a voxel's sum is then from the walk's depends on which voxels share its
 // chunk.  Voxels within fp64_band of the threshold take the FP64 walk's sign
 // whatever their sum, so a band above that difference leaves every sign the
-// walk's.  On eight open and closed meshes, two grids each, seven thresholds, no
-// sign differed with a band of 0.02 at accuracies from 1.5 to 5, up to 23,321 of
-// 478,748 with none; at accuracy 1, where terms are taken a node's radius from the
-// node, some still did with 0.3.  So the far field is for the default accuracy
+// walk's.  On eight open meshes and soups, three grids each, seven thresholds, no
+// sign differed with the default band at accuracies of 2, 3 and 4, nor with one of
+// 0.05; without one up to 23,321 did, over the thresholds, on 478,748 voxels; at
+// accuracy 1, where terms are taken a node's radius from the node, some still did
+// with 0.3.  So the far field is for the default accuracy
 // and band upwards; below either, every voxel walks from the root.
 //
 // Upwards to an accuracy of 4: the lists grow with its square, and from 5 on most
