@@ -334,7 +334,7 @@ struct CsgWork {
     int32_t n_a;             // leaves of a: a leaf of b is known as n_a + its index in nodes of a
     const uint8_t *fa, *fb;  // leaf flags
     int4* pairs;             // (slot of a's 32^3 nodes, 16^3 node of a, of b, 0)
-    uint32_t* flips;         // 16^3 nodes of b moved in and negated
+    uint32_t *flips, *flipped;  // 16^3 nodes of b moved in and negated: their list, a word per node
     int32_t* partner;        // per leaf of a: the leaf of b it is combined with, -1
     uint32_t* negate;        // per leaf of b
     CsgCounts* counts;
@@ -394,7 +394,10 @@ __global__ void k_csg_slots1(CsgWork w, uint32_t n, const int2* __restrict__ roo
         w.a.kind1[s] = SLOT_BRANCH;
         w.a.tile1[s] = w.b.tile1[o];
         w.a.child1[s] = (int32_t)w.a.n2 + node;  // a node of b
-        if (res == CSG_TAKEN_FLIPPED) w.flips[atomicAdd(&w.counts->flips, 1u)] = (uint32_t)node;
+        if (res == CSG_TAKEN_FLIPPED) {
+            w.flips[atomicAdd(&w.counts->flips, 1u)] = (uint32_t)node;
+            w.flipped[node] = 1;
+        }
     } else if (k != k0 || __float_as_uint(tile) != __float_as_uint(tile0)) {
         w.a.kind1[s] = k;
         w.a.tile1[s] = tile;
@@ -444,15 +447,13 @@ __global__ __launch_bounds__(256) void k_csg_slots2(CsgWork w) {
     }
 }
 
-// internal_node/csg.rs:154-162
+// internal_node/csg.rs:154-162: the leaves here, the tiles where the result is
+// written (b's own slots stay as they are)
 __global__ __launch_bounds__(256) void k_csg_flip(CsgWork w) {
     if (blockIdx.x >= w.counts->flips) return;
     const uint64_t base = (uint64_t)w.flips[blockIdx.x] * N2_SLOTS;
-    for (uint32_t q = threadIdx.x; q < N2_SLOTS; q += 256) {
-        const uint8_t k = w.b.kind2[base + q];
-        if (k == SLOT_BRANCH) w.negate[w.b.child2[base + q]] = 1;
-        else if (k == SLOT_TILE) w.b.tile2[base + q] = -w.b.tile2[base + q];
-    }
+    for (uint32_t q = threadIdx.x; q < N2_SLOTS; q += 256)
+        if (w.b.kind2[base + q] == SLOT_BRANCH) w.negate[w.b.child2[base + q]] = 1;
 }
 
 // ------------------------------------------------------------------ result
@@ -543,8 +544,9 @@ __device__ inline int4 slot2_origin(int4 org, uint32_t s) {
 
 // Everything of the result in tree order, a wave per item: its active tiles to
 // tile_org (x, y, z, size) and tile_val from tile_at[i] on; with units, its
-// leaves (index) and tiles (-1 - tile) from unit_at[i] on.
+// leaves (index) and tiles (-1 - tile) from unit_at[i] on.  flipped (or null): see CsgWork.
 __global__ __launch_bounds__(256) void k_item_write(TreeView a, TreeView b, uint32_t n, const int32_t* __restrict__ nodes,
+                                                    const uint32_t* __restrict__ flipped,
                                                     const uint32_t* __restrict__ tile_at, int4* tile_org, float* tile_val,
                                                     const uint32_t* __restrict__ unit_at, int64_t* units) {
     const uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -564,7 +566,9 @@ __global__ __launch_bounds__(256) void k_item_write(TreeView a, TreeView b, uint
     }
     const bool of_b = it.node2 >= (int32_t)a.n2;
     const TreeView& t = of_b ? b : a;
-    const uint64_t base = (uint64_t)(of_b ? it.node2 - (int32_t)a.n2 : it.node2) * N2_SLOTS;
+    const int32_t node = of_b ? it.node2 - (int32_t)a.n2 : it.node2;
+    const uint64_t base = (uint64_t)node * N2_SLOTS;
+    const bool flip = of_b && flipped && flipped[node];
     const unsigned long long lt = (1ull << lane) - 1;
     for (uint32_t q = lane; q < N2_SLOTS; q += 64) {
         const uint8_t k = t.kind2[base + q];
@@ -572,7 +576,7 @@ __global__ __launch_bounds__(256) void k_item_write(TreeView a, TreeView b, uint
         const uint32_t ti = t0 + (uint32_t)__popcll(bt & lt);
         if (k == SLOT_TILE) {
             tile_org[ti] = slot2_origin(org, q);
-            tile_val[ti] = t.tile2[base + q];
+            tile_val[ti] = flip ? -t.tile2[base + q] : t.tile2[base + q];
         }
         if (units && k != SLOT_EMPTY)
             units[u0 + (uint32_t)__popcll(bu & lt)] = k == SLOT_TILE ? -1 - (int64_t)ti : (int64_t)t.child2[base + q];
@@ -634,16 +638,18 @@ __global__ void k_copy_nodes1(TreeView a, TreeView b, uint32_t n, const int32_t*
     if (i % N1_SLOTS == 0) out.org1[i / N1_SLOTS] = it.org;
 }
 __global__ __launch_bounds__(256) void k_copy_nodes2(TreeView a, TreeView b, int32_t n_a, const int32_t* __restrict__ refs,
+                                                     const uint32_t* __restrict__ flipped,
                                                      const int32_t* __restrict__ place, TreeView out) {
     const int32_t r = refs[blockIdx.x];
     const bool of_b = r >= (int32_t)a.n2;
     const int32_t node = of_b ? r - (int32_t)a.n2 : r;
     const TreeView& t = of_b ? b : a;
+    const bool flip = of_b && flipped[node];
     const uint64_t src = (uint64_t)node * N2_SLOTS, dst = (uint64_t)blockIdx.x * N2_SLOTS;
     for (uint32_t q = threadIdx.x; q < N2_SLOTS; q += 256) {
         const uint8_t k = t.kind2[src + q];
         out.kind2[dst + q] = k;
-        out.tile2[dst + q] = t.tile2[src + q];
+        out.tile2[dst + q] = flip && k == SLOT_TILE ? -t.tile2[src + q] : t.tile2[src + q];
         out.child2[dst + q] = k == SLOT_BRANCH ? place[t.child2[src + q] + (of_b ? n_a : 0)] : -1;
     }
     if (threadIdx.x == 0) out.org2[blockIdx.x] = t.org2[node];
@@ -806,11 +812,10 @@ static void plan_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, cons
     for (const auto& kv : res) nodes.push_back(kv.second);
     if (nodes.size() > MAX_ROOTS) return;
 
-    // 40 MB per copy at 570 k leaves; b's slots are written by a subtraction alone (k_csg_flip).  Working in place
-    // a subtraction of that size takes 3.40 ms instead of 3.45, a union of 1,400 leaves 0.54 instead of 0.55.
-    r.work_a = copy_slots(ctx, a);
-    if (op == CSG_SUBTRACT) r.work_b = copy_slots(ctx, b);
-    const TreeView av = r.work_a->v, bv = r.work_b ? r.work_b->v : b.v;
+    // 20 MB for 285 k leaves; working in place a subtraction of two such volumes takes 3.38 ms instead of 3.40, a
+    // union of 1,400 leaves 0.53 either way.
+    r.work = copy_slots(ctx, a);
+    const TreeView av = r.work->v, bv = b.v;
     CsgWork w{};
     w.a = av;
     w.b = bv;
@@ -823,13 +828,15 @@ static void plan_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, cons
     w.pairs = S.as<int4>(S_TREE_PAIRS, std::min(av.n2, bv.n2) + 1);
     w.flips = S.as<uint32_t>(S_TREE_FLIPS, bv.n2 + 1);
     w.partner = S.as<int32_t>(S_TREE_PARTNER, la.n);
-    // cleared together: counts, negate, keep of a's leaves, then b's, and one entry more for the total
-    uint32_t* zero = S.as<uint32_t>(S_TREE_ZERO, sizeof(CsgCounts) / 4 + lb.n + leaves + 1);
+    // cleared together: counts, negate, keep of a's leaves, then b's, and one entry more for the total, flipped
+    const uint64_t zero_n = sizeof(CsgCounts) / 4 + lb.n + leaves + 1 + bv.n2;
+    uint32_t* zero = S.as<uint32_t>(S_TREE_ZERO, zero_n);
     w.counts = reinterpret_cast<CsgCounts*>(zero);
     w.negate = zero + sizeof(CsgCounts) / 4;
     uint32_t* keep = w.negate + lb.n;
+    w.flipped = keep + leaves + 1;
     uint32_t* rank = S.as<uint32_t>(S_TREE_RANK, leaves + 1);
-    BS_HIP(hipMemsetAsync(zero, 0, sizeof(CsgCounts) + sizeof(uint32_t) * (lb.n + leaves + 1), st));
+    BS_HIP(hipMemsetAsync(zero, 0, sizeof(uint32_t) * zero_n, st));
     BS_HIP(hipMemsetAsync(w.partner, 0xFF, sizeof(int32_t) * la.n, st));
     const int2* d_roots = upload(ctx, S_TREE_ROOTS, roots);
     const int32_t* d_nodes = upload(ctx, S_TREE_NODES, nodes);
@@ -876,13 +883,13 @@ static void plan_csg(bs_ctx* ctx, const DeviceTree& a, const DeviceTree& b, cons
     int32_t i1 = 0;
     for (const auto& kv : res) tree->root[kv.first] = i1++;
     if (n_items) k_copy_nodes1<<<blocks(n_items), 256, 0, st>>>(av, bv, n_items, d_nodes, at, tree->v);
-    if (c.n2) k_copy_nodes2<<<c.n2, 256, 0, st>>>(av, bv, w.n_a, refs2, place, tree->v);
+    if (c.n2) k_copy_nodes2<<<c.n2, 256, 0, st>>>(av, bv, w.n_a, refs2, w.flipped, place, tree->v);
     BS_HIP(hipGetLastError());
     if (c.tiles) {
         int4* tile_org = S.as<int4>(S_TREE_TILES, c.tiles);
         float* tile_val = S.as<float>(S_TREE_TILE_VAL, c.tiles);
-        k_item_write<<<blocks(n_items, 4), 256, 0, st>>>(av, bv, n_items, d_nodes, tile_at, tile_org, tile_val, nullptr,
-                                                         nullptr);
+        k_item_write<<<blocks(n_items, 4), 256, 0, st>>>(av, bv, n_items, d_nodes, w.flipped, tile_at, tile_org, tile_val,
+                                                         nullptr, nullptr);
         BS_HIP(hipGetLastError());
         r.tiles = read_tiles(ctx, tile_org, tile_val, c.tiles);
     }
@@ -969,7 +976,8 @@ uint64_t tree_units(bs_ctx* ctx, const DeviceTree& t, const int64_t** units, std
     int64_t* out = S.as<int64_t>(S_MC_UNITS, n_units);
     int4* tile_org = S.as<int4>(S_TREE_TILES, n_tiles);
     float* tile_val = S.as<float>(S_TREE_TILE_VAL, n_tiles);
-    k_item_write<<<blocks(n_items, 4), 256, 0, st>>>(t.v, none, n_items, d_nodes, tile_at, tile_org, tile_val, unit_at, out);
+    k_item_write<<<blocks(n_items, 4), 256, 0, st>>>(t.v, none, n_items, d_nodes, nullptr, tile_at, tile_org, tile_val,
+                                                     unit_at, out);
     BS_HIP(hipGetLastError());
     tiles = read_tiles(ctx, tile_org, tile_val, n_tiles);
     *units = out;

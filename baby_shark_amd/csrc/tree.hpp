@@ -62,8 +62,8 @@ std::unique_ptr<Topology> download_tree(bs_ctx* ctx, const bs_volume* v);
 void tree_flood_fill(bs_ctx* ctx, const DeviceTree& t, const uint8_t* leaf_flags);
 
 // CSG of two flood-filled trees (root_node/csg.rs:9-58, internal_node/csg.rs:
-// 68-162) with `a` as self.  The slot rules work on copies, so that a call that
-// fails leaves both operands' trees as they were.  The result's leaves in origin
+// 68-162) with `a` as self.  The slot rules work on a copy of a's, so that a call
+// that fails leaves both operands' trees as they were.  The result's leaves in origin
 // order: refs[i] = (leaf of a, leaf of b, LEAF_* | negate << 8, 0), origins[i].
 // No tree when the result has more than 256 root blocks or 2^16 nodes, or when
 // device memory runs out.
@@ -74,8 +74,8 @@ struct TreeOperand {
 };
 struct TreeCsg {
     std::unique_ptr<DeviceTree> tree;
-    std::unique_ptr<DeviceTree> work_a, work_b;  // the copies, read until the stream is done
-    std::vector<TileRec> tiles;                  // active tiles in tree order
+    std::unique_ptr<DeviceTree> work;  // the copy, read until the stream is done
+    std::vector<TileRec> tiles;        // active tiles in tree order
     uint64_t n_out = 0, n_paired = 0;
     const int4 *refs = nullptr, *origins = nullptr;  // context scratch
 };

@@ -722,7 +722,7 @@ void volume_csg(bs_ctx* ctx, bs_volume* a, bs_volume* b, CsgOp op) {
             throw;
         }
         lap();
-        for (DeviceTree* t : {plan.tree.get(), plan.work_a.get(), plan.work_b.get()})
+        for (DeviceTree* t : {plan.tree.get(), plan.work.get()})
             if (t) t->pending = nullptr;
         if (plan.tree) {
             finish(out, std::move(plan.tiles));

@@ -268,3 +268,31 @@ def test_chain_keeps_the_tree(gpu_ctx, oracle_lib, extra):
     got = bs.MarchingCubesMesher(gpu_ctx).with_voxel_size(h).mesh(g)
     want = r.marching_cubes(h)
     assert got.shape == want.shape and np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("order", ["small in large", "twice"])
+def test_subtract_flips_nodes_with_tiles(gpu_ctx, oracle_lib, order):
+    """A volume that holds tiles, cut out of the inside of a large one: its 16^3
+    nodes move in negated, leaves and tiles, and so they are in the tree that
+    the next operation works on."""
+    h = 0.05
+    B = bs.VolumeBuilder(gpu_ctx, h)
+
+    def both(f):
+        return f(B.sphere), f(lambda r, c: oracle_lib.sphere(r, c, h))
+    a, ra = both(lambda sphere: sphere(22.0, (0.3, 0.1, -0.2)))
+    b, rb = both(lambda sphere: sphere(2.0, (1.0, 0.0, 0.5)).union(sphere(7.5, (0.5, 0.5, 0.0))))
+    assert b.info()["n_tiles"] > 0
+    g, r = a.subtract(b), ra.subtract(rb)
+    if order == "twice":
+        c, rc = both(lambda sphere: sphere(3.0, (1.0, -12.0, 0.5)).union(sphere(6.0, (0.5, -12.0, 0.0))))
+        g, r = g.subtract(c), r.subtract(rc)
+        c, rc = both(lambda sphere: sphere(10.0, (-4.0, -3.0, 0.5)))
+        g, r = g.union(c), r.union(rc)
+    ge, re_ = g.export(), r.export()
+    assert_same_volume(ge, re_)
+    ax = np.arange(-440, 441, 40, dtype=np.int32)
+    q = np.stack(np.meshgrid(ax, ax, ax, indexing="ij"), -1).reshape(-1, 3)
+    assert np.array_equal(g.signs_at(q), r.signs_at(q))
+    got, want = bs.MarchingCubesMesher(gpu_ctx).with_voxel_size(h).mesh(g), r.marching_cubes(h)
+    assert got.shape == want.shape and np.array_equal(got.view(np.uint32), want.view(np.uint32))
